@@ -81,7 +81,7 @@ extern "C" int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, con
     return fail(RHLLC_ERR_ARG, "bad argument (n must be a positive multiple of 256)");
   HIP_TRY(hipSetDevice(device));
   const int nw = n / 64;
-  Buf P, W2, Xd, Yd, Od, Gd, Ld;
+  Buf P, W2, Xd, Yd, Od, Gd, Ld, Sd;
   HIP_TRY(alloc(P, sizeof(float) * kModel));
   HIP_TRY(alloc(W2, sizeof(short) * kH * kH * 2));
   HIP_TRY(alloc(Xd, sizeof(float) * 3 * n));
@@ -89,6 +89,7 @@ extern "C" int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, con
   HIP_TRY(alloc(Od, sizeof(float) * n));
   HIP_TRY(alloc(Gd, sizeof(float) * kParams * nw));
   HIP_TRY(alloc(Ld, sizeof(float) * nw));
+  HIP_TRY(alloc(Sd, sizeof(float) * (kParams + 1)));
   HIP_TRY(hipMemcpy(P.p, model, sizeof(float) * kModel, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(Xd.p, X, sizeof(float) * 3 * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(Yd.p, y, sizeof(float) * n, hipMemcpyHostToDevice));
@@ -96,18 +97,10 @@ extern "C" int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, con
   HIP_TRY(launch_pack(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, nullptr));
   HIP_TRY(launch_grad(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, Xd.as<float>(), Yd.as<float>(),
                       Od.as<float>(), 1.0f / (float)n, n, Gd.as<float>(), Ld.as<float>(), nullptr));
+  HIP_TRY(launch_sum(Gd.as<float>(), Ld.as<float>(), nw, Sd.as<float>(), Sd.as<float>() + kParams, nullptr));
   HIP_TRY(hipDeviceSynchronize());
-  std::vector<float> g((size_t)kParams * nw), l(nw);
-  HIP_TRY(hipMemcpy(g.data(), Gd.p, sizeof(float) * g.size(), hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(l.data(), Ld.p, sizeof(float) * nw, hipMemcpyDeviceToHost));
-  for (int p = 0; p < kParams; ++p) {
-    float s = 0.f;
-    for (int w = 0; w < nw; ++w) s += g[(size_t)w * kParams + p];
-    grad[p] = s;
-  }
-  float s = 0.f;
-  for (int w = 0; w < nw; ++w) s += l[w];
-  *loss = s;
+  HIP_TRY(hipMemcpy(grad, Sd.p, sizeof(float) * kParams, hipMemcpyDeviceToHost));
+  HIP_TRY(hipMemcpy(loss, Sd.as<float>() + kParams, sizeof(float), hipMemcpyDeviceToHost));
   return RHLLC_OK;
 }
 
@@ -174,13 +167,13 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
   HIP_TRY(alloc(G, sizeof(float) * kParams * nw));
   HIP_TRY(alloc(L, sizeof(float) * nw));
   HIP_TRY(alloc(H, sizeof(float) * cfg->steps));
-  HIP_TRY(alloc(S, sizeof(uint32_t)));
+  HIP_TRY(alloc(S, 2 * sizeof(uint32_t)));
   HIP_TRY(hipMemcpy(P.p, model.data(), sizeof(float) * kModel, hipMemcpyHostToDevice));
   std::vector<float> zeros(kParams, 0.f);
   HIP_TRY(hipMemcpy(M.p, zeros.data(), sizeof(float) * kParams, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(V.p, zeros.data(), sizeof(float) * kParams, hipMemcpyHostToDevice));
-  const uint32_t zero = 0;
-  HIP_TRY(hipMemcpy(S.p, &zero, sizeof(uint32_t), hipMemcpyHostToDevice));
+  const uint32_t zero[2] = {0, 0};
+  HIP_TRY(hipMemcpy(S.p, zero, sizeof(zero), hipMemcpyHostToDevice));
   HIP_TRY(launch_pack(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, st));
   const float *norm = P.as<float>() + kOffNorm;
 
@@ -194,7 +187,6 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
   if (e == hipSuccess)
     e = launch_adam(P.as<float>(), M.as<float>(), V.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH,
                     G.as<float>(), nw, S.as<uint32_t>(), cfg->steps, (float)cfg->lr, L.as<float>(), H.as<float>(), st);
-  if (e == hipSuccess) e = launch_tick(S.as<uint32_t>(), st);
   hipGraph_t graph = nullptr;
   hipError_t e2 = hipStreamEndCapture(st, &graph);
   if (e != hipSuccess || e2 != hipSuccess) {
@@ -272,7 +264,6 @@ extern "C" int rhllc_mlp_grad_noalloc(int32_t device, const float *model, int32_
   // (pack: all of W2; grad: nw partial rows and nw losses), so nothing is cleared.
   HIP_TRY(launch_pack(model, W2b, W2b + kH * kH, st));
   HIP_TRY(launch_grad(model, W2b, W2b + kH * kH, X, y, ok, 1.0f / (float)n, n, part, lpart, st));
-  HIP_TRY(launch_sum_partials(part, nw, kParams, grad, st));
-  HIP_TRY(launch_sum_partials(lpart, nw, 1, loss, st));
+  HIP_TRY(launch_sum(part, lpart, nw, grad, loss, st));
   return RHLLC_OK;
 }

@@ -7,8 +7,8 @@
 //                FP32 accumulate),
 //                backward, per-wave gradient partials written to global memory;
 //   k_mlp_adam   fixed-order sum of the partials (deterministic), Adam on the
-//                FP32 master weights, BF16 copies of W2 and W2^T;
-//   k_mlp_tick   advances the device step counter.
+//                FP32 master weights, BF16 copies of W2 and W2^T, the step's
+//                loss, and the device step counter.
 #include <hip/hip_runtime.h>
 
 #include "mlp.h"
@@ -60,11 +60,14 @@ __device__ void make_sample(double gamma, uint64_t seed, uint64_t k, float x[3],
   if (!ok) x[0] = x[1] = x[2] = 0.0f;
 }
 
-__global__ void k_mlp_gen(double gamma, uint64_t seed, const uint32_t *step, int n, const float *norm, float *X,
-                          float *Y, float *OK) {
+// step: null, or {the next step's number, this step's}; see k_mlp_adam.
+__global__ void k_mlp_gen(double gamma, uint64_t seed, uint32_t *step, int n, const float *norm, float *X, float *Y,
+                          float *OK) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const uint64_t k = (uint64_t)(step ? *step : 0u) * (uint64_t)n + (uint64_t)i;
+  const uint32_t now = step ? step[0] : 0u;
+  if (step && i == 0) step[1] = now;
+  const uint64_t k = (uint64_t)now * (uint64_t)n + (uint64_t)i;
   float x[3], y;
   int ok;
   make_sample(gamma, seed, k, x, y, ok);
@@ -257,15 +260,106 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
   if (l == 0) G[kOffB3] = db, loss[wave] = ls;
 }
 
+// Fixed-order column sums of the wave partials: column p of the nw x kParams
+// array, added in row (wave) order in FP32, whatever the grid.  One thread per
+// column walking the rows waits for memory once per few rows (289 us for the
+// 1,024 rows of a 65,536-sample batch).  Here a workgroup of 1,024 threads owns
+// kSumCols columns: all of it loads kSumRows rows into LDS, 16 loads in flight a
+// thread and the next chunk's loads issued before the current one is added, and
+// one thread per column adds from LDS in order.  32 columns are one 128-byte
+// line of a row and make 141 workgroups of the 4,481 columns; with 64 columns
+// half the chip would idle.
+constexpr int kSumCols = 32;
+constexpr int kSumRows = 512;
+constexpr int kSumThreads = 1024;
+constexpr int kSumPer = kSumRows * kSumCols / kSumThreads;          // rows a thread loads of a chunk
+constexpr int kSumBlocks = (kParams + kSumCols - 1) / kSumCols;     // workgroups of the columns
+static_assert(kSumThreads % kSumCols == 0 && kSumPer * (kSumThreads / kSumCols) == kSumRows, "chunk split");
+
+// The sum of column col0 + threadIdx.x in the threads below kSumCols (0 for
+// columns past the last; other threads: unspecified).  Called by the whole block.
+__device__ __forceinline__ float ordered_column_sum(const float *__restrict__ part, int nw, int col0,
+                                                    float (*lds)[kSumCols]) {
+  const int c = threadIdx.x % kSumCols, r0 = threadIdx.x / kSumCols;
+  constexpr int kStep = kSumThreads / kSumCols;
+  const bool in = col0 + c < kParams;
+  float v[kSumPer], s = 0.f;
+  auto load = [&](int base) {
+#pragma unroll
+    for (int k = 0; k < kSumPer; ++k) {
+      const int r = base + r0 + k * kStep;
+      v[k] = in && r < nw ? part[(size_t)r * kParams + col0 + c] : 0.f;
+    }
+  };
+  load(0);
+  for (int base = 0; base < nw; base += kSumRows) {
+    __syncthreads();  // the previous chunk has been added
+#pragma unroll
+    for (int k = 0; k < kSumPer; ++k) lds[r0 + k * kStep][c] = v[k];
+    __syncthreads();
+    if (base + kSumRows < nw) load(base + kSumRows);
+    if (threadIdx.x < kSumCols) {
+      const int m = nw - base < kSumRows ? nw - base : kSumRows;
+      int r = 0;
+      for (; r + 16 <= m; r += 16) {
+        float t[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) t[k] = lds[r + k][c];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) s += t[k];
+      }
+      for (; r < m; ++r) s += lds[r][c];
+    }
+  }
+  return s;
+}
+
+// The sum of the nw wave losses in wave order, in thread 0 of the block.
+__device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss, int nw, float *lds) {
+  constexpr int kChunk = kSumRows * kSumCols;
+  float s = 0.f;
+  for (int base = 0; base < nw; base += kChunk) {
+    const int m = nw - base < kChunk ? nw - base : kChunk;
+    __syncthreads();
+    for (int k = threadIdx.x; k < m; k += kSumThreads) lds[k] = loss[base + k];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int r = 0;
+      for (; r + 16 <= m; r += 16) {
+        float t[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) t[k] = lds[r + k];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) s += t[k];
+      }
+      for (; r < m; ++r) s += lds[r];
+    }
+  }
+  return s;
+}
+
 // Sum of the wave partials in wave order, then Adam (bias-corrected) with a
-// cosine learning-rate schedule.
-__global__ void k_mlp_adam(float *P, float *Mo, float *Vo, short *W2b, short *W2Tb, const float *grad, int nwaves,
-                           const uint32_t *step, int total_steps, float lr0, const float *loss, float *loss_hist) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t s = *step;
-  if (p < kParams) {
-    float gsum = 0.f;
-    for (int wv = 0; wv < nwaves; ++wv) gsum += grad[(size_t)wv * kParams + p];
+// cosine learning-rate schedule.  The last workgroup sums the losses instead
+// and advances the step: step[1] is this step's number, which k_mlp_gen copied
+// from step[0]; only this workgroup writes step[0], which nobody reads here.
+__global__ __launch_bounds__(kSumThreads) void k_mlp_adam(float *P, float *Mo, float *Vo, short *W2b, short *W2Tb,
+                                                          const float *grad, int nwaves, uint32_t *step,
+                                                          int total_steps, float lr0, const float *loss,
+                                                          float *loss_hist) {
+  __shared__ float lds[kSumRows][kSumCols];
+  const uint32_t s = step[1];
+  if (blockIdx.x == kSumBlocks) {
+    const float t = ordered_loss_sum(loss, nwaves, &lds[0][0]);
+    if (threadIdx.x == 0) {
+      loss_hist[s] = t;
+      step[0] = s + 1u;
+    }
+    return;
+  }
+  const int col0 = blockIdx.x * kSumCols;
+  const float gsum = ordered_column_sum(grad, nwaves, col0, lds);
+  const int p = col0 + threadIdx.x;
+  if (threadIdx.x < kSumCols && p < kParams) {
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float m = b1 * Mo[p] + (1.f - b1) * gsum;
     const float v = b2 * Vo[p] + (1.f - b2) * gsum * gsum;
@@ -282,23 +376,21 @@ __global__ void k_mlp_adam(float *P, float *Mo, float *Vo, short *W2b, short *W2
       W2Tb[j * kH + i] = f2bf(np);
     }
   }
-  if (p == 0 && loss_hist) {
-    float t = 0.f;
-    for (int wv = 0; wv < nwaves; ++wv) t += loss[wv];
-    loss_hist[s] = t;
-  }
 }
 
-__global__ void k_mlp_tick(uint32_t *step) { *step += 1u; }
-
-// out[p] = sum over w < nw of part[w * np + p], added in w order in FP32 (the
-// order of the host reduction of rhllc_mlp_grad).
-__global__ void k_mlp_sum_partials(const float *part, int nw, int np, float *out) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  float s = 0.f;
-  for (int w = 0; w < nw; ++w) s += part[(size_t)w * np + p];
-  out[p] = s;
+// The gradient and the loss of one batch from the wave partials, each added in
+// wave order in FP32.
+__global__ __launch_bounds__(kSumThreads) void k_mlp_sum(const float *part, const float *lpart, int nw, float *grad,
+                                                         float *loss) {
+  __shared__ float lds[kSumRows][kSumCols];
+  if (blockIdx.x == kSumBlocks) {
+    const float t = ordered_loss_sum(lpart, nw, &lds[0][0]);
+    if (threadIdx.x == 0) *loss = t;
+    return;
+  }
+  const int col0 = blockIdx.x * kSumCols;
+  const float g = ordered_column_sum(part, nw, col0, lds);
+  if (threadIdx.x < kSumCols && col0 + (int)threadIdx.x < kParams) grad[col0 + threadIdx.x] = g;
 }
 
 __global__ void k_mlp_pack(const float *P, short *W2b, short *W2Tb) {
@@ -355,7 +447,7 @@ __global__ void k_mlp_selftest(float *out) {
   for (int r = 0; r < 4; ++r) out[4 * l + r] = acc[r];
 }
 
-hipError_t launch_gen(double gamma, uint64_t seed, const uint32_t *step, int n, const float *norm, float *X, float *Y,
+hipError_t launch_gen(double gamma, uint64_t seed, uint32_t *step, int n, const float *norm, float *X, float *Y,
                       float *OK, hipStream_t s) {
   hipLaunchKernelGGL(k_mlp_gen, dim3((n + 255) / 256), dim3(256), 0, s, gamma, seed, step, n, norm, X, Y, OK);
   return hipGetLastError();
@@ -367,18 +459,14 @@ hipError_t launch_grad(const float *P, const short *W2b, const short *W2Tb, cons
   return hipGetLastError();
 }
 hipError_t launch_adam(float *P, float *M, float *V, short *W2b, short *W2Tb, const float *grad, int nwaves,
-                       const uint32_t *step, int total_steps, float lr0, const float *loss, float *loss_hist,
+                       uint32_t *step, int total_steps, float lr0, const float *loss, float *loss_hist,
                        hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kParams + 255) / 256), dim3(256), 0, s, P, M, V, W2b, W2Tb, grad, nwaves, step,
+  hipLaunchKernelGGL(k_mlp_adam, dim3(kSumBlocks + 1), dim3(kSumThreads), 0, s, P, M, V, W2b, W2Tb, grad, nwaves, step,
                      total_steps, lr0, loss, loss_hist);
   return hipGetLastError();
 }
-hipError_t launch_sum_partials(const float *part, int nw, int np, float *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_sum_partials, dim3((np + 255) / 256), dim3(256), 0, s, part, nw, np, out);
-  return hipGetLastError();
-}
-hipError_t launch_tick(uint32_t *step, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_tick, dim3(1), dim3(1), 0, s, step);
+hipError_t launch_sum(const float *part, const float *lpart, int nw, float *grad, float *loss, hipStream_t s) {
+  hipLaunchKernelGGL(k_mlp_sum, dim3(kSumBlocks + 1), dim3(kSumThreads), 0, s, part, lpart, nw, grad, loss);
   return hipGetLastError();
 }
 hipError_t launch_pack(const float *P, short *W2b, short *W2Tb, hipStream_t s) {

@@ -52,6 +52,26 @@ def test_gradient_matches_cpu_restatement():
             assert gg @ oo / (np.linalg.norm(gg) * np.linalg.norm(oo)) > 0.9995, name
 
 
+@pytest.mark.parametrize("n", [256, 32768, 33536])  # 4, 512 (one chunk of rows) and 524 waves
+def test_gradient_is_the_sum_of_the_waves_in_order(n):
+    """Each wave's gradient and loss alone (the other samples masked, so they add zeros), added
+    in wave order in FP32, are the batch's gradient and loss bit for bit."""
+    rng = np.random.default_rng(SEED + n)
+    model = _model(rng)
+    X = rng.normal(size=(n, 3)).astype(np.float32)
+    y = rng.normal(size=n).astype(np.float32)
+    g, loss = capi.mlp_grad(model, X, y, np.ones(n, np.float32))
+    sg, sl = np.zeros(capi.MLP_PARAMS, np.float32), np.float32(0)
+    for w in range(n // 64):
+        ok = np.zeros(n, np.float32)
+        ok[64 * w: 64 * w + 64] = 1
+        gw, lw = capi.mlp_grad(model, X, y, ok)
+        sg += gw
+        sl += np.float32(lw)
+    assert np.array_equal(g, sg)
+    assert np.float32(loss) == sl
+
+
 def test_forward_matches_cpu_restatement():
     rng = np.random.default_rng(SEED + 1)
     model = _model(rng)
