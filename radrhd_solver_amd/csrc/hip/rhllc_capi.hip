@@ -79,9 +79,16 @@ struct rhllc_solver {
   float *rad_T_add = nullptr;    // pressure tensor of rhllc_add_rad_flux_tensor
   float2 *rad_k = nullptr;
   double *tab = nullptr;  // opacity table (nx*ny), owned
+  // The tiled steps of one rhllc_run rotate through the slot buffers of the
+  // speed maximum: `slot` is the next step's, and `open` says that the last
+  // step's maximum is still in its buffer (fold_speed of the next step takes
+  // it, or close_steps).  Between calls nothing is open and slot is 0; on
+  // meshes of more than kFoldMaxTiles tiles every step is closed at once.
+  int slot = 0;
+  bool open = false;
   // Captured step graphs: the two-kernel step keeps one step in [0]; the
-  // tiled step keeps two steps starting from buffer k in [k], so a replay
-  // leaves the buffer parity as it was.
+  // tiled step keeps kGraphSteps steps starting from state buffer k in [k]
+  // (folding: from slot 1 and an open step), so a replay leaves them as they were.
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   hipGraph_t graph_src[2] = {nullptr, nullptr};
   float *mlp_P = nullptr;
@@ -140,17 +147,26 @@ struct rhllc_solver {
     if (r == hipSuccess && variant == kMixedMlp) r = launch_cell_mlp(e, rad, prm.collect_stats != 0, stream);
     return r;
   }
-  // One step from buffer cur; the tiled step flips cur.
+  // State and slot buffers both return after six steps.
+  static constexpr int kGraphSteps = 2 * kSpeedBufs;
+
+  bool folds() const { return tiled && n_tiles <= kFoldMaxTiles; }
+
+  // One step from buffer cur; the tiled step flips cur and, if it folds, stays open.
   hipError_t enqueue_step() {
     hipError_t e;
     if (tiled) {
-      const Dev x = dev(cur, cur ^ 1);
+      Dev x = dev(cur, cur ^ 1);
+      x.slot = slot;
+      x.fold = open;
       e = launch_tile(x, mixed, variant, rad, prm.collect_stats != 0, n_tiles, tile_slots, stream);
       if (e == hipSuccess && variant == kMixedMlp) e = launch_cell_mlp(x, rad, prm.collect_stats != 0, stream);
-      if (e == hipSuccess) e = launch_dt(x, stream);
       if (e == hipSuccess) {
         last_in = cur;
         cur ^= 1;
+        slot = (slot + 1) % kSpeedBufs;
+        open = true;
+        if (!folds()) e = close_steps();
       }
       return e;
     }
@@ -161,16 +177,28 @@ struct rhllc_solver {
     if (e == hipSuccess) last_in = cur;
     return e;
   }
-  // Captures graph[cur]: two steps (tiled) or one (two-kernel).
+  // Takes the open step's maximum into the device scalars (tau, t, max_speed).
+  hipError_t close_steps() {
+    if (!open) return hipSuccess;
+    Dev x = now();
+    x.slot = (slot + kSpeedBufs - 1) % kSpeedBufs;
+    slot = 0;
+    open = false;
+    return launch_dt(x, stream);
+  }
+  // Captures graph[cur]: kGraphSteps steps (tiled) or one (two-kernel).
   hipError_t capture() {
-    const int k = cur, saved_in = last_in;
+    const int k = cur, saved_in = last_in, saved_slot = slot;
+    const bool saved_open = open;
     hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
-    for (int s = 0; s < (tiled ? 2 : 1) && e == hipSuccess; ++s) e = enqueue_step();
+    for (int s = 0; s < (tiled ? kGraphSteps : 1) && e == hipSuccess; ++s) e = enqueue_step();
     hipGraph_t g = nullptr;
     const hipError_t e2 = hipStreamEndCapture(stream, &g);
-    cur = k;  // capture enqueues nothing; replays set the parity
+    cur = k;  // capture enqueues nothing; replays leave these as they find them
     last_in = saved_in;
+    slot = saved_slot;
+    open = saved_open;
     if (e == hipSuccess) e = e2;
     if (e == hipSuccess) e = hipGraphInstantiate(&graph[k], g, nullptr, nullptr, 0);
     if (e != hipSuccess) {
@@ -347,7 +375,7 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   }
   if (variant == kMixedMlp) HIP_TRY(h->alloc(&d.mlp_list, N));
   HIP_TRY(h->alloc(&d.sc, 1));
-  HIP_TRY(h->alloc(&d.speed_slots, (size_t)kSpeedSlots * kSlotStride));
+  HIP_TRY(h->alloc(&d.speed_slots, (size_t)kSpeedBufs * kSpeedSlots * kSlotStride));
   std::memset(h->host_sc, 0, sizeof(Scalars));
   h->host_sc->tau = d.cfl_hmin / 1.0;
   h->host_sc->last_speed = 1.0;
@@ -475,6 +503,7 @@ extern "C" int rhllc_step(rhllc_solver *h, double tau, double *max_speed) {
   h->host_sc->tau = tau;
   HIP_TRY(hipMemcpyAsync(&h->d.sc->tau, &h->host_sc->tau, sizeof(double), hipMemcpyHostToDevice, h->stream));
   HIP_TRY(h->enqueue_step());
+  HIP_TRY(h->close_steps());
   HIP_TRY(hipMemcpyAsync(h->host_sc, h->d.sc, sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
   const double s = h->host_sc->last_speed;
@@ -487,18 +516,22 @@ extern "C" int rhllc_run(rhllc_solver *h, int32_t nsteps, int32_t use_graph) {
   if (!h->ready()) return fail(RHLLC_ERR_STATE, "no state uploaded (or no MLP model set for RHLLC_GUESS_MLP)");
   if (nsteps < 0) return fail(RHLLC_ERR_ARG, "nsteps < 0");
   HIP_TRY(hipSetDevice(h->prm.device));
-  if (!use_graph) {
-    for (int32_t k = 0; k < nsteps; ++k) HIP_TRY(h->enqueue_step());
-    return RHLLC_OK;
+  int32_t k = 0;
+  hipError_t e = hipSuccess;
+  if (use_graph) {
+    // A folding step's graph continues from an open step: the first step goes out by itself.
+    const int per = h->tiled ? rhllc_solver::kGraphSteps : 1, before = h->folds() ? 1 : 0;
+    if (nsteps >= before + per) {
+      for (; k < before && e == hipSuccess; ++k) e = h->enqueue_step();
+      if (e == hipSuccess && !h->graph[h->cur]) e = h->capture();
+      for (; k + per <= nsteps && e == hipSuccess; k += per) e = hipGraphLaunch(h->graph[h->cur], h->stream);
+      h->last_in = h->tiled ? h->cur ^ 1 : h->cur;
+    }
   }
-  const int per = h->tiled ? 2 : 1;
-  const int32_t reps = nsteps / per;
-  if (reps > 0) {
-    if (!h->graph[h->cur]) HIP_TRY(h->capture());
-    for (int32_t k = 0; k < reps; ++k) HIP_TRY(hipGraphLaunch(h->graph[h->cur], h->stream));
-    h->last_in = h->tiled ? h->cur ^ 1 : h->cur;
-  }
-  for (int32_t k = reps * per; k < nsteps; ++k) HIP_TRY(h->enqueue_step());
+  for (; k < nsteps && e == hipSuccess; ++k) e = h->enqueue_step();
+  const hipError_t e2 = h->close_steps();
+  if (e == hipSuccess) e = e2;
+  if (e != hipSuccess) return hip_fail(e, "step");
   return RHLLC_OK;
 }
 

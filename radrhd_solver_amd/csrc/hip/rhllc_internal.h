@@ -9,7 +9,16 @@ namespace rhllc_dev {
 
 constexpr int kBlock = 256;         // threads per workgroup of the face and cell kernels
 constexpr int kFacesPerThread = 1;  // faces per k_face thread (2 measured slower: fewer waves to hide latency)
-constexpr int kSpeedSlots = 1024;  // per-step max-speed partials (one atomic slot per block group)
+constexpr int kSpeedSlots = 64;     // per-step max-speed partials: one per lane of the wave that takes their maximum
+constexpr int kSpeedBufs = 3;       // slot buffers the tiled steps rotate through (fold_speed)
+// Tiled steps of up to this many tiles (4.2M cells) take the previous step's
+// speed maximum themselves (fold_speed) instead of a kernel between the steps.
+// A block then waits for one more load, which the step pays once for every
+// round of blocks the chip runs: measured with and without, 9.1 against 13.0 us
+// a step at 384 cells, 18.7 against 23.6 at 118,098 (FP64), 34.8 against 39.0
+// at 663,552 (mixed, surrogate start), 140.6 against 142.9 at 3.07M (mixed, TAUB),
+// but 474 against 471 at 6M (FP64) and 1291 against 1282 at 24M (mixed).
+constexpr int kFoldMaxTiles = 16384;
 constexpr int kSlotStride = 16;    // doubles between slots: one 128-byte line each
 constexpr int kHistBins = 41;
 constexpr int kTileCells = 256;     // cells per tile of the tiled step (one workgroup, one cell per thread)
@@ -26,7 +35,7 @@ struct Scalars {
   unsigned long long hist[kHistBins];
   unsigned long long max_residual_bits;
   unsigned long long mlp_starts;
-  unsigned int mlp_count;  // cells appended to Dev::mlp_list in the current step
+  unsigned int mlp_count[kSpeedBufs];  // cells appended to Dev::mlp_list by the step of each slot buffer
 };
 
 // Everything a kernel needs, passed by value.  Cells and faces are in the
@@ -103,7 +112,12 @@ struct Dev {
   const short *mlpW2b;
   int32_t *mlp_list;  // kMixedMlp: cells deferred to k_cell_mlp (n_cells entries)
   Scalars *sc;
-  double *speed_slots;  // kSpeedSlots * kSlotStride
+  double *speed_slots;  // kSpeedBufs buffers of kSpeedSlots * kSlotStride
+  // The slot buffer this step's maximum goes to, and whether the previous
+  // step's is still in its own (the buffer before, cyclically) instead of in
+  // sc: the tiled step then forms its tau from there (fold_speed).
+  int32_t slot;
+  int32_t fold;
 };
 
 enum Variant : int {
@@ -124,6 +138,7 @@ hipError_t launch_tile(const Dev &d, bool mixed, int variant, bool rad, bool sta
 // Face fluxes of the state in d's input buffers as the step computes them
 // (FP64 S * F, energy slot = E flux), into F4/FE: for rhllc_download_face_flux.
 hipError_t launch_face_fp64_out(const Dev &d, bool mixed, double4 *F4, double *FE, hipStream_t s);
+// Ends a step (or a run of folded steps): the maximum of slot buffer d.slot into sc.
 hipError_t launch_dt(const Dev &d, hipStream_t s);
 hipError_t launch_clear_scalars(const Dev &d, hipStream_t s);
 // Mixed path: W (FP64) recovered from U by c2p (start from the FP32 pressure).

@@ -1,13 +1,17 @@
 // gfx950 kernels of the RHLLC step.
 //
-// One step = three launches on one stream (solvers/rhllc/src/rhllc_3d_stab.cpp:10-65
-// plus rhllc_utils.cpp:15-23):
-//   k_face  one thread per face: gather left/right states, HLLC flux, write
-//           the face flux, fold the signal speed into per-slot maxima;
-//   k_cell  one thread per cell: gather its 4 face fluxes in slot order with
-//           their signs, U -= tau/V * sum, c2p (Newton, FP64) with the
-//           PhysPressureFix fallback, optional radiation source + second c2p;
-//   k_dt    one workgroup: max over the slots, tau = CFL*h_min/speed, t += tau.
+// The tiled step (the default; solvers/rhllc/src/rhllc_3d_stab.cpp:10-65 plus
+// rhllc_utils.cpp:15-23) is one launch of
+//   k_tile  one workgroup per tile: the HLLC fluxes of the tile's faces into
+//           LDS, the signal speed into per-slot maxima, then one thread per
+//           cell: its 4 face fluxes in slot order with their signs,
+//           U -= tau/V * sum, c2p (Newton, FP64) with the PhysPressureFix
+//           fallback, optional radiation source + second c2p; tau from the
+//           previous step's maxima or from k_dt,
+// then k_cell_mlp (surrogate start only) and, on large meshes and after the
+// last step of a call,
+//   k_dt    one wave: max over the slots, tau = CFL*h_min/speed, t += tau.
+// The two-kernel step is k_face (fluxes to memory), k_cell, k_dt.
 // No float atomics: face fluxes are written once and read by a fixed-order
 // gather, so the step is deterministic; the speed maximum is order-free.
 #include "rhllc_internal.h"
@@ -84,15 +88,68 @@ __device__ __forceinline__ void store_W32(const Dev &d, float4 *va_out, double2 
 extern "C" __device__ __attribute__((const)) unsigned long long __ockl_wfred_max_u64(unsigned long long);
 namespace rhllc_dev {
 
-// Per-block max of non-negative speeds into one of kSpeedSlots slots.
+__device__ __forceinline__ unsigned long long *speed_slot(const Dev &d, int buf, int i) {
+  return reinterpret_cast<unsigned long long *>(d.speed_slots + ((size_t)buf * kSpeedSlots + i) * kSlotStride);
+}
+// The maximum over a slot buffer, in every lane of the wave.
+__device__ __forceinline__ double slots_max(const Dev &d, int buf) {
+  const unsigned long long m = __ockl_wfred_max_u64(*speed_slot(d, buf, threadIdx.x & (kSpeedSlots - 1)));
+  return __longlong_as_double((long long)m);
+}
+static_assert(kSpeedSlots == 64, "one slot per lane");
+
+// The bookkeeping between two steps (rhllc_utils.cpp:15-23): tau = CFL*h_min /
+// speed of the step whose slot buffer is `buf`.  Built before the maximum is
+// known, so the scalars' loads overlap its load; store() by one thread.
+struct StepClose {
+  double t, tau0;
+  unsigned long long steps, starts;
+  __device__ __forceinline__ StepClose(const Dev &d, int buf)
+      : t(d.sc->t), tau0(d.sc->tau), steps(d.sc->steps), starts(d.sc->mlp_starts + d.sc->mlp_count[buf]) {}
+  __device__ __forceinline__ void store(const Dev &d, double speed, double tau) const {
+    Scalars *sc = d.sc;
+    sc->t = t + tau0;
+    sc->last_speed = speed;
+    sc->tau = tau;
+    sc->steps = steps + 1;
+    sc->mlp_starts = starts;
+  }
+};
+
+// Per-block max of non-negative speeds into one of kSpeedSlots slots of buffer
+// d.slot; returns the step's tau.
 // Non-negative doubles order like their bit patterns (a NaN above all), so the
 // maximum is an exact unsigned 64-bit maximum.  Every thread leaves its speed
 // in LDS; after the barrier the first wave alone takes the maximum of four
 // each and the DPP reduction of the ROCm device library, so the other waves
 // skip the cross-lane steps.
-__device__ __forceinline__ void fold_speed(const Dev &d, double speed) {
+//
+// With d.fold the previous step's maximum has not been taken yet: the block's
+// last wave (the face loop leaves it the fewest faces) reads the 64 slots of
+// the buffer before and leaves tau in LDS before the same barrier, and block 0
+// does the bookkeeping (nobody else reads what it writes in this launch) and
+// clears the buffer of the step after this one, which the step before the
+// previous one used.  This replaces a kernel between every two steps (4.2 us
+// and a launch gap) by one load of the last wave; kFoldMaxTiles has the sizes.
+__device__ __forceinline__ double fold_speed(const Dev &d, double speed) {
   __shared__ unsigned long long part[kBlock];
+  __shared__ double tau_lds;
   part[threadIdx.x] = (unsigned long long)__double_as_longlong(speed);
+  double tau = 0.0;
+  if (!d.fold) tau = d.sc->tau;  // before the barrier: a cold load
+  if (d.fold && threadIdx.x >= kBlock - 64) {
+    const int prev = d.slot == 0 ? kSpeedBufs - 1 : d.slot - 1, next = d.slot == kSpeedBufs - 1 ? 0 : d.slot + 1;
+    const double s = slots_max(d, prev);
+    tau = d.cfl_hmin / s;
+    if ((threadIdx.x & 63) == 0) tau_lds = tau;
+    if (blockIdx.x == 0) {
+      *speed_slot(d, next, threadIdx.x & 63) = 0;
+      if ((threadIdx.x & 63) == 0) {
+        StepClose(d, prev).store(d, s, tau);
+        d.sc->mlp_count[next] = 0;
+      }
+    }
+  }
   __syncthreads();
   if (threadIdx.x < 64) {
     unsigned long long m = part[threadIdx.x];
@@ -102,12 +159,9 @@ __device__ __forceinline__ void fold_speed(const Dev &d, double speed) {
       m = m < v ? v : m;
     }
     m = __ockl_wfred_max_u64(m);
-    if (threadIdx.x == 0) {
-      unsigned long long *slot =
-          reinterpret_cast<unsigned long long *>(d.speed_slots + (size_t)(blockIdx.x % kSpeedSlots) * kSlotStride);
-      atomicMax(slot, m);
-    }
+    if (threadIdx.x == 0) atomicMax(speed_slot(d, d.slot, blockIdx.x % kSpeedSlots), m);
   }
+  return d.fold ? tau_lds : tau;
 }
 
 // The mixed path's face vector S n from its 16-byte form: the FP32 vector
@@ -496,7 +550,7 @@ __device__ __forceinline__ bool defer_stale(const Dev &d, int c, bool live, cons
     const int lane = threadIdx.x & 63;
     const int first = __ffsll((long long)m) - 1;
     unsigned int base = 0;
-    if (lane == first) base = atomicAdd(&d.sc->mlp_count, (unsigned int)__popcll(m));
+    if (lane == first) base = atomicAdd(&d.sc->mlp_count[d.slot], (unsigned int)__popcll(m));
     base = __shfl(base, first, 64);
     if (stale) {
       st(d.mlp_list, base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)), c);
@@ -568,10 +622,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     B[k] = make_double2(F.v[1], F.v[2]);
     C[k] = F.p;
   }
-  fold_speed(d, speed);  // its barrier also publishes the LDS fluxes
+  const double tau = fold_speed(d, speed);  // its barrier also publishes the LDS fluxes
   const int c = t * kTileCells + (int)threadIdx.x;
   bool live = c < d.n_cells;
-  const double tau = d.sc->tau;
   State<double> U;
   double dtau = 0.0;
   float p32 = -1.f;
@@ -594,7 +647,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
 // The surrogate is trained for the ideal gas only.
 template <bool RAD, bool STATS>
 __global__ __launch_bounds__(kBlock) void k_cell_mlp(Dev d) {
-  const unsigned int n = d.sc->mlp_count;
+  const unsigned int n = d.sc->mlp_count[d.slot];
   const double tau = d.sc->tau;
   for (unsigned int b0 = blockIdx.x * kBlock; b0 < n; b0 += gridDim.x * kBlock) {
     const unsigned int i = b0 + threadIdx.x;
@@ -609,30 +662,17 @@ __global__ __launch_bounds__(kBlock) void k_cell_mlp(Dev d) {
 }
 
 // tau of the next step from the max signal speed (rhllc_utils.cpp:15-23):
-// tau = CFL*h_min / speed.  Also clears the slots for the next step.
-__global__ __launch_bounds__(1024) void k_dt(Dev d) {
-  __shared__ double part[1024 / 64];
-  double m = 0.0;
-  for (int i = threadIdx.x; i < kSpeedSlots; i += 1024) {
-    double *slot = d.speed_slots + (size_t)i * kSlotStride;
-    const double v = *slot;
-    m = m < v ? v : m;
-    *slot = 0.0;
-  }
-  m = wave_max(m);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-  __syncthreads();
+// tau = CFL*h_min / speed.  Also clears every slot buffer, so the next step
+// starts from buffer 0.  One wave.
+__global__ __launch_bounds__(64) void k_dt(Dev d) {
+  const StepClose c(d, d.slot);
+  const double s = slots_max(d, d.slot);
   if (threadIdx.x == 0) {
-    double s = part[0];
-    for (int k = 1; k < 1024 / 64; ++k) s = s < part[k] ? part[k] : s;
-    Scalars *sc = d.sc;
-    sc->t += sc->tau;
-    sc->last_speed = s;
-    sc->tau = d.cfl_hmin / s;
-    sc->steps += 1;
-    sc->mlp_starts += sc->mlp_count;
-    sc->mlp_count = 0;
+    c.store(d, s, d.cfl_hmin / s);
+    for (int k = 0; k < kSpeedBufs; ++k) d.sc->mlp_count[k] = 0;
   }
+#pragma unroll
+  for (int k = 0; k < kSpeedBufs; ++k) *speed_slot(d, k, threadIdx.x) = 0;
 }
 
 // HllcPhysToConv (rhllc_utils.cpp:25-33): U = p2c(W), W clamped in place.
@@ -736,13 +776,13 @@ __global__ __launch_bounds__(kBlock) void k_add_rad(Dev d, double tau) {
 // Clears the counters and speed slots with plain stores (graph-safe).
 __global__ void k_clear(Dev d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kSpeedSlots) d.speed_slots[(size_t)i * kSlotStride] = 0.0;
+  if (i < kSpeedBufs * kSpeedSlots) d.speed_slots[(size_t)i * kSlotStride] = 0.0;
   if (i == 0) {
     Scalars *sc = d.sc;
     sc->steps = 0;
     for (int k = 0; k < 6; ++k) sc->c2p_fail[k] = 0;
     sc->fix_calls = sc->fix_fail = sc->fallback = sc->newton_iters = sc->mlp_starts = 0;
-    sc->mlp_count = 0;
+    for (int k = 0; k < kSpeedBufs; ++k) sc->mlp_count[k] = 0;
     for (int k = 0; k < kHistBins; ++k) sc->hist[k] = 0;
     sc->max_residual_bits = 0;
   }
@@ -905,7 +945,7 @@ hipError_t launch_face_fp64_out(const Dev &d, bool mixed, double4 *F4, double *F
 }
 
 hipError_t launch_dt(const Dev &d, hipStream_t s) {
-  hipLaunchKernelGGL(k_dt, dim3(1), dim3(1024), 0, s, d);
+  hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, s, d);
   return hipGetLastError();
 }
 
@@ -949,7 +989,7 @@ hipError_t launch_add_rad(const Dev &d, bool mixed, double tau, hipStream_t s) {
 }
 
 hipError_t launch_clear_scalars(const Dev &d, hipStream_t s) {
-  hipLaunchKernelGGL(k_clear, dim3((kSpeedSlots + 255) / 256), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_clear, dim3((kSpeedBufs * kSpeedSlots + 255) / 256), dim3(256), 0, s, d);
   return hipGetLastError();
 }
 
