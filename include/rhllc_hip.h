@@ -96,7 +96,7 @@ typedef struct rhllc_params {
  * only: the tiled step keeps it in FP64, the two-kernel step stores it packed
  * (FP32 with 8-bit extensions). */
 #define RHLLC_SCHED_TILED 0      /* one kernel: each workgroup computes the faces of a tile of 256
-                                    cells (Hilbert order) into LDS, then updates the tile's cells
+                                    cells (64 on small meshes; Hilbert order) into LDS, then updates the tile's cells
                                     from there; faces shared with another tile are computed by
                                     both; the state the faces read is double-buffered */
 #define RHLLC_SCHED_TWO_KERNEL 1 /* a face kernel writes every face flux to device memory, a cell
@@ -220,7 +220,8 @@ int rhllc_add_rad_flux_tensor(rhllc_solver *h, double tau, const float *Ur, cons
  * only), out[2] dt kernel, out[3] whole step. */
 int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]);
 
-/* The tiled step's layout of a mesh, computed on the host (no device is
+/* The tiled step's layout of a mesh at 256 cells a tile (a handle on a mesh
+ * too small to fill the chip uses 64), computed on the host (no device is
  * touched), for tests and tools; no counterpart in the reference.  Returns
  * the tile count, the total of extra faces and the largest face count of a
  * tile; each non-NULL array receives: cell_new_to_old[n_cells] and

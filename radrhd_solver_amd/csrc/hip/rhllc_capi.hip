@@ -38,6 +38,23 @@ int hip_fail(hipError_t e, const char *what) {
     if (e_ != hipSuccess) return hip_fail(e_, #expr);   \
   } while (0)
 
+// Cells per tile of a handle's tiled step: 256, or 64 on a mesh too small to
+// fill the chip.  A workgroup of 256 threads takes a 64-cell tile's ~180 faces
+// in one pass where a 256-cell tile needs three, so a step that waits for one
+// workgroup's chain of loads and divides is shorter; but only one of its four
+// waves has cells, and 37% of the faces are shared with another tile (23% at
+// 256), so it loses once every CU has several workgroups.  Measured, us a step
+// with 64 / 256 cells: FP64 7.7 / 10.8 at 6,000 cells, 11.2 / 12.7 at 34,992,
+// 15.9 / 15.5 at 55,566 (TAUB), 20.5 / 19.5 at 118,098; mixed 5.5 / 7.4, 7.4 / 8.4,
+// 9.1 / 9.7, 13.9 / 13.8, 14.5 / 15.1 at 162,000, 16.2 / 16.2 at 215,622.  Just
+// past one 256-cell tile per CU (65,536 cells) the second workgroup of a few
+// CUs costs the FP64 step 19.0 against 17.7 (82,944 cells).
+int32_t tile_cells_for(int64_t n, bool mixed) {
+  constexpr int64_t kPerRound = 256 * kTileCells;  // one tile on each of 256 CUs
+  if (mixed) return n <= 5 * kPerRound / 2 ? kSmallTileCells : kTileCells;
+  return n <= 3 * kPerRound / 4 || (n > kPerRound && n <= 3 * kPerRound / 2) ? kSmallTileCells : kTileCells;
+}
+
 }  // namespace
 
 namespace rhllc_capi_detail {
@@ -261,7 +278,7 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   opt.lock_wall = p.lock_wall != 0;
   opt.reject_outer_surface = p.reject_outer_surface != 0;
   opt.out_source_copy = p.out_source_copy != 0;
-  opt.tile_cells = kTileCells;
+  opt.tile_cells = tile_cells_for(n_cells, mixed);
   rhllc_layout::Layout L;
   {
     std::string err;
@@ -337,6 +354,7 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
     uint2 *cs;
     HIP_TRY(upload(&tm, L.tile_meta.data(), L.n_tiles));
     HIP_TRY(upload(&cs, L.cell_slots.data(), N));
+    d.tile_cells = opt.tile_cells;
     d.tile_meta = tm;
     d.cell_slots = cs;
     h->n_tiles = L.n_tiles;

@@ -21,7 +21,8 @@ constexpr int kSpeedBufs = 3;       // slot buffers the tiled steps rotate throu
 constexpr int kFoldMaxTiles = 16384;
 constexpr int kSlotStride = 16;    // doubles between slots: one 128-byte line each
 constexpr int kHistBins = 41;
-constexpr int kTileCells = 256;     // cells per tile of the tiled step (one workgroup, one cell per thread)
+constexpr int kTileCells = 256;     // cells per tile of the tiled step (one workgroup, at most one cell per thread)
+constexpr int kSmallTileCells = 64;  // the same on small meshes (tile_cells_for)
 constexpr int kTileMaxSlots = 4 * kTileCells;  // faces a tile can touch (4 per cell)
 
 // Device-resident scalars of the time loop and the step counters.
@@ -77,7 +78,7 @@ struct Dev {
   double *Wpo;
   float4 *Wvao;
   double2 *Wsgo;
-  // Tiled step: tile t owns cells [t kTileCells, (t + 1) kTileCells) and
+  // Tiled step: tile t owns cells [t tile_cells, (t + 1) tile_cells) and
   // computes every face of them: its own faces (those whose earlier cell is in
   // the tile, a contiguous range since faces are grouped by their earlier
   // cell) and the extra faces it shares with an earlier tile (recomputed, same
@@ -87,6 +88,7 @@ struct Dev {
   // face_lr and face_nS / face_Sn hold n_faces + (extra faces of all tiles)
   // entries: extra face j of tile t is entry n_faces + first extra + j, a copy
   // of the face's own entry, so a tile reads its extra faces contiguously.
+  int32_t tile_cells;
   const int4 *tile_meta;
   const uint2 *cell_slots;
   int32_t tile_reverse;  // walk the tiles last to first (steps from buffer 1)

@@ -207,7 +207,7 @@ __device__ __forceinline__ FaceIn<MIXED> tile_face_in(const Dev &d, int t, int i
     o.g = ld(d.face_Sn, i);
     const int far = ld(d.face_far, i);
     const unsigned int w = (unsigned int)__float_as_int(o.g.w);
-    const int nc = t * kTileCells + (int)((w >> 21) & 0xFFu);
+    const int nc = t * d.tile_cells + (int)((w >> 21) & 0xFFu);
     const bool right = (w >> 29) & 1u;
     o.lr = right ? make_int2(far, nc) : make_int2(nc, far);
     return o;
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(kBlock) void k_cell(Dev d) {
   finish_cell<VARIANT, RAD, STATS, EOS>(d, c, live, U, guess, false, tau);
 }
 
-// The tiled step, one workgroup per tile of kTileCells cells (Hilbert order).
+// The tiled step, one workgroup per tile of d.tile_cells cells (Hilbert order).
 // Face phase: every face of the tile's cells, own faces then extra faces,
 // block-strided; the flux goes to LDS in FP64 and the speed into the per-step
 // maximum.  Cell phase, after the barrier of the speed fold: one thread per
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(kBlock) void k_cell(Dev d) {
 // 116 for the mixed variants and the kernel runs at four waves.
 template <int VARIANT, bool RAD, bool STATS, int EOS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_tile(Dev d) {
-  static_assert(kTileCells == kBlock, "one cell per thread in the cell phase");
+  static_assert(kTileCells <= kBlock && kSmallTileCells <= kBlock, "at most one cell per thread in the cell phase");
   constexpr bool MIXED = VARIANT >= kMixedPrev;
   extern __shared__ double2 lds_flux[];
   // Every other step walks the tiles backwards, so a step starts on the tiles
@@ -623,8 +623,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     C[k] = F.p;
   }
   const double tau = fold_speed(d, speed);  // its barrier also publishes the LDS fluxes
-  const int c = t * kTileCells + (int)threadIdx.x;
-  bool live = c < d.n_cells;
+  const int c = t * d.tile_cells + (int)threadIdx.x;
+  bool live = (int)threadIdx.x < d.tile_cells && c < d.n_cells;
   State<double> U;
   double dtau = 0.0;
   float p32 = -1.f;

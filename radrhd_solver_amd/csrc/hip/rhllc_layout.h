@@ -37,7 +37,7 @@ struct Layout {
   // of the FP32 vector, that restore what the FP32 rounding took: fp32 + k Q
   // is the vector to 2^-30 of its largest component, so a cell's four vectors
   // close to that (FP32 alone: 2^-24).  On the tiled step bits 21-28 hold the
-  // entry's cell in its tile (cell - 256 t) and bit 29 whether that is the
+  // entry's cell in its tile (cell - tile_cells t) and bit 29 whether that is the
   // right cell; far holds the other cell (or the right side's boundary
   // encoding), so (left, right) = bit 29 ? (far, near) : (near, far).
   rhllc_mesh::RawVec<float> Sn;

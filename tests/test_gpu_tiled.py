@@ -172,3 +172,27 @@ def test_add_rad_flux_keeps_the_fused_source_fields(tmp_path):
         res.append(s.download()[1])
         s.close()
     assert np.array_equal(res[0], res[1])
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 2), (4, 4, 4), (7, 5, 3), (20, 20, 20), (21, 21, 21), (23, 23, 22),
+                                   (26, 26, 25), (30, 30, 30), (31, 30, 30)])
+def test_tile_sizes(shape):
+    """Meshes on both sides of the lines between 64 and 256 cells a tile (FP64: 49,152, 65,536 and
+    98,304 cells; mixed: 163,840), less than one tile, and whole and ragged last tiles: the FP64 tiled
+    step gives the two-kernel step's bits, the mixed one its states to the FP32 records' rounding."""
+    m = M.kuhn_box(*shape, seed=SEED)
+    print("mesh", m.n_cells, m.n_faces, flush=True)
+    W0 = M.init_state(m, M.INIT_BLAST, params=[0.5, 0.5, 0.5, 0.3, 1.0, 100.0, 1.0])
+    U = {}
+    for prec, guess in ((capi.PREC_FP64, capi.GUESS_REFERENCE), (capi.PREC_MIXED, capi.GUESS_PREVIOUS)):
+        for sched in (capi.SCHED_TILED, capi.SCHED_TWO_KERNEL):
+            s = capi.Solver(m, cfl=0.4, precision=prec, guess=guess, schedule=sched)
+            s.upload_W(W0)
+            s.run(9)
+            s.sync()
+            U[prec, sched] = (*s.download(), s.face_flux())
+            s.close()
+    for a, b in zip(U[0, 0], U[0, 1]):
+        assert np.array_equal(a, b)
+    for k in (0, 1):
+        assert max(_l1(U[1, k][1], U[0, 0][1], m.cells["V"])) <= 1e-5
