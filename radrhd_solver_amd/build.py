@@ -52,10 +52,10 @@ def build_hip() -> str:
         obj = os.path.join(objdir, os.path.basename(src) + ".o")
         _run([HIPCC] + HIP_FLAGS + ["-c", src, "-o", obj])
         objs.append(obj)
-    # Host preparation of a handle's layout (validation, relabelling, tiles):
+    # Host preparation of a handle's layout (validation, relabelling, tiles) and record copies:
     # g++ with OpenMP (libgomp, as the mesh library uses).
     for src in (os.path.join(CSRC, "mesh", "curve_order.cpp"), os.path.join(CSRC, "mesh", "mesh_check.cpp"),
-                os.path.join(CSRC, "hip", "rhllc_layout.cpp")):
+                os.path.join(CSRC, "hip", "rhllc_layout.cpp"), os.path.join(CSRC, "hip", "rhllc_records.cpp")):
         obj = os.path.join(objdir, os.path.splitext(os.path.basename(src))[0] + ".o")
         _run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-fopenmp", "-fPIC", "-c", src, "-o", obj])
         objs.append(obj)

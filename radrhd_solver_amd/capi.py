@@ -214,9 +214,15 @@ class Solver:
         check(_lib().rhllc_upload_state(self.h, rec.ctypes.data, 80, 0, 40))
 
     def download(self):
-        rec = np.zeros((self.n_cells, 10))
-        check(_lib().rhllc_download_state(self.h, rec.ctypes.data, 80, 0, 40))
-        return rec[:, :5].copy(), rec[:, 5:].copy()
+        """(W, U) of the current state."""
+        if self.n_cells <= 4096:  # one call: the second would cost more than splitting the records here
+            rec = np.empty((self.n_cells, 10))
+            check(_lib().rhllc_download_state(self.h, rec.ctypes.data, 80, 0, 40))
+            return rec[:, :5].copy(), rec[:, 5:].copy()
+        W, U = np.empty((self.n_cells, 5)), np.empty((self.n_cells, 5))
+        check(_lib().rhllc_download_state(self.h, W.ctypes.data, 40, 0, -1))
+        check(_lib().rhllc_download_state(self.h, U.ctypes.data, 40, -1, 0))
+        return W, U
 
     def step(self, tau: float) -> float:
         s = C.c_double()
@@ -244,7 +250,7 @@ class Solver:
         check(_lib().rhllc_reset_stats(self.h))
 
     def face_flux(self):
-        F = np.zeros((self.n_faces, 5))
+        F = np.empty((self.n_faces, 5))
         check(_lib().rhllc_download_face_flux(self.h, F.ctypes.data))
         return F
 

@@ -5,6 +5,7 @@
 // when asked), one HIP stream, and optionally a captured hipGraph of the step.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -17,6 +18,7 @@
 #include "rhllc_internal.h"
 #include "flux_ext.h"
 #include "rhllc_layout.h"
+#include "rhllc_records.h"
 
 using namespace rhllc_dev;
 
@@ -61,6 +63,83 @@ namespace rhllc_capi_detail {
 int set_error(int code, const std::string &msg) { return fail(code, msg); }
 }  // namespace rhllc_capi_detail
 
+// Two pinned chunks that the transfers of a handle go through in turn: the
+// host fills (or drains) one while the device works on the other.  One thread
+// uses a handle, and everything runs on its stream.
+struct Staging {
+  // Largest chunk: 8 MB take 150 us over the link, so a transfer of many is
+  // pipelined and the launch and wait of each are small beside it.  A 480 MB
+  // snapshot measured 15.0 ms with 1 MB chunks, 13.3 with 2, 10.5 with 4 and 8
+  // and 9.5 with 16 (173 ms as whole-array copies and serial host loops).
+  static constexpr size_t kMaxBytes = (size_t)8 << 20;
+  uint8_t *host[2] = {nullptr, nullptr};
+  void *dev[2] = {nullptr, nullptr};
+  hipEvent_t done[2] = {nullptr, nullptr};
+  bool busy[2] = {false, false};  // the device may still use the chunk (done records its end)
+  size_t bytes = 0;
+
+  hipError_t alloc(size_t want) {
+    bytes = ((want < kMaxBytes ? want : kMaxBytes) + 63) & ~(size_t)63;
+    for (int b = 0; b < 2; ++b) {
+      hipError_t e = hipHostMalloc((void **)&host[b], bytes, hipHostMallocDefault);
+      if (e == hipSuccess) e = hipHostGetDevicePointer(&dev[b], host[b], 0);
+      if (e == hipSuccess) e = hipEventCreateWithFlags(&done[b], hipEventDisableTiming);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  ~Staging() {
+    for (int b = 0; b < 2; ++b) {
+      if (host[b]) (void)hipHostFree(host[b]);
+      if (done[b]) (void)hipEventDestroy(done[b]);
+    }
+  }
+  hipError_t wait(int b) {
+    if (!busy[b]) return hipSuccess;
+    busy[b] = false;
+    return hipEventSynchronize(done[b]);
+  }
+  hipError_t mark(int b, hipStream_t s) {
+    busy[b] = true;
+    return hipEventRecord(done[b], s);
+  }
+  // n entries of `each` bytes to the device: fill(first, count, host chunk),
+  // then launch(first, count, device address of the chunk).
+  template <typename Fill, typename Launch>
+  hipError_t send(int64_t n, size_t each, hipStream_t s, Fill fill, Launch launch) {
+    const int64_t per = (int64_t)(bytes / each);
+    int b = 0;
+    for (int64_t i = 0; i < n; i += per, b ^= 1) {
+      const int64_t c = n - i < per ? n - i : per;
+      hipError_t e = wait(b);
+      if (e == hipSuccess) fill(i, c, host[b]), e = launch((int)i, (int)c, dev[b]);
+      if (e == hipSuccess) e = mark(b, s);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  // n entries of `each` bytes from the device: launch, then drain(first, count,
+  // host chunk).  Everything queued on s before is done when it returns.
+  template <typename Launch, typename Drain>
+  hipError_t receive(int64_t n, size_t each, hipStream_t s, Launch launch, Drain drain) {
+    const int64_t per = (int64_t)(bytes / each), chunks = (n + per - 1) / per;
+    for (int64_t k = 0; k <= chunks; ++k) {
+      if (k < chunks) {
+        const int64_t i = k * per;
+        hipError_t e = launch((int)i, (int)(n - i < per ? n - i : per), dev[k & 1]);
+        if (e == hipSuccess) e = mark((int)(k & 1), s);
+        if (e != hipSuccess) return e;
+      }
+      if (k > 0) {
+        const int64_t i = (k - 1) * per;
+        if (const hipError_t e = wait((int)((k - 1) & 1)); e != hipSuccess) return e;
+        drain(i, n - i < per ? n - i : per, host[(k - 1) & 1]);
+      }
+    }
+    return hipSuccess;
+  }
+};
+
 struct rhllc_solver {
   rhllc_params prm{};
   int32_t n_cells = 0, n_faces = 0;
@@ -87,8 +166,11 @@ struct rhllc_solver {
   double2 *Wsgb[2] = {nullptr, nullptr};
   int32_t n_tiles = 0, tile_slots = 0;
   std::vector<void *> allocs;
-  std::vector<int32_t> cell_new_to_old, face_new_to_old;
-  Scalars *host_sc = nullptr;  // pinned staging of the device scalars
+  int32_t *cell_old_to_new = nullptr;  // device
+  int32_t *face_old_to_new = nullptr;  // device, from the first download of face fluxes on
+  rhllc_mesh::RawVec<int32_t> face_old_to_new_host;
+  Staging staging;
+  Scalars *host_sc = nullptr;  // pinned staging of the device scalars (two: [1] holds an earlier value)
   unsigned long long fix_fail_seen = 0;  // fix_fail already reported by rhllc_step / rhllc_sync
   float4 *rad_FU = nullptr;
   float4 *rad_FU_add = nullptr;  // moments of rhllc_add_rad_flux
@@ -299,9 +381,9 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   h->variant = variant;
   HIP_TRY(hipSetDevice(p.device));
   HIP_TRY(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-  HIP_TRY(hipHostMalloc((void **)&h->host_sc, sizeof(Scalars), hipHostMallocDefault));
-  h->cell_new_to_old = std::move(L.cell_new_to_old);
-  h->face_new_to_old = std::move(L.face_new_to_old);
+  HIP_TRY(hipHostMalloc((void **)&h->host_sc, 2 * sizeof(Scalars), hipHostMallocDefault));
+  // Large enough for a pass over all faces or cells, up to the chunk limit.
+  HIP_TRY(h->staging.alloc(std::max((size_t)N * 80, (size_t)F * 40)));
 
   Dev &d = h->d;
   d.n_cells = N;
@@ -322,6 +404,8 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
     if (e == hipSuccess && count) e = hipMemcpy(*dst, src, sizeof(**dst) * count, hipMemcpyHostToDevice);
     return e;
   };
+  HIP_TRY(upload(&h->cell_old_to_new, L.cell_old_to_new.data(), N));
+  h->face_old_to_new_host = std::move(L.face_old_to_new);
   // The face arrays, followed on the tiled step by the extra faces' copies
   // (the tiled mixed step reads face_far and the tile-local cells in face_Sn
   // in place of face_lr, which keeps the F faces for the flux download).
@@ -379,8 +463,10 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
     if (k == 0 || twoU) {
       HIP_TRY(h->alloc(&h->U4b[k], N + 2));
       HIP_TRY(h->alloc(&h->UEb[k], N + 2));
-      HIP_TRY(h->alloc(&h->W4b[k], N + 2));
-      HIP_TRY(h->alloc(&h->Wpb[k], N + 2));
+      if (!mixed) {
+        HIP_TRY(h->alloc(&h->W4b[k], N + 2));
+        HIP_TRY(h->alloc(&h->Wpb[k], N + 2));
+      }
     } else {
       h->U4b[k] = h->U4b[0], h->UEb[k] = h->UEb[0], h->W4b[k] = h->W4b[0], h->Wpb[k] = h->Wpb[0];
     }
@@ -394,7 +480,7 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   if (variant == kMixedMlp) HIP_TRY(h->alloc(&d.mlp_list, N));
   HIP_TRY(h->alloc(&d.sc, 1));
   HIP_TRY(h->alloc(&d.speed_slots, (size_t)kSpeedBufs * kSpeedSlots * kSlotStride));
-  std::memset(h->host_sc, 0, sizeof(Scalars));
+  std::memset(h->host_sc, 0, 2 * sizeof(Scalars));
   h->host_sc->tau = d.cfl_hmin / 1.0;
   h->host_sc->last_speed = 1.0;
   HIP_TRY(hipMemcpy(d.sc, h->host_sc, sizeof(Scalars), hipMemcpyHostToDevice));
@@ -416,47 +502,18 @@ extern "C" int rhllc_upload_state(rhllc_solver *h, const void *recs, int64_t str
   if (off_phys < 0 || stride < 40 || off_phys + 40 > stride || (off_conv >= 0 && off_conv + 40 > stride))
     return fail(RHLLC_ERR_ARG, "bad record stride/offsets");
   HIP_TRY(hipSetDevice(h->prm.device));
-  // The copies below are synchronous with the host but not with the
-  // handle's (non-blocking) stream: finish what rhllc_run left in flight.
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  const int32_t N = h->n_cells;
-  const uint8_t *base = static_cast<const uint8_t *>(recs);
-  std::vector<double4> w4(N), u4(off_conv >= 0 ? N : 0);
-  std::vector<double> wp(N), ue(off_conv >= 0 ? N : 0);
-  const int32_t *order = h->cell_new_to_old.data();
-  for (int32_t i = 0; i < N; ++i) {
-    const uint8_t *r = base + (size_t)order[i] * (size_t)stride;
-    double w[5];
-    std::memcpy(w, r + off_phys, 40);
-    w4[i] = make_double4(w[0], w[1], w[2], w[3]);
-    wp[i] = w[4];
-    if (off_conv >= 0) {
-      double u[5];
-      std::memcpy(u, r + off_conv, 40);
-      u4[i] = make_double4(u[0], u[1], u[2], u[3]);
-      ue[i] = u[4];
-    }
-  }
+  // On the handle's stream, so after what rhllc_run left in flight.
   const Dev d = h->now();
-  HIP_TRY(hipMemcpy(d.W4, w4.data(), sizeof(double4) * N, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(d.Wp, wp.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-  if (off_conv >= 0) {
-    HIP_TRY(hipMemcpy(d.U4, u4.data(), sizeof(double4) * N, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(d.UE, ue.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-    if (h->mixed) HIP_TRY(launch_seed_mixed(d, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-  } else {
-    // rhllc::Init (rhllc_init.cpp:190-192): HllcPhysToConv, max_signal_speed = 1,
-    // tau = GetTimeStep.
-    HIP_TRY(launch_p2c_init(d, h->stream));
-    if (h->mixed) HIP_TRY(launch_seed_mixed(d, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    HIP_TRY(hipMemcpy(h->host_sc, d.sc, sizeof(Scalars), hipMemcpyDeviceToHost));
-    h->host_sc->tau = d.cfl_hmin / 1.0;
-    h->host_sc->t = 0.0;
-    h->host_sc->last_speed = 1.0;
-    HIP_TRY(hipMemcpy(d.sc, h->host_sc, sizeof(Scalars), hipMemcpyHostToDevice));
-  }
+  const bool conv = off_conv >= 0;
+  HIP_TRY(h->staging.send(
+      h->n_cells, conv ? 80 : 40, h->stream,
+      [&](int64_t i, int64_t n, void *chunk) {
+        rhllc_records::gather(static_cast<const uint8_t *>(recs) + i * stride, stride, off_phys, off_conv, n, chunk);
+      },
+      [&](int i, int n, void *chunk) {
+        return launch_unpack_state(d, h->mixed, h->cell_old_to_new, i, n, conv, !conv, static_cast<double *>(chunk),
+                                   h->stream);
+      }));
   h->has_state = true;
   h->last_in = -1;
   return RHLLC_OK;
@@ -469,36 +526,18 @@ extern "C" int rhllc_download_state(rhllc_solver *h, void *recs, int64_t stride,
     return fail(RHLLC_ERR_ARG, "bad record stride/offsets");
   if (!h->has_state) return fail(RHLLC_ERR_STATE, "no state uploaded");
   HIP_TRY(hipSetDevice(h->prm.device));
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  const int32_t N = h->n_cells;
   const Dev d = h->now();
-  uint8_t *base = static_cast<uint8_t *>(recs);
-  const int32_t *order = h->cell_new_to_old.data();
-  if (off_phys >= 0) {
-    if (h->mixed) {
-      // The mixed step keeps W in FP32; rebuild FP64 W from the FP64 U.
-      HIP_TRY(launch_recover_W(d, h->stream));
-      HIP_TRY(hipStreamSynchronize(h->stream));
-    }
-    std::vector<double> wp(N);
-    std::vector<double4> w4(N);
-    HIP_TRY(hipMemcpy(wp.data(), d.Wp, sizeof(double) * N, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(w4.data(), d.W4, sizeof(double4) * N, hipMemcpyDeviceToHost));
-    for (int32_t i = 0; i < N; ++i) {
-      const double w[5] = {w4[i].x, w4[i].y, w4[i].z, w4[i].w, wp[i]};
-      std::memcpy(base + (size_t)order[i] * stride + off_phys, w, 40);
-    }
-  }
-  if (off_conv >= 0) {
-    std::vector<double4> u4(N);
-    std::vector<double> ue(N);
-    HIP_TRY(hipMemcpy(u4.data(), d.U4, sizeof(double4) * N, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(ue.data(), d.UE, sizeof(double) * N, hipMemcpyDeviceToHost));
-    for (int32_t i = 0; i < N; ++i) {
-      const double u[5] = {u4[i].x, u4[i].y, u4[i].z, u4[i].w, ue[i]};
-      std::memcpy(base + (size_t)order[i] * stride + off_conv, u, 40);
-    }
-  }
+  const bool phys = off_phys >= 0, conv = off_conv >= 0;
+  if (!phys && !conv) return RHLLC_OK;
+  HIP_TRY(h->staging.receive(
+      h->n_cells, phys && conv ? 80 : 40, h->stream,
+      [&](int i, int n, void *chunk) {
+        return launch_pack_state(d, h->mixed, h->cell_old_to_new, i, n, phys, conv, static_cast<double *>(chunk),
+                                 h->stream);
+      },
+      [&](int64_t i, int64_t n, const void *chunk) {
+        rhllc_records::scatter(static_cast<uint8_t *>(recs) + i * stride, stride, off_phys, off_conv, n, chunk);
+      }));
   return RHLLC_OK;
 }
 
@@ -616,44 +655,52 @@ extern "C" int rhllc_reset_stats(rhllc_solver *h) {
 extern "C" int rhllc_download_face_flux(rhllc_solver *h, double *F) {
   if (!h || !F) return fail(RHLLC_ERR_ARG, "null argument");
   HIP_TRY(hipSetDevice(h->prm.device));
-  HIP_TRY(hipStreamSynchronize(h->stream));
   const int32_t nf = h->n_faces;
   if (h->last_in < 0) {  // no step since the state was set
     std::memset(F, 0, sizeof(double) * 5 * (size_t)nf);
     return RHLLC_OK;
   }
-  std::vector<double4> a(nf);
-  std::vector<double> e(nf);
-  if (h->tiled) {
-    // The tiled step keeps its fluxes in LDS; they are recomputed, to the same
-    // bits, from the state the last step read (its input buffer is intact).
-    double4 *F4 = nullptr;
-    double *FE = nullptr;
-    HIP_TRY(hipMalloc((void **)&F4, sizeof(double4) * nf));
-    hipError_t r = hipMalloc((void **)&FE, sizeof(double) * nf);
-    if (r == hipSuccess) r = launch_face_fp64_out(h->dev(h->last_in, h->last_in), h->mixed, F4, FE, h->stream);
-    if (r == hipSuccess) r = hipStreamSynchronize(h->stream);
-    if (r == hipSuccess) r = hipMemcpy(a.data(), F4, sizeof(double4) * nf, hipMemcpyDeviceToHost);
-    if (r == hipSuccess) r = hipMemcpy(e.data(), FE, sizeof(double) * nf, hipMemcpyDeviceToHost);
-    (void)hipFree(F4);
-    if (FE) (void)hipFree(FE);
-    HIP_TRY(r);
-  } else if (!h->mixed) {
-    HIP_TRY(hipMemcpy(a.data(), h->d.F4, sizeof(double4) * nf, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(e.data(), h->d.FE, sizeof(double) * nf, hipMemcpyDeviceToHost));
-  } else {
-    std::vector<float4> pa(nf);
-    std::vector<uint2> pe(nf);
-    HIP_TRY(hipMemcpy(pa.data(), h->d.F4f, sizeof(float4) * nf, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(pe.data(), h->d.FXf, sizeof(uint2) * nf, hipMemcpyDeviceToHost));
-    for (int32_t i = 0; i < nf; ++i) rhllc_ext::unpack(pa[i], pe[i], F + 5 * (size_t)h->face_new_to_old[i]);
-    return RHLLC_OK;
+  if (!h->face_old_to_new) {
+    HIP_TRY(h->alloc(&h->face_old_to_new, nf));
+    HIP_TRY(hipMemcpy(h->face_old_to_new, h->face_old_to_new_host.data(), sizeof(int32_t) * nf,
+                      hipMemcpyHostToDevice));
+    rhllc_mesh::RawVec<int32_t>().swap(h->face_old_to_new_host);
   }
-  for (int32_t i = 0; i < nf; ++i) {
-    double *o = F + 5 * (size_t)h->face_new_to_old[i];
-    o[0] = a[i].x, o[1] = a[i].y, o[2] = a[i].z, o[3] = a[i].w, o[4] = e[i];
-  }
+  // The tiled step keeps its fluxes in LDS; they are recomputed, to the same
+  // bits, from the state the last step read (its input buffer is intact).
+  const Dev d = h->tiled ? h->dev(h->last_in, h->last_in) : h->now();
+  HIP_TRY(h->staging.receive(
+      nf, 40, h->stream,
+      [&](int i, int n, void *chunk) {
+        return launch_face_out(d, h->mixed, !h->tiled, h->face_old_to_new, i, n, static_cast<double *>(chunk),
+                               h->stream);
+      },
+      [&](int64_t i, int64_t n, const void *chunk) { rhllc_records::copy(F + 5 * i, chunk, sizeof(double) * 5 * n); }));
   return RHLLC_OK;
+}
+
+// Per-cell FP32 fields of the caller (moments, opacities, pressure tensor;
+// null: not given) into the device arrays, through the staging chunks in the
+// order launch_unpack_fields reads them.
+static hipError_t send_fields(rhllc_solver *h, const float *Ur, const float *Fr3, const float *ka, const float *ks,
+                              const float *Tr9, float4 *FU, float2 *k, float *T) {
+  const size_t each = sizeof(float) * ((FU ? 4 : 0) + (ka ? 2 : 0) + (T ? 9 : 0));
+  return h->staging.send(
+      h->n_cells, each, h->stream,
+      [&](int64_t i, int64_t n, void *chunk) {
+        float *o = static_cast<float *>(chunk);
+        auto put = [&](const float *src, int w) {
+          rhllc_records::copy(o, src + w * i, sizeof(float) * w * n);
+          o += w * n;
+        };
+        if (FU) put(Ur, 1), put(Fr3, 3);
+        if (ka) put(ka, 1), put(ks, 1);
+        if (T) put(Tr9, 9);
+      },
+      [&](int i, int n, void *chunk) {
+        return launch_unpack_fields(h->cell_old_to_new, i, n, static_cast<const float *>(chunk), FU, k, ka != nullptr,
+                                    T, h->stream);
+      });
 }
 
 extern "C" int rhllc_set_radiation(rhllc_solver *h, const float *Ur, const float *Fr3, const float *kappa_a,
@@ -670,32 +717,13 @@ extern "C" int rhllc_set_radiation(rhllc_solver *h, const float *Ur, const float
   if (!kappa_a != !kappa_s) return fail(RHLLC_ERR_ARG, "kappa_a and kappa_s must both be given or both be NULL");
   if (!kappa_a && !h->tab) return fail(RHLLC_ERR_ARG, "no opacities: give kappa_a/kappa_s or set an opacity table");
   const int32_t N = h->n_cells;
-  std::vector<float4> fu(N);
-  std::vector<float2> kk(N);
-  for (int32_t i = 0; i < N; ++i) {
-    const int32_t c = h->cell_new_to_old[i];
-    fu[i] = make_float4(Fr3[3 * (size_t)c], Fr3[3 * (size_t)c + 1], Fr3[3 * (size_t)c + 2], Ur[c]);
-    kk[i] = kappa_a ? make_float2(kappa_a[c], kappa_s[c]) : make_float2(0.f, 0.f);
-  }
   if (!h->rad_FU) HIP_TRY(hipMalloc((void **)&h->rad_FU, sizeof(float4) * N));
   if (!h->rad_k) HIP_TRY(hipMalloc((void **)&h->rad_k, sizeof(float2) * N));
-  HIP_TRY(hipMemcpy(h->rad_FU, fu.data(), sizeof(float4) * N, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(h->rad_k, kk.data(), sizeof(float2) * N, hipMemcpyHostToDevice));
+  HIP_TRY(send_fields(h, Ur, Fr3, kappa_a, kappa_s, nullptr, h->rad_FU, h->rad_k, nullptr));
   h->d.rad_FU = h->rad_FU;
   h->d.rad_k = h->rad_k;
   h->rad = true;
   h->rad_kappa = kappa_a != nullptr;
-  return RHLLC_OK;
-}
-
-// Per-cell FP32 tensors (9 values, caller's numbering) into device order.
-static int upload_tensor(rhllc_solver *h, const float *Tr9, float **dst) {
-  const int32_t N = h->n_cells;
-  std::vector<float> t(9 * (size_t)N);
-  for (int32_t i = 0; i < N; ++i)
-    std::memcpy(&t[9 * (size_t)i], Tr9 + 9 * (size_t)h->cell_new_to_old[i], 9 * sizeof(float));
-  if (!*dst) HIP_TRY(hipMalloc((void **)dst, sizeof(float) * 9 * N));
-  HIP_TRY(hipMemcpy(*dst, t.data(), sizeof(float) * 9 * N, hipMemcpyHostToDevice));
   return RHLLC_OK;
 }
 
@@ -708,7 +736,8 @@ extern "C" int rhllc_set_radiation_tensor(rhllc_solver *h, const float *Tr9) {
     h->d.rad_T = nullptr;
     return RHLLC_OK;
   }
-  if (int e = upload_tensor(h, Tr9, &h->rad_T)) return e;
+  if (!h->rad_T) HIP_TRY(hipMalloc((void **)&h->rad_T, sizeof(float) * 9 * (size_t)h->n_cells));
+  HIP_TRY(send_fields(h, nullptr, nullptr, nullptr, nullptr, Tr9, nullptr, nullptr, h->rad_T));
   h->d.rad_T = h->rad_T;
   return RHLLC_OK;
 }
@@ -720,30 +749,22 @@ static int add_rad_flux(rhllc_solver *h, double tau, const float *Ur, const floa
   if (!h->tab) return fail(RHLLC_ERR_STATE, "no opacity table set (rhllc_set_opacity_table)");
   if (!h->ready()) return fail(RHLLC_ERR_STATE, "no state uploaded");
   HIP_TRY(hipSetDevice(h->prm.device));
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  const int32_t N = h->n_cells;
-  std::vector<float4> fu(N);
-  for (int32_t i = 0; i < N; ++i) {
-    const int32_t c = h->cell_new_to_old[i];
-    fu[i] = make_float4(Fr3[3 * (size_t)c], Fr3[3 * (size_t)c + 1], Fr3[3 * (size_t)c + 2], Ur[c]);
-  }
+  const size_t N = (size_t)h->n_cells;
   // Its own buffers: the moments of rhllc_set_radiation (the step's fused
   // source, also held by a captured graph) stay as they were.
   if (!h->rad_FU_add) HIP_TRY(hipMalloc((void **)&h->rad_FU_add, sizeof(float4) * N));
-  HIP_TRY(hipMemcpy(h->rad_FU_add, fu.data(), sizeof(float4) * N, hipMemcpyHostToDevice));
+  if (Tr9 && !h->rad_T_add) HIP_TRY(hipMalloc((void **)&h->rad_T_add, sizeof(float) * 9 * N));
+  HIP_TRY(send_fields(h, Ur, Fr3, nullptr, nullptr, Tr9, h->rad_FU_add, nullptr, Tr9 ? h->rad_T_add : nullptr));
   Dev x = h->now();
   x.rad_FU = h->rad_FU_add;
-  x.rad_T = nullptr;
-  if (Tr9) {
-    if (int e = upload_tensor(h, Tr9, &h->rad_T_add)) return e;
-    x.rad_T = h->rad_T_add;
-  }
-  HIP_TRY(hipMemcpy(h->host_sc, h->d.sc, sizeof(Scalars), hipMemcpyDeviceToHost));
-  const unsigned long long fix_fail_before = h->host_sc->fix_fail;
+  x.rad_T = Tr9 ? h->rad_T_add : nullptr;
+  // The failures counted before, in stream order: the source's own are the difference.
+  HIP_TRY(hipMemcpyAsync(&h->host_sc[1].fix_fail, &h->d.sc->fix_fail, sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                         h->stream));
   HIP_TRY(launch_add_rad(x, h->mixed, tau, h->stream));
   HIP_TRY(hipMemcpyAsync(h->host_sc, h->d.sc, sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
-  const unsigned long long now_failed = h->host_sc->fix_fail - fix_fail_before;
+  const unsigned long long now_failed = h->host_sc->fix_fail - h->host_sc[1].fix_fail;
   h->fix_fail_seen += now_failed;  // reported here; earlier steps' failures stay for rhllc_sync
   if (now_failed)
     return fail(RHLLC_ERR_C2P, std::to_string(now_failed) + " cells failed PhysPressureFix after the radiation source");

@@ -69,7 +69,7 @@ struct Dev {
   double4 *U4;   // (D, mx, my, mz), FP64 on both paths (c2p amplifies errors in U)
   double *UE;    // E
   double4 *W4;   // (rho, vx, vy, vz), FP64 path
-  double *Wp;    // p (both paths: the FP64 pressure)
+  double *Wp;    // p, FP64 path
   float4 *Wva;   // mixed path: (vx, vy, vz, p) in FP32 (mixed_record)
   double2 *Wsg;  // mixed path: (s - D, D) in FP64, s = rho h W^2
   double4 *U4o;
@@ -129,7 +129,19 @@ enum Variant : int {
   kMixedMlp = 3,  // mixed, MLP start (previous pressure, then reference start as fallbacks)
 };
 
-hipError_t launch_p2c_init(const Dev &d, hipStream_t s);
+// State transfer of cells [first, first + n) of the caller's numbering, n
+// entries of 5 or 10 doubles at `staged` (pinned host memory, 16-byte aligned).
+// unpack: W, or W and U (conv); without U the state is W's (HllcPhysToConv).
+// reset: the time loop starts over (rhllc::Init).
+hipError_t launch_unpack_state(const Dev &d, bool mixed, const int32_t *old_to_new, int first, int n, bool conv,
+                               bool reset, const double *staged, hipStream_t s);
+hipError_t launch_pack_state(const Dev &d, bool mixed, const int32_t *old_to_new, int first, int n, bool phys,
+                             bool conv, double *staged, hipStream_t s);
+// Per-cell FP32 fields of cells [first, first + n): the regions Ur[n], Fr[3 n]
+// (with FU), kappa_a[n], kappa_s[n] (with kappa) and Tr[9 n] (with T) of
+// `staged` in this order, into the device numbering.  k without kappa: zeros.
+hipError_t launch_unpack_fields(const int32_t *old_to_new, int first, int n, const float *staged, float4 *FU,
+                                float2 *k, bool kappa, float *T, hipStream_t s);
 hipError_t launch_face(const Dev &d, bool mixed, hipStream_t s);
 hipError_t launch_cell(const Dev &d, int variant, bool rad, bool stats, hipStream_t s);
 hipError_t launch_cell_mlp(const Dev &d, bool rad, bool stats, hipStream_t s);
@@ -137,18 +149,18 @@ hipError_t launch_cell_mlp(const Dev &d, bool rad, bool stats, hipStream_t s);
 // lds_slots = the largest face count of any tile.
 hipError_t launch_tile(const Dev &d, bool mixed, int variant, bool rad, bool stats, int n_tiles, int lds_slots,
                        hipStream_t s);
-// Face fluxes of the state in d's input buffers as the step computes them
-// (FP64 S * F, energy slot = E flux), into F4/FE: for rhllc_download_face_flux.
-hipError_t launch_face_fp64_out(const Dev &d, bool mixed, double4 *F4, double *FE, hipStream_t s);
+// Face fluxes (FP64 S * F, energy slot = E flux) of faces [first, first + n) of
+// the caller's numbering, 5 doubles each, at `staged`: recomputed from the
+// state in d's input buffers as the step computes them, or (stored) from the
+// two-kernel step's flux array.
+hipError_t launch_face_out(const Dev &d, bool mixed, bool stored, const int32_t *old_to_new, int first, int n,
+                           double *staged, hipStream_t s);
 // Ends a step (or a run of folded steps): the maximum of slot buffer d.slot into sc.
 hipError_t launch_dt(const Dev &d, hipStream_t s);
 hipError_t launch_clear_scalars(const Dev &d, hipStream_t s);
-// Mixed path: W (FP64) recovered from U by c2p (start from the FP32 pressure).
-hipError_t launch_seed_mixed(const Dev &d, hipStream_t s);
 // Writes the ghost states into entries n_cells and n_cells + 1 of the input and output buffers
 // of d (U and W on the FP64 path, the cell record on the mixed path).
 hipError_t launch_ghost_cell(const Dev &d, bool mixed, hipStream_t s);
-hipError_t launch_recover_W(const Dev &d, hipStream_t s);
 // The radiation source alone (d.rad_FU set): U += tau G(W), then c2p.
 hipError_t launch_add_rad(const Dev &d, bool mixed, double tau, hipStream_t s);
 

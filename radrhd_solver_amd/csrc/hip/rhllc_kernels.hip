@@ -283,18 +283,6 @@ __global__ __launch_bounds__(kBlock) void k_face(Dev d) {
   fold_speed(d, speed);
 }
 
-// The step's face fluxes in FP64 (energy slot = E flux) for a download; on
-// the mixed path the same arithmetic as the step, E flux = D flux + tau flux.
-template <bool MIXED, int EOS>
-__global__ __launch_bounds__(kBlock) void k_face_fp64_out(Dev d, double4 *F4, double *FE) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= d.n_faces) return;
-  State<double> F;
-  (void)face_flux<MIXED, EOS>(d, i, F);
-  F4[i] = make_double4(F.d, F.v[0], F.v[1], F.v[2]);
-  FE[i] = MIXED ? F.d + F.p : F.p;
-}
-
 template <bool MIXED>
 __device__ __forceinline__ void load_flux(const Dev &d, int f, State<double> &F) {
   if (!MIXED) {
@@ -675,31 +663,6 @@ __global__ __launch_bounds__(64) void k_dt(Dev d) {
   for (int k = 0; k < kSpeedBufs; ++k) *speed_slot(d, k, threadIdx.x) = 0;
 }
 
-// HllcPhysToConv (rhllc_utils.cpp:25-33): U = p2c(W), W clamped in place.
-template <int EOS>
-__global__ __launch_bounds__(kBlock) void k_p2c_init(Dev d) {
-  const int c = blockIdx.x * kBlock + threadIdx.x;
-  if (c >= d.n_cells) return;
-  State<double> W, U;
-  load_W(d, c, W);
-  p2c<double, Ieee, EOS>(d.Gg, W, U);
-  d.W4[c] = make_double4(W.d, W.v[0], W.v[1], W.v[2]);
-  d.Wp[c] = W.p;
-  d.U4[c] = make_double4(U.d, U.v[0], U.v[1], U.v[2]);
-  d.UE[c] = U.p;
-}
-
-// Mixed path: the FP32 cell records from the FP64 primitives (after an
-// upload or HllcPhysToConv).
-template <int EOS>
-__global__ __launch_bounds__(kBlock) void k_seed_mixed(Dev d) {
-  const int c = blockIdx.x * kBlock + threadIdx.x;
-  if (c >= d.n_cells) return;
-  State<double> W;
-  load_W(d, c, W);
-  store_W32<EOS>(d, d.Wva, d.Wsg, c, W);
-}
-
 // The ghost states of boundary codes -3 and -4 as entries n_cells and
 // n_cells + 1 of the state arrays, input and output buffers alike (two threads).
 template <int EOS>
@@ -719,20 +682,6 @@ __global__ void k_ghost_cell(Dev d, bool mixed) {
   const double4 w = make_double4(W.d, W.v[0], W.v[1], W.v[2]);
   d.U4[c] = u, d.UE[c] = gu[4], d.W4[c] = w, d.Wp[c] = W.p;
   d.U4o[c] = u, d.UEo[c] = gu[4], d.W4o[c] = w, d.Wpo[c] = W.p;
-}
-
-// Mixed path: FP64 primitives from the FP64 conserved state (for download).
-template <int EOS>
-__global__ __launch_bounds__(kBlock) void k_recover_W(Dev d) {
-  const int c = blockIdx.x * kBlock + threadIdx.x;
-  if (c >= d.n_cells) return;
-  State<double> U, W;
-  load_U(d, c, U);
-  load_W32(d, c, W);
-  int it = 0;
-  c2p<Ieee, EOS>(d.Gg, U, W, W.p, it);  // W keeps the FP32 values if c2p fails
-  d.W4[c] = make_double4(W.d, W.v[0], W.v[1], W.v[2]);
-  d.Wp[c] = W.p;
 }
 
 // The radiation source on its own, after a step without it: AddRadFlux then
@@ -773,6 +722,138 @@ __global__ __launch_bounds__(kBlock) void k_add_rad(Dev d, double tau) {
   }
 }
 
+// ------------------------------------------------------------ state transfer
+// The caller's records live in the caller's numbering, the device arrays in
+// the Hilbert one.  These kernels renumber: one thread per cell (or face) of
+// the caller's numbering, the staged chunk (pinned host memory, read and
+// written over the host link) moved through LDS so that its accesses are
+// whole consecutive lines, the device arrays by scattered 8- to 32-byte
+// accesses, which cost far less than the link.  The host then only copies
+// records in order.
+template <typename T>
+__device__ __forceinline__ void staged_load(const T *__restrict__ src, T *lds, int count) {
+  for (int k = threadIdx.x; k < count; k += kBlock) lds[k] = src[k];
+}
+__device__ __forceinline__ void staged_store(double *__restrict__ dst, const double *lds, int count) {
+  // 16 bytes a lane; a chunk of a block starts at a multiple of 256 * 40 bytes.
+  const double2 *l2 = reinterpret_cast<const double2 *>(lds);
+  double2 *d2 = reinterpret_cast<double2 *>(dst);
+  for (int k = threadIdx.x; k < count / 2; k += kBlock) d2[k] = l2[k];
+  if ((count & 1) && threadIdx.x == 0) dst[count - 1] = lds[count - 1];
+}
+
+// W (and U) of n cells from the chunk; without U, U = p2c(W) with W clamped in
+// place (HllcPhysToConv, rhllc_utils.cpp:25-33).  The mixed path keeps W as
+// the cell records.  reset: rhllc::Init's time (rhllc_init.cpp:190-192).
+template <bool MIXED, int EOS>
+__global__ __launch_bounds__(kBlock) void k_unpack_state(Dev d, const int32_t *old_to_new, int first, int n,
+                                                         bool conv, bool reset, const double *staged) {
+  __shared__ __align__(16) double buf[10 * kBlock];
+  const int b0 = blockIdx.x * kBlock, w = conv ? 10 : 5;
+  const int m = n - b0 < kBlock ? n - b0 : kBlock;
+  staged_load(staged + (size_t)b0 * w, buf, m * w);
+  __syncthreads();
+  if (reset && b0 == 0 && threadIdx.x == 0) d.sc->tau = d.cfl_hmin / 1.0, d.sc->t = 0.0, d.sc->last_speed = 1.0;
+  if ((int)threadIdx.x >= m) return;
+  const int c = old_to_new[first + b0 + threadIdx.x];
+  const double *p = buf + threadIdx.x * w;
+  State<double> W, U;
+  W.d = p[0], W.v[0] = p[1], W.v[1] = p[2], W.v[2] = p[3], W.p = p[4];
+  if (conv)
+    U.d = p[5], U.v[0] = p[6], U.v[1] = p[7], U.v[2] = p[8], U.p = p[9];
+  else
+    p2c<double, Ieee, EOS>(d.Gg, W, U);
+  st(d.U4, c, make_double4(U.d, U.v[0], U.v[1], U.v[2]));
+  st(d.UE, c, U.p);
+  if (MIXED) {
+    store_W32<EOS>(d, d.Wva, d.Wsg, c, W);
+  } else {
+    st(d.W4, c, make_double4(W.d, W.v[0], W.v[1], W.v[2]));
+    st(d.Wp, c, W.p);
+  }
+}
+
+// W and/or U of n cells into the chunk.  On the mixed path the FP64 W is
+// recovered from U by c2p, started from the record's pressure; where c2p fails
+// it is the record's.
+template <bool MIXED, int EOS>
+__global__ __launch_bounds__(kBlock) void k_pack_state(Dev d, const int32_t *old_to_new, int first, int n, bool phys,
+                                                       bool conv, double *staged) {
+  __shared__ __align__(16) double buf[10 * kBlock];
+  const int b0 = blockIdx.x * kBlock, w = (phys ? 5 : 0) + (conv ? 5 : 0);
+  const int m = n - b0 < kBlock ? n - b0 : kBlock;
+  if ((int)threadIdx.x < m) {
+    const int c = old_to_new[first + b0 + threadIdx.x];
+    double *p = buf + threadIdx.x * w;
+    State<double> W, U;
+    if (MIXED || conv) load_U(d, c, U);
+    if (phys) {
+      if (MIXED) {
+        load_W32(d, c, W);
+        int it = 0;
+        c2p<Ieee, EOS>(d.Gg, U, W, W.p, it);
+      } else {
+        load_W(d, c, W);
+      }
+      p[0] = W.d, p[1] = W.v[0], p[2] = W.v[1], p[3] = W.v[2], p[4] = W.p;
+      p += 5;
+    }
+    if (conv) p[0] = U.d, p[1] = U.v[0], p[2] = U.v[1], p[3] = U.v[2], p[4] = U.p;
+  }
+  __syncthreads();
+  staged_store(staged + (size_t)b0 * w, buf, m * w);
+}
+
+// Face fluxes of n faces into the chunk, FP64 with the E flux in the energy
+// slot (mixed path: D flux + tau flux): recomputed as the tiled step computes
+// them, or the two-kernel step's stored ones.
+template <bool MIXED, bool STORED, int EOS>
+__global__ __launch_bounds__(kBlock) void k_face_out(Dev d, const int32_t *old_to_new, int first, int n,
+                                                     double *staged) {
+  __shared__ __align__(16) double buf[5 * kBlock];
+  const int b0 = blockIdx.x * kBlock;
+  const int m = n - b0 < kBlock ? n - b0 : kBlock;
+  if ((int)threadIdx.x < m) {
+    const int i = old_to_new[first + b0 + threadIdx.x];
+    State<double> F;
+    if (STORED) {
+      load_flux<MIXED>(d, i, F);
+    } else {
+      (void)face_flux<MIXED, EOS>(d, i, F);
+      if (MIXED) F.p = F.d + F.p;
+    }
+    double *p = buf + threadIdx.x * 5;
+    p[0] = F.d, p[1] = F.v[0], p[2] = F.v[1], p[3] = F.v[2], p[4] = F.p;
+  }
+  __syncthreads();
+  staged_store(staged + (size_t)b0 * 5, buf, m * 5);
+}
+
+__global__ __launch_bounds__(kBlock) void k_unpack_fields(const int32_t *old_to_new, int first, int n,
+                                                          const float *staged, float4 *FU, float2 *k, bool kappa,
+                                                          float *T) {
+  __shared__ float buf[15 * kBlock];
+  const int b0 = blockIdx.x * kBlock;
+  const int m = n - b0 < kBlock ? n - b0 : kBlock;
+  const float *src = staged;  // regions of n entries of 1, 3, 1, 1 and 9 floats
+  float *Ur = buf, *Fr = buf + kBlock, *ka = buf + 4 * kBlock, *ks = buf + 5 * kBlock, *Tr = buf + 6 * kBlock;
+  auto region = [&](float *lds, int w) {
+    staged_load(src + (size_t)b0 * w, lds, m * w);
+    src += (size_t)n * w;
+  };
+  if (FU) region(Ur, 1), region(Fr, 3);
+  if (kappa) region(ka, 1), region(ks, 1);
+  if (T) region(Tr, 9);
+  __syncthreads();
+  const int j = threadIdx.x;
+  if (j >= m) return;
+  const int c = old_to_new[first + b0 + j];
+  if (FU) FU[c] = make_float4(Fr[3 * j], Fr[3 * j + 1], Fr[3 * j + 2], Ur[j]);
+  if (k) k[c] = kappa ? make_float2(ka[j], ks[j]) : make_float2(0.f, 0.f);
+  if (T)
+    for (int i = 0; i < 9; ++i) T[9 * (size_t)c + i] = Tr[9 * j + i];
+}
+
 // Clears the counters and speed slots with plain stores (graph-safe).
 __global__ void k_clear(Dev d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -793,12 +874,60 @@ static inline unsigned int face_blocks(int64_t n) {
   return (unsigned int)((n + kBlock * kFacesPerThread - 1) / (kBlock * kFacesPerThread));
 }
 
-hipError_t launch_p2c_init(const Dev &d, hipStream_t s) {
-  if (d.n_cells == 0) return hipSuccess;
-  if (d.eos == kTaub)
-    hipLaunchKernelGGL(k_p2c_init<kTaub>, dim3(blocks_for(d.n_cells)), dim3(kBlock), 0, s, d);
+template <bool MIXED, int EOS>
+static void pack_state_v(const Dev &d, const int32_t *o2n, int first, int n, bool phys, bool conv, double *staged,
+                         hipStream_t s) {
+  hipLaunchKernelGGL((k_pack_state<MIXED, EOS>), dim3(blocks_for(n)), dim3(kBlock), 0, s, d, o2n, first, n, phys, conv,
+                     staged);
+}
+template <bool MIXED, int EOS>
+static void unpack_state_v(const Dev &d, const int32_t *o2n, int first, int n, bool conv, bool reset,
+                           const double *staged, hipStream_t s) {
+  hipLaunchKernelGGL((k_unpack_state<MIXED, EOS>), dim3(blocks_for(n)), dim3(kBlock), 0, s, d, o2n, first, n, conv,
+                     reset, staged);
+}
+template <bool MIXED, int EOS>
+static void face_out_v(const Dev &d, bool stored, const int32_t *o2n, int first, int n, double *staged,
+                       hipStream_t s) {
+  if (stored)
+    hipLaunchKernelGGL((k_face_out<MIXED, true, EOS>), dim3(blocks_for(n)), dim3(kBlock), 0, s, d, o2n, first, n,
+                       staged);
   else
-    hipLaunchKernelGGL(k_p2c_init<kIdeal>, dim3(blocks_for(d.n_cells)), dim3(kBlock), 0, s, d);
+    hipLaunchKernelGGL((k_face_out<MIXED, false, EOS>), dim3(blocks_for(n)), dim3(kBlock), 0, s, d, o2n, first, n,
+                       staged);
+}
+
+hipError_t launch_unpack_state(const Dev &d, bool mixed, const int32_t *o2n, int first, int n, bool conv, bool reset,
+                               const double *staged, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  if (d.eos == kTaub)
+    (mixed ? unpack_state_v<true, kTaub> : unpack_state_v<false, kTaub>)(d, o2n, first, n, conv, reset, staged, s);
+  else
+    (mixed ? unpack_state_v<true, kIdeal> : unpack_state_v<false, kIdeal>)(d, o2n, first, n, conv, reset, staged, s);
+  return hipGetLastError();
+}
+hipError_t launch_pack_state(const Dev &d, bool mixed, const int32_t *o2n, int first, int n, bool phys, bool conv,
+                             double *staged, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  if (d.eos == kTaub)
+    (mixed ? pack_state_v<true, kTaub> : pack_state_v<false, kTaub>)(d, o2n, first, n, phys, conv, staged, s);
+  else
+    (mixed ? pack_state_v<true, kIdeal> : pack_state_v<false, kIdeal>)(d, o2n, first, n, phys, conv, staged, s);
+  return hipGetLastError();
+}
+hipError_t launch_face_out(const Dev &d, bool mixed, bool stored, const int32_t *o2n, int first, int n,
+                           double *staged, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  if (d.eos == kTaub)
+    (mixed ? face_out_v<true, kTaub> : face_out_v<false, kTaub>)(d, stored, o2n, first, n, staged, s);
+  else
+    (mixed ? face_out_v<true, kIdeal> : face_out_v<false, kIdeal>)(d, stored, o2n, first, n, staged, s);
+  return hipGetLastError();
+}
+hipError_t launch_unpack_fields(const int32_t *o2n, int first, int n, const float *staged, float4 *FU, float2 *k,
+                                bool kappa, float *T, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_unpack_fields, dim3(blocks_for(n)), dim3(kBlock), 0, s, o2n, first, n, staged, FU, k, kappa, T);
   return hipGetLastError();
 }
 
@@ -927,36 +1056,11 @@ hipError_t launch_tile(const Dev &d, bool mixed, int variant, bool rad, bool sta
   return hipGetLastError();
 }
 
-hipError_t launch_face_fp64_out(const Dev &d, bool mixed, double4 *F4, double *FE, hipStream_t s) {
-  if (d.n_faces == 0) return hipSuccess;
-  const dim3 g(blocks_for(d.n_faces)), b(kBlock);
-  if (d.eos == kTaub) {
-    if (mixed)
-      hipLaunchKernelGGL((k_face_fp64_out<true, kTaub>), g, b, 0, s, d, F4, FE);
-    else
-      hipLaunchKernelGGL((k_face_fp64_out<false, kTaub>), g, b, 0, s, d, F4, FE);
-  } else {
-    if (mixed)
-      hipLaunchKernelGGL((k_face_fp64_out<true, kIdeal>), g, b, 0, s, d, F4, FE);
-    else
-      hipLaunchKernelGGL((k_face_fp64_out<false, kIdeal>), g, b, 0, s, d, F4, FE);
-  }
-  return hipGetLastError();
-}
-
 hipError_t launch_dt(const Dev &d, hipStream_t s) {
   hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, s, d);
   return hipGetLastError();
 }
 
-hipError_t launch_seed_mixed(const Dev &d, hipStream_t s) {
-  if (d.n_cells == 0) return hipSuccess;
-  if (d.eos == kTaub)
-    hipLaunchKernelGGL(k_seed_mixed<kTaub>, dim3(blocks_for(d.n_cells)), dim3(kBlock), 0, s, d);
-  else
-    hipLaunchKernelGGL(k_seed_mixed<kIdeal>, dim3(blocks_for(d.n_cells)), dim3(kBlock), 0, s, d);
-  return hipGetLastError();
-}
 hipError_t launch_ghost_cell(const Dev &d, bool mixed, hipStream_t s) {
   if (d.eos == kTaub)
     hipLaunchKernelGGL(k_ghost_cell<kTaub>, dim3(1), dim3(64), 0, s, d, mixed);
@@ -964,15 +1068,6 @@ hipError_t launch_ghost_cell(const Dev &d, bool mixed, hipStream_t s) {
     hipLaunchKernelGGL(k_ghost_cell<kIdeal>, dim3(1), dim3(64), 0, s, d, mixed);
   return hipGetLastError();
 }
-hipError_t launch_recover_W(const Dev &d, hipStream_t s) {
-  if (d.n_cells == 0) return hipSuccess;
-  if (d.eos == kTaub)
-    hipLaunchKernelGGL(k_recover_W<kTaub>, dim3(blocks_for(d.n_cells)), dim3(kBlock), 0, s, d);
-  else
-    hipLaunchKernelGGL(k_recover_W<kIdeal>, dim3(blocks_for(d.n_cells)), dim3(kBlock), 0, s, d);
-  return hipGetLastError();
-}
-
 hipError_t launch_add_rad(const Dev &d, bool mixed, double tau, hipStream_t s) {
   if (d.n_cells == 0) return hipSuccess;
   const dim3 g(blocks_for(d.n_cells)), b(kBlock);

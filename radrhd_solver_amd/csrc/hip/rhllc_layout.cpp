@@ -75,7 +75,9 @@ bool build(const Options &opt, int64_t n_cells, const void *geo_cells, int64_t n
       for (int32_t f = 0; f < F; ++f) L.face_new_to_old[start[owner(f)]++] = f;
     }
   }
-  RawVec<int32_t> cnew(N), fnew(F);
+  RawVec<int32_t> &cnew = L.cell_old_to_new, &fnew = L.face_old_to_new;
+  cnew.resize(N);
+  fnew.resize(F);
 #pragma omp parallel for schedule(static)
   for (int32_t i = 0; i < N; ++i) cnew[L.cell_new_to_old[i]] = i;
 #pragma omp parallel for schedule(static)

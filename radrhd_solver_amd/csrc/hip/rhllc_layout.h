@@ -26,6 +26,7 @@ struct Options {
 
 struct Layout {
   std::vector<int32_t> cell_new_to_old, face_new_to_old;
+  rhllc_mesh::RawVec<int32_t> cell_old_to_new, face_old_to_new;
   // per face (left, right): right = the neighbour; N and N + 1 the ghost
   // states of codes -3 and -4; ~left (negative) a wall of code -2; left for
   // the copy-type codes

@@ -1,0 +1,64 @@
+#include "rhllc_records.h"
+
+#include <algorithm>
+#include <cstring>
+
+namespace rhllc_records {
+namespace {
+
+constexpr int64_t kField = 40;
+// Below this many bytes one thread is faster than waking the others.
+constexpr int64_t kParallelBytes = 1 << 18;
+
+template <typename Fn>
+void over_blocks(int64_t n, int64_t bytes_each, Fn fn) {
+  constexpr int64_t kBlock = 1024;
+  const int64_t nb = (n + kBlock - 1) / kBlock;
+#pragma omp parallel for schedule(static) if (n * bytes_each > kParallelBytes)
+  for (int64_t b = 0; b < nb; ++b) fn(b * kBlock, std::min(n, (b + 1) * kBlock));
+}
+
+}  // namespace
+
+void gather(const void *recs, int64_t stride, int64_t off_a, int64_t off_b, int64_t n, void *out) {
+  const uint8_t *r = static_cast<const uint8_t *>(recs);
+  uint8_t *o = static_cast<uint8_t *>(out);
+  const int64_t w = (off_a >= 0 ? kField : 0) + (off_b >= 0 ? kField : 0);
+  over_blocks(n, w, [=](int64_t i0, int64_t i1) {
+    if (stride == w && (off_a < 0 ? off_b : off_a) == 0 && (off_a < 0 || off_b < 0 || off_b == kField)) {
+      std::memcpy(o + i0 * w, r + i0 * w, (size_t)((i1 - i0) * w));
+      return;
+    }
+    for (int64_t i = i0; i < i1; ++i) {
+      uint8_t *q = o + i * w;
+      if (off_a >= 0) std::memcpy(q, r + i * stride + off_a, kField), q += kField;
+      if (off_b >= 0) std::memcpy(q, r + i * stride + off_b, kField);
+    }
+  });
+}
+
+void scatter(void *recs, int64_t stride, int64_t off_a, int64_t off_b, int64_t n, const void *in) {
+  uint8_t *r = static_cast<uint8_t *>(recs);
+  const uint8_t *o = static_cast<const uint8_t *>(in);
+  const int64_t w = (off_a >= 0 ? kField : 0) + (off_b >= 0 ? kField : 0);
+  over_blocks(n, w, [=](int64_t i0, int64_t i1) {
+    if (stride == w && (off_a < 0 ? off_b : off_a) == 0 && (off_a < 0 || off_b < 0 || off_b == kField)) {
+      std::memcpy(r + i0 * w, o + i0 * w, (size_t)((i1 - i0) * w));
+      return;
+    }
+    for (int64_t i = i0; i < i1; ++i) {
+      const uint8_t *q = o + i * w;
+      if (off_a >= 0) std::memcpy(r + i * stride + off_a, q, kField), q += kField;
+      if (off_b >= 0) std::memcpy(r + i * stride + off_b, q, kField);
+    }
+  });
+}
+
+void copy(void *dst, const void *src, size_t bytes) {
+  over_blocks(((int64_t)bytes + 63) / 64, 64, [=](int64_t i0, int64_t i1) {
+    const size_t a = (size_t)i0 * 64, b = std::min(bytes, (size_t)i1 * 64);
+    std::memcpy(static_cast<uint8_t *>(dst) + a, static_cast<const uint8_t *>(src) + a, b - a);
+  });
+}
+
+}  // namespace rhllc_records
