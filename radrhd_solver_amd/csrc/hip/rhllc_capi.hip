@@ -170,7 +170,8 @@ struct rhllc_solver {
   int32_t *face_old_to_new = nullptr;  // device, from the first download of face fluxes on
   rhllc_mesh::RawVec<int32_t> face_old_to_new_host;
   Staging staging;
-  Scalars *host_sc = nullptr;  // pinned staging of the device scalars (two: [1] holds an earlier value)
+  Scalars *host_sc = nullptr;   // pinned copy of the device scalars, written by the device
+  Scalars *host_sc_dev = nullptr;  // its device address
   unsigned long long fix_fail_seen = 0;  // fix_fail already reported by rhllc_step / rhllc_sync
   float4 *rad_FU = nullptr;
   float4 *rad_FU_add = nullptr;  // moments of rhllc_add_rad_flux
@@ -251,13 +252,15 @@ struct rhllc_solver {
 
   bool folds() const { return tiled && n_tiles <= kFoldMaxTiles; }
 
-  // One step from buffer cur; the tiled step flips cur and, if it folds, stays open.
-  hipError_t enqueue_step() {
+  // One step from buffer cur, at *tau or the device's own; the tiled step flips
+  // cur and, if it folds, stays open.  With a tau nothing is open before.
+  hipError_t enqueue_step(const double *tau = nullptr) {
     hipError_t e;
     if (tiled) {
       Dev x = dev(cur, cur ^ 1);
       x.slot = slot;
       x.fold = open;
+      if (tau) x.use_tau = 1, x.tau = *tau;
       e = launch_tile(x, mixed, variant, rad, prm.collect_stats != 0, n_tiles, tile_slots, stream);
       if (e == hipSuccess && variant == kMixedMlp) e = launch_cell_mlp(x, rad, prm.collect_stats != 0, stream);
       if (e == hipSuccess) {
@@ -265,25 +268,36 @@ struct rhllc_solver {
         cur ^= 1;
         slot = (slot + 1) % kSpeedBufs;
         open = true;
-        if (!folds()) e = close_steps();
+        if (!tau && !folds()) e = close_steps();
       }
       return e;
     }
-    const Dev x = now();
+    Dev x = now();
+    if (tau) x.use_tau = 1, x.tau = *tau;
     e = launch_face(x, mixed, stream);
+    x.use_tau = 0;  // the cell kernels read it from the scalars
     if (e == hipSuccess) e = enqueue_cells(x);
-    if (e == hipSuccess) e = launch_dt(x, stream);
-    if (e == hipSuccess) last_in = cur;
+    if (e == hipSuccess) {
+      last_in = cur;
+      open = true;
+      if (!tau) e = close_steps();
+    }
     return e;
   }
-  // Takes the open step's maximum into the device scalars (tau, t, max_speed).
-  hipError_t close_steps() {
+  // Takes the open step's maximum into the device scalars (tau, t, max_speed),
+  // and into host_sc what rhllc_step reports.
+  hipError_t close_steps(bool to_host = false) {
     if (!open) return hipSuccess;
     Dev x = now();
-    x.slot = (slot + kSpeedBufs - 1) % kSpeedBufs;
+    x.slot = tiled ? (slot + kSpeedBufs - 1) % kSpeedBufs : 0;
     slot = 0;
     open = false;
-    return launch_dt(x, stream);
+    return launch_dt(x, to_host ? host_sc_dev : nullptr, stream);
+  }
+  // The device scalars into host_sc, after everything queued so far.
+  hipError_t fetch_scalars() {
+    const hipError_t e = launch_report(d, host_sc_dev, stream);
+    return e == hipSuccess ? hipStreamSynchronize(stream) : e;
   }
   // Captures graph[cur]: kGraphSteps steps (tiled) or one (two-kernel).
   hipError_t capture() {
@@ -381,7 +395,8 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   h->variant = variant;
   HIP_TRY(hipSetDevice(p.device));
   HIP_TRY(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-  HIP_TRY(hipHostMalloc((void **)&h->host_sc, 2 * sizeof(Scalars), hipHostMallocDefault));
+  HIP_TRY(hipHostMalloc((void **)&h->host_sc, sizeof(Scalars), hipHostMallocDefault));
+  HIP_TRY(hipHostGetDevicePointer((void **)&h->host_sc_dev, h->host_sc, 0));
   // Large enough for a pass over all faces or cells, up to the chunk limit.
   HIP_TRY(h->staging.alloc(std::max((size_t)N * 80, (size_t)F * 40)));
 
@@ -480,7 +495,7 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   if (variant == kMixedMlp) HIP_TRY(h->alloc(&d.mlp_list, N));
   HIP_TRY(h->alloc(&d.sc, 1));
   HIP_TRY(h->alloc(&d.speed_slots, (size_t)kSpeedBufs * kSpeedSlots * kSlotStride));
-  std::memset(h->host_sc, 0, 2 * sizeof(Scalars));
+  std::memset(h->host_sc, 0, sizeof(Scalars));
   h->host_sc->tau = d.cfl_hmin / 1.0;
   h->host_sc->last_speed = 1.0;
   HIP_TRY(hipMemcpy(d.sc, h->host_sc, sizeof(Scalars), hipMemcpyHostToDevice));
@@ -557,11 +572,10 @@ extern "C" int rhllc_step(rhllc_solver *h, double tau, double *max_speed) {
   if (!h) return fail(RHLLC_ERR_ARG, "null handle");
   if (!h->ready()) return fail(RHLLC_ERR_STATE, "no state uploaded (or no MLP model set for RHLLC_GUESS_MLP)");
   HIP_TRY(hipSetDevice(h->prm.device));
-  h->host_sc->tau = tau;
-  HIP_TRY(hipMemcpyAsync(&h->d.sc->tau, &h->host_sc->tau, sizeof(double), hipMemcpyHostToDevice, h->stream));
-  HIP_TRY(h->enqueue_step());
-  HIP_TRY(h->close_steps());
-  HIP_TRY(hipMemcpyAsync(h->host_sc, h->d.sc, sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
+  // Two launches and a wait: tau goes in as an argument, and the speed, the
+  // next tau and the failures come back through pinned memory.
+  HIP_TRY(h->enqueue_step(&tau));
+  HIP_TRY(h->close_steps(true));
   HIP_TRY(hipStreamSynchronize(h->stream));
   const double s = h->host_sc->last_speed;
   if (max_speed) *max_speed = s;
@@ -595,8 +609,7 @@ extern "C" int rhllc_run(rhllc_solver *h, int32_t nsteps, int32_t use_graph) {
 extern "C" int rhllc_sync(rhllc_solver *h) {
   if (!h) return fail(RHLLC_ERR_ARG, "null handle");
   HIP_TRY(hipSetDevice(h->prm.device));
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  HIP_TRY(hipMemcpy(h->host_sc, h->d.sc, sizeof(Scalars), hipMemcpyDeviceToHost));
+  HIP_TRY(h->fetch_scalars());
   return report_step_errors(h);
 }
 
@@ -622,9 +635,8 @@ extern "C" int rhllc_set_time(rhllc_solver *h, double tau, double t) {
 extern "C" int rhllc_get_stats(rhllc_solver *h, rhllc_stats *out) {
   if (!h || !out) return fail(RHLLC_ERR_ARG, "null argument");
   HIP_TRY(hipSetDevice(h->prm.device));
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  Scalars s;
-  HIP_TRY(hipMemcpy(&s, h->d.sc, sizeof(Scalars), hipMemcpyDeviceToHost));
+  HIP_TRY(h->fetch_scalars());
+  const Scalars &s = *h->host_sc;
   std::memset(out, 0, sizeof(*out));
   out->steps = (int64_t)s.steps;
   for (int k = 0; k < 6; ++k) out->c2p_fail[k] = (int64_t)s.c2p_fail[k];
@@ -683,7 +695,7 @@ extern "C" int rhllc_download_face_flux(rhllc_solver *h, double *F) {
 // null: not given) into the device arrays, through the staging chunks in the
 // order launch_unpack_fields reads them.
 static hipError_t send_fields(rhllc_solver *h, const float *Ur, const float *Fr3, const float *ka, const float *ks,
-                              const float *Tr9, float4 *FU, float2 *k, float *T) {
+                              const float *Tr9, float4 *FU, float2 *k, float *T, bool mark = false) {
   const size_t each = sizeof(float) * ((FU ? 4 : 0) + (ka ? 2 : 0) + (T ? 9 : 0));
   return h->staging.send(
       h->n_cells, each, h->stream,
@@ -699,7 +711,7 @@ static hipError_t send_fields(rhllc_solver *h, const float *Ur, const float *Fr3
       },
       [&](int i, int n, void *chunk) {
         return launch_unpack_fields(h->cell_old_to_new, i, n, static_cast<const float *>(chunk), FU, k, ka != nullptr,
-                                    T, h->stream);
+                                    T, mark && i == 0 ? h->d.sc : nullptr, h->stream);
       });
 }
 
@@ -754,17 +766,14 @@ static int add_rad_flux(rhllc_solver *h, double tau, const float *Ur, const floa
   // source, also held by a captured graph) stay as they were.
   if (!h->rad_FU_add) HIP_TRY(hipMalloc((void **)&h->rad_FU_add, sizeof(float4) * N));
   if (Tr9 && !h->rad_T_add) HIP_TRY(hipMalloc((void **)&h->rad_T_add, sizeof(float) * 9 * N));
-  HIP_TRY(send_fields(h, Ur, Fr3, nullptr, nullptr, Tr9, h->rad_FU_add, nullptr, Tr9 ? h->rad_T_add : nullptr));
+  HIP_TRY(send_fields(h, Ur, Fr3, nullptr, nullptr, Tr9, h->rad_FU_add, nullptr, Tr9 ? h->rad_T_add : nullptr,
+                      true));
   Dev x = h->now();
   x.rad_FU = h->rad_FU_add;
   x.rad_T = Tr9 ? h->rad_T_add : nullptr;
-  // The failures counted before, in stream order: the source's own are the difference.
-  HIP_TRY(hipMemcpyAsync(&h->host_sc[1].fix_fail, &h->d.sc->fix_fail, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                         h->stream));
   HIP_TRY(launch_add_rad(x, h->mixed, tau, h->stream));
-  HIP_TRY(hipMemcpyAsync(h->host_sc, h->d.sc, sizeof(Scalars), hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  const unsigned long long now_failed = h->host_sc->fix_fail - h->host_sc[1].fix_fail;
+  HIP_TRY(h->fetch_scalars());
+  const unsigned long long now_failed = h->host_sc->fix_fail - h->host_sc->fix_mark;  // the source's own
   h->fix_fail_seen += now_failed;  // reported here; earlier steps' failures stay for rhllc_sync
   if (now_failed)
     return fail(RHLLC_ERR_C2P, std::to_string(now_failed) + " cells failed PhysPressureFix after the radiation source");
@@ -888,7 +897,7 @@ extern "C" int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]
         e = launch_cell_mlp(x, h->rad, stats, h->stream);
     }
     if (e == hipSuccess && e4) e = hipEventRecord(e4[2], h->stream);
-    if (e == hipSuccess) e = launch_dt(x, h->stream);
+    if (e == hipSuccess) e = launch_dt(x, nullptr, h->stream);
     if (e == hipSuccess && e4) e = hipEventRecord(e4[3], h->stream);
     if (e != hipSuccess) {
       rc = hip_fail(e, "kernel timing");

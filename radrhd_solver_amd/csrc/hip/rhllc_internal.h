@@ -36,6 +36,7 @@ struct Scalars {
   unsigned long long hist[kHistBins];
   unsigned long long max_residual_bits;
   unsigned long long mlp_starts;
+  unsigned long long fix_mark;  // fix_fail when the moments of rhllc_add_rad_flux arrived
   unsigned int mlp_count[kSpeedBufs];  // cells appended to Dev::mlp_list by the step of each slot buffer
 };
 
@@ -120,6 +121,9 @@ struct Dev {
   // sc: the tiled step then forms its tau from there (fold_speed).
   int32_t slot;
   int32_t fold;
+  // A step at the caller's tau (rhllc_step): its first kernel also puts it into sc.
+  int32_t use_tau;
+  double tau;
 };
 
 enum Variant : int {
@@ -140,8 +144,9 @@ hipError_t launch_pack_state(const Dev &d, bool mixed, const int32_t *old_to_new
 // Per-cell FP32 fields of cells [first, first + n): the regions Ur[n], Fr[3 n]
 // (with FU), kappa_a[n], kappa_s[n] (with kappa) and Tr[9 n] (with T) of
 // `staged` in this order, into the device numbering.  k without kappa: zeros.
+// mark (or null): mark->fix_mark = mark->fix_fail.
 hipError_t launch_unpack_fields(const int32_t *old_to_new, int first, int n, const float *staged, float4 *FU,
-                                float2 *k, bool kappa, float *T, hipStream_t s);
+                                float2 *k, bool kappa, float *T, Scalars *mark, hipStream_t s);
 hipError_t launch_face(const Dev &d, bool mixed, hipStream_t s);
 hipError_t launch_cell(const Dev &d, int variant, bool rad, bool stats, hipStream_t s);
 hipError_t launch_cell_mlp(const Dev &d, bool rad, bool stats, hipStream_t s);
@@ -155,8 +160,11 @@ hipError_t launch_tile(const Dev &d, bool mixed, int variant, bool rad, bool sta
 // two-kernel step's flux array.
 hipError_t launch_face_out(const Dev &d, bool mixed, bool stored, const int32_t *old_to_new, int first, int n,
                            double *staged, hipStream_t s);
-// Ends a step (or a run of folded steps): the maximum of slot buffer d.slot into sc.
-hipError_t launch_dt(const Dev &d, hipStream_t s);
+// Ends a step (or a run of folded steps): the maximum of slot buffer d.slot
+// into sc.  host (pinned, or null) receives tau, last_speed and fix_fail.
+hipError_t launch_dt(const Dev &d, Scalars *host, hipStream_t s);
+// All of sc into host (pinned).
+hipError_t launch_report(const Dev &d, Scalars *host, hipStream_t s);
 hipError_t launch_clear_scalars(const Dev &d, hipStream_t s);
 // Writes the ghost states into entries n_cells and n_cells + 1 of the input and output buffers
 // of d (U and W on the FP64 path, the cell record on the mixed path).

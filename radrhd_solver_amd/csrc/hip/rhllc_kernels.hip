@@ -124,6 +124,9 @@ struct StepClose {
 // each and the DPP reduction of the ROCm device library, so the other waves
 // skip the cross-lane steps.
 //
+// With d.use_tau the step runs at d.tau, which block 0 also puts into sc for the
+// kernels after this one (none of this launch reads it there).
+//
 // With d.fold the previous step's maximum has not been taken yet: the block's
 // last wave (the face loop leaves it the fewest faces) reads the 64 slots of
 // the buffer before and leaves tau in LDS before the same barrier, and block 0
@@ -136,7 +139,12 @@ __device__ __forceinline__ double fold_speed(const Dev &d, double speed) {
   __shared__ double tau_lds;
   part[threadIdx.x] = (unsigned long long)__double_as_longlong(speed);
   double tau = 0.0;
-  if (!d.fold) tau = d.sc->tau;  // before the barrier: a cold load
+  if (d.use_tau) {
+    tau = d.tau;
+    if (blockIdx.x == 0 && threadIdx.x == 0) d.sc->tau = tau;
+  } else if (!d.fold) {
+    tau = d.sc->tau;  // before the barrier: a cold load
+  }
   if (d.fold && threadIdx.x >= kBlock - 64) {
     const int prev = d.slot == 0 ? kSpeedBufs - 1 : d.slot - 1, next = d.slot == kSpeedBufs - 1 ? 0 : d.slot + 1;
     const double s = slots_max(d, prev);
@@ -652,11 +660,14 @@ __global__ __launch_bounds__(kBlock) void k_cell_mlp(Dev d) {
 // tau of the next step from the max signal speed (rhllc_utils.cpp:15-23):
 // tau = CFL*h_min / speed.  Also clears every slot buffer, so the next step
 // starts from buffer 0.  One wave.
-__global__ __launch_bounds__(64) void k_dt(Dev d) {
+__global__ __launch_bounds__(64) void k_dt(Dev d, Scalars *host) {
   const StepClose c(d, d.slot);
+  const unsigned long long fix_fail = d.sc->fix_fail;
   const double s = slots_max(d, d.slot);
   if (threadIdx.x == 0) {
-    c.store(d, s, d.cfl_hmin / s);
+    const double tau = d.cfl_hmin / s;
+    if (host) host->tau = tau, host->last_speed = s, host->fix_fail = fix_fail;
+    c.store(d, s, tau);
     for (int k = 0; k < kSpeedBufs; ++k) d.sc->mlp_count[k] = 0;
   }
 #pragma unroll
@@ -720,6 +731,15 @@ __global__ __launch_bounds__(kBlock) void k_add_rad(Dev d, double tau) {
     count_if(&d.sc->fix_calls, fixed);
     count_if(&d.sc->fix_fail, fix_failed);
   }
+}
+
+// The scalars for the host, as 8-byte words into pinned memory: a launch on the
+// stream in order, where a copy of a few hundred bytes costs two more.
+static_assert(sizeof(Scalars) % 8 == 0 && sizeof(Scalars) <= 8 * 128, "two words a lane");
+__global__ __launch_bounds__(64) void k_report(const Scalars *sc, Scalars *host) {
+  const unsigned long long *src = reinterpret_cast<const unsigned long long *>(sc);
+  unsigned long long *dst = reinterpret_cast<unsigned long long *>(host);
+  for (unsigned int k = threadIdx.x; k < sizeof(Scalars) / 8; k += 64) dst[k] = src[k];
 }
 
 // ------------------------------------------------------------ state transfer
@@ -831,7 +851,7 @@ __global__ __launch_bounds__(kBlock) void k_face_out(Dev d, const int32_t *old_t
 
 __global__ __launch_bounds__(kBlock) void k_unpack_fields(const int32_t *old_to_new, int first, int n,
                                                           const float *staged, float4 *FU, float2 *k, bool kappa,
-                                                          float *T) {
+                                                          float *T, Scalars *mark) {
   __shared__ float buf[15 * kBlock];
   const int b0 = blockIdx.x * kBlock;
   const int m = n - b0 < kBlock ? n - b0 : kBlock;
@@ -846,6 +866,7 @@ __global__ __launch_bounds__(kBlock) void k_unpack_fields(const int32_t *old_to_
   if (T) region(Tr, 9);
   __syncthreads();
   const int j = threadIdx.x;
+  if (mark && b0 == 0 && j == 0) mark->fix_mark = mark->fix_fail;
   if (j >= m) return;
   const int c = old_to_new[first + b0 + j];
   if (FU) FU[c] = make_float4(Fr[3 * j], Fr[3 * j + 1], Fr[3 * j + 2], Ur[j]);
@@ -925,9 +946,10 @@ hipError_t launch_face_out(const Dev &d, bool mixed, bool stored, const int32_t 
   return hipGetLastError();
 }
 hipError_t launch_unpack_fields(const int32_t *o2n, int first, int n, const float *staged, float4 *FU, float2 *k,
-                                bool kappa, float *T, hipStream_t s) {
+                                bool kappa, float *T, Scalars *mark, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_unpack_fields, dim3(blocks_for(n)), dim3(kBlock), 0, s, o2n, first, n, staged, FU, k, kappa, T);
+  hipLaunchKernelGGL(k_unpack_fields, dim3(blocks_for(n)), dim3(kBlock), 0, s, o2n, first, n, staged, FU, k, kappa, T,
+                     mark);
   return hipGetLastError();
 }
 
@@ -1056,8 +1078,12 @@ hipError_t launch_tile(const Dev &d, bool mixed, int variant, bool rad, bool sta
   return hipGetLastError();
 }
 
-hipError_t launch_dt(const Dev &d, hipStream_t s) {
-  hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, s, d);
+hipError_t launch_dt(const Dev &d, Scalars *host, hipStream_t s) {
+  hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, s, d, host);
+  return hipGetLastError();
+}
+hipError_t launch_report(const Dev &d, Scalars *host, hipStream_t s) {
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s, d.sc, host);
   return hipGetLastError();
 }
 
