@@ -321,7 +321,7 @@ int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, const float *X
  * (1 float) are device pointers; the work is enqueued on `stream` (a
  * hipStream_t; NULL = the null stream) and the caller synchronizes.  The
  * packed weights, per-wave partials and losses live in a scratch array the
- * library holds on each GPU (18.4 MB, for n <= RHLLC_MLP_NOALLOC_MAX_N; larger
+ * library holds on each GPU (18.5 MB, for n <= RHLLC_MLP_NOALLOC_MAX_N; larger
  * n is RHLLC_ERR_ARG); grad and loss are the same bits as rhllc_mlp_grad's.
  * Calls that overlap on one GPU share that scratch and race.  No counterpart
  * in the reference: for callers that cannot allocate (code under HIP graph

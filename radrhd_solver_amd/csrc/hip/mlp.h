@@ -70,12 +70,9 @@ __device__ __forceinline__ short f2bf(float x) {  // round to nearest even
 }
 __device__ __forceinline__ float bf2f(short b) { return __uint_as_float(((uint32_t)(uint16_t)b) << 16); }
 
-__device__ __forceinline__ float silu(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
-// d silu / dz = s (1 + z (1 - s)), s = sigmoid(z)
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
-  return s * (1.0f + z * (1.0f - s));
-}
+// silu = z s, d silu / dz = s (1 + z (1 - s)), s = sigmoid(z)
+__device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
+__device__ __forceinline__ float silu(float z) { return z * sigmoid(z); }
 
 // Frozen-Lorentz-factor pressure p0 (see the top of this file), floored at
 // 1e-12 D; NaN for E <= |m| (no physical state).

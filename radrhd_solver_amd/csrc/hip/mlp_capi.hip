@@ -87,7 +87,7 @@ extern "C" int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, con
   HIP_TRY(alloc(Xd, sizeof(float) * 3 * n));
   HIP_TRY(alloc(Yd, sizeof(float) * n));
   HIP_TRY(alloc(Od, sizeof(float) * n));
-  HIP_TRY(alloc(Gd, sizeof(float) * kParams * nw));
+  HIP_TRY(alloc(Gd, sizeof(float) * kGradStride * nw));
   HIP_TRY(alloc(Ld, sizeof(float) * nw));
   HIP_TRY(alloc(Sd, sizeof(float) * (kParams + 1)));
   HIP_TRY(hipMemcpy(P.p, model, sizeof(float) * kModel, hipMemcpyHostToDevice));
@@ -96,7 +96,7 @@ extern "C" int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, con
   HIP_TRY(hipMemcpy(Od.p, ok, sizeof(float) * n, hipMemcpyHostToDevice));
   HIP_TRY(launch_pack(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, nullptr));
   HIP_TRY(launch_grad(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, Xd.as<float>(), Yd.as<float>(),
-                      Od.as<float>(), 1.0f / (float)n, n, Gd.as<float>(), Ld.as<float>(), nullptr));
+                      Od.as<float>(), 1.0f / (float)n, n, Gd.as<float>(), Ld.as<float>(), nullptr, nullptr));
   HIP_TRY(launch_sum(Gd.as<float>(), Ld.as<float>(), nw, Sd.as<float>(), Sd.as<float>() + kParams, nullptr));
   HIP_TRY(hipDeviceSynchronize());
   HIP_TRY(hipMemcpy(grad, Sd.p, sizeof(float) * kParams, hipMemcpyDeviceToHost));
@@ -123,7 +123,7 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
   HIP_TRY(alloc(Xn, sizeof(float) * 3 * nn));
   HIP_TRY(alloc(Yn, sizeof(float) * nn));
   HIP_TRY(alloc(On, sizeof(float) * nn));
-  HIP_TRY(launch_gen(cfg->gamma, cfg->seed + 17, nullptr, nn, nullptr, Xn.as<float>(), Yn.as<float>(), On.as<float>(), st));
+  HIP_TRY(launch_gen(cfg->gamma, cfg->seed + 17, nn, nullptr, Xn.as<float>(), Yn.as<float>(), On.as<float>(), st));
   HIP_TRY(hipStreamSynchronize(st));
   std::vector<float> xh(3 * (size_t)nn), yh(nn), oh(nn);
   HIP_TRY(hipMemcpy(xh.data(), Xn.p, sizeof(float) * xh.size(), hipMemcpyDeviceToHost));
@@ -164,7 +164,7 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
   HIP_TRY(alloc(X, sizeof(float) * 3 * B));
   HIP_TRY(alloc(Y, sizeof(float) * B));
   HIP_TRY(alloc(O, sizeof(float) * B));
-  HIP_TRY(alloc(G, sizeof(float) * kParams * nw));
+  HIP_TRY(alloc(G, sizeof(float) * kGradStride * nw));
   HIP_TRY(alloc(L, sizeof(float) * nw));
   HIP_TRY(alloc(H, sizeof(float) * cfg->steps));
   HIP_TRY(alloc(S, 2 * sizeof(uint32_t)));
@@ -177,16 +177,17 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
   HIP_TRY(launch_pack(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, st));
   const float *norm = P.as<float>() + kOffNorm;
 
+  // The first step's samples; each step makes the next one's.
+  const Batch batch{cfg->gamma, cfg->seed, B, norm, X.as<float>(), Y.as<float>(), O.as<float>()};
+  HIP_TRY(launch_gen(cfg->gamma, cfg->seed, B, norm, batch.X, batch.Y, batch.OK, st));
   // One training step, captured once and replayed.
   HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  hipError_t e = launch_gen(cfg->gamma, cfg->seed, S.as<uint32_t>(), B, norm, X.as<float>(), Y.as<float>(),
-                            O.as<float>(), st);
-  if (e == hipSuccess)
-    e = launch_grad(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, X.as<float>(), Y.as<float>(),
-                    O.as<float>(), 1.0f / (float)B, B, G.as<float>(), L.as<float>(), st);
+  hipError_t e = launch_grad(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, batch.X, batch.Y, batch.OK,
+                             1.0f / (float)B, B, G.as<float>(), L.as<float>(), S.as<uint32_t>(), st);
   if (e == hipSuccess)
     e = launch_adam(P.as<float>(), M.as<float>(), V.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH,
-                    G.as<float>(), nw, S.as<uint32_t>(), cfg->steps, (float)cfg->lr, L.as<float>(), H.as<float>(), st);
+                    G.as<float>(), nw, S.as<uint32_t>(), cfg->steps, (float)cfg->lr, L.as<float>(), H.as<float>(),
+                    batch, st);
   hipGraph_t graph = nullptr;
   hipError_t e2 = hipStreamEndCapture(st, &graph);
   if (e != hipSuccess || e2 != hipSuccess) {
@@ -211,7 +212,7 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
 
 // ---------------------------------------------------------------- no-alloc
 // Scratch of rhllc_mlp_grad_noalloc: the packed BF16 weights (2 x 64 x 64
-// shorts = 4096 floats), the per-wave gradient partials (kParams floats a
+// shorts = 4096 floats), the per-wave gradient partials (kGradStride floats a
 // wave) and the per-wave losses, for batches of up to kNoAllocMaxN samples.
 // Each GPU holds its own copy until the process ends.  Host code uses the
 // device address hipGetSymbolAddress returns, never the array's name.
@@ -220,7 +221,7 @@ constexpr int kNoAllocMaxN = 65536;
 constexpr int kNoAllocMaxWaves = kNoAllocMaxN / 64;
 constexpr size_t kScratchW2 = 0;                                              // floats
 constexpr size_t kScratchGrad = kScratchW2 + (size_t)kH * kH;                 // 2 x 4096 shorts
-constexpr size_t kScratchLoss = kScratchGrad + (size_t)kParams * kNoAllocMaxWaves;
+constexpr size_t kScratchLoss = kScratchGrad + (size_t)kGradStride * kNoAllocMaxWaves;
 constexpr size_t kScratchFloats = kScratchLoss + kNoAllocMaxWaves;
 }  // namespace
 
@@ -263,7 +264,7 @@ extern "C" int rhllc_mlp_grad_noalloc(int32_t device, const float *model, int32_
   // Every scratch element these kernels read is written first in the same call
   // (pack: all of W2; grad: nw partial rows and nw losses), so nothing is cleared.
   HIP_TRY(launch_pack(model, W2b, W2b + kH * kH, st));
-  HIP_TRY(launch_grad(model, W2b, W2b + kH * kH, X, y, ok, 1.0f / (float)n, n, part, lpart, st));
+  HIP_TRY(launch_grad(model, W2b, W2b + kH * kH, X, y, ok, 1.0f / (float)n, n, part, lpart, nullptr, st));
   HIP_TRY(launch_sum(part, lpart, nw, grad, loss, st));
   return RHLLC_OK;
 }

@@ -1,14 +1,16 @@
 // Training and evaluation kernels of the c2p surrogate MLP (see mlp.h).
 //
 // Training step (captured in a hipGraph and replayed):
-//   k_mlp_gen    seeded primitives -> FP64 p2c -> FP64 c2p (reference start)
-//                -> normalised features/targets (failed states are masked);
 //   k_mlp_grad   one wave per 64 samples: forward (BF16 MFMA with K = 32,
 //                FP32 accumulate),
 //                backward, per-wave gradient partials written to global memory;
 //   k_mlp_adam   fixed-order sum of the partials (deterministic), Adam on the
 //                FP32 master weights, BF16 copies of W2 and W2^T, the step's
-//                loss, and the device step counter.
+//                loss and the device step counter; and on the CUs that the sum
+//                leaves idle the next step's samples: seeded primitives -> FP64
+//                p2c -> FP64 c2p (reference start) -> normalised features and
+//                targets (failed states are masked).
+// k_mlp_gen makes the samples of the normalisation and of the first step.
 #include <hip/hip_runtime.h>
 
 #include "mlp.h"
@@ -60,14 +62,9 @@ __device__ void make_sample(double gamma, uint64_t seed, uint64_t k, float x[3],
   if (!ok) x[0] = x[1] = x[2] = 0.0f;
 }
 
-// step: null, or {the next step's number, this step's}; see k_mlp_adam.
-__global__ void k_mlp_gen(double gamma, uint64_t seed, uint32_t *step, int n, const float *norm, float *X, float *Y,
-                          float *OK) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t now = step ? step[0] : 0u;
-  if (step && i == 0) step[1] = now;
-  const uint64_t k = (uint64_t)now * (uint64_t)n + (uint64_t)i;
+// Entry i of a batch: sample k of the stream, normalised unless norm is null.
+__device__ void put_sample(double gamma, uint64_t seed, uint64_t k, int i, const float *norm, float *X, float *Y,
+                           float *OK) {
   float x[3], y;
   int ok;
   make_sample(gamma, seed, k, x, y, ok);
@@ -80,19 +77,57 @@ __global__ void k_mlp_gen(double gamma, uint64_t seed, uint32_t *step, int n, co
   OK[i] = ok ? 1.0f : 0.0f;
 }
 
-// One wave = 64 consecutive samples.  grad[wave][kParams] receives the
+__global__ void k_mlp_gen(double gamma, uint64_t seed, int n, const float *norm, float *X, float *Y, float *OK) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) put_sample(gamma, seed, (uint64_t)i, i, norm, X, Y, OK);
+}
+
+// Four consecutive floats of the model, which a caller may hold at any float's
+// address (one 16-byte load either way).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f32x4u ld4(const float *p) { return *reinterpret_cast<const f32x4u *>(p); }
+
+// v plus v of the lane across bit 0, 1, 2 or 3 of the lane number, the sum of
+// 16 lanes in the order of a butterfly of lane exchanges: each level adds two
+// values that all lanes of their halves hold alike, so a mirrored lane serves
+// as well as the exchanged one.  One VALU instruction a level (DPP); the
+// exchange through LDS that __shfl_xor makes costs a round trip each.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float sum16(float v) {
+  v = dpp_add<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v = dpp_add<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v = dpp_add<0x141>(v);  // row_half_mirror
+  return dpp_add<0x140>(v);  // row_mirror
+}
+
+// Row length of the transposed operands in LDS: 64 samples and 4 shorts of
+// padding, so the 16 rows a load touches start in different banks.
+constexpr int kLdT = kH + 4;
+
+// One wave = 64 consecutive samples.  grad[wave][kGradStride] receives the
 // wave's gradient of sum_s ok_s (out_s - y_s)^2 * inv_n; loss[wave] the sum
-// of squared errors.
+// of squared errors.  A full batch is one wave per SIMD, so the kernel takes as
+// long as one wave's chain: the activations' derivatives are formed with them
+// from one sigmoid and kept instead of the pre-activations (128 exponentials a
+// lane, not 320), the sums over 16 lanes use DPP, the vectors come in 16-byte
+// loads and the LDS rows are padded: 38.2 -> 25.2 us at 65,536 samples, no
+// scratch (248 bytes a lane spilled before).
 __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, const short *__restrict__ W2b,
                                                   const short *__restrict__ W2Tb, const float *__restrict__ X,
                                                   const float *__restrict__ Y, const float *__restrict__ OK,
                                                   float inv_n, int n, float *__restrict__ grad,
-                                                  float *__restrict__ loss) {
-  __shared__ short lds[4][2][kH * kH];  // per wave: dZ2^T [h2][s] and H1^T [h1][s], bf16
+                                                  float *__restrict__ loss, uint32_t *step) {
+  if (step && blockIdx.x == 0 && threadIdx.x == 0) step[1] = step[0];
+  __shared__ __align__(16) short lds[4][2][kH * kLdT];  // per wave: dZ2^T [h2][s] and H1^T [h1][s], bf16
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = l >> 4, c = l & 15;
   const int wave = blockIdx.x * 4 + w;
   const int base = wave * 64;
+  short *dzT = lds[w][0];
+  short *h1T = lds[w][1];
   // own sample (lane l) and the 4 samples s_t = 16 t + c this lane works on
   float xl[3] = {0.f, 0.f, 0.f}, yl = 0.f, okl = 0.f;
   if (base + l < n) {
@@ -108,28 +143,36 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
     ok[t] = __shfl(okl, 16 * t + c, 64);
   }
   // ---- forward
-  float z1[4][4][4];  // [q][t][e]
+  float d1[4][4][4];  // [q][t][e] dsilu of layer 1
   bf16x4 h1[4][4];    // [q][t]
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
+  for (int q = 0; q < 4; ++q) {
+    const int h0 = 16 * q + 4 * g;
+    float wr[12];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int h = 16 * q + 4 * g + e;
-      const float w0 = P[kOffW1 + 3 * h], w1 = P[kOffW1 + 3 * h + 1], w2 = P[kOffW1 + 3 * h + 2], bb = P[kOffB1 + h];
+    for (int k = 0; k < 3; ++k) *reinterpret_cast<f32x4u *>(wr + 4 * k) = ld4(P + kOffW1 + 3 * h0 + 4 * k);
+    const f32x4u bb = ld4(P + kOffB1 + h0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const float z = ((w0 * x[t][0] + w1 * x[t][1]) + w2 * x[t][2]) + bb;
-        z1[q][t][e] = z;
-        h1[q][t][e] = f2bf(silu(z));
+        const float z = ((wr[3 * e] * x[t][0] + wr[3 * e + 1] * x[t][1]) + wr[3 * e + 2] * x[t][2]) + bb[e];
+        const float s = sigmoid(z);
+        d1[q][t][e] = s * (1.0f + z * (1.0f - s));
+        h1[q][t][e] = f2bf(z * s);
+        h1T[(h0 + e) * kLdT + 16 * t + c] = h1[q][t][e];
       }
-    }
-  float z2[4][4][4];  // [u][t][r] pre-activation of h2 = 16 u + 4 g + r, sample s_t
+  }
+  float a2[4][4][4], d2[4][4][4];  // [u][t][r] silu and dsilu of layer 2, unit 16 u + 4 g + r, sample s_t
+  f32x4u w3[4];
   float out[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     bf16x4 a[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const bf16x4 *>(W2b + (16 * u + c) * kH + 16 * q + 4 * g);
+    const f32x4u b2 = ld4(P + kOffB2 + 16 * u + 4 * g);
+    w3[u] = ld4(P + kOffW3 + 16 * u + 4 * g);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -137,9 +180,11 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
       for (int q = 0; q < 4; q += 2) acc = mfma32(a[q], a[q + 1], h1[q][t], h1[q + 1][t], acc);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int h2 = 16 * u + 4 * g + r;
-        z2[u][t][r] = acc[r] + P[kOffB2 + h2];
-        out[t] += P[kOffW3 + h2] * silu(z2[u][t][r]);
+        const float z = acc[r] + b2[r];
+        const float s = sigmoid(z);
+        a2[u][t][r] = z * s;
+        d2[u][t][r] = s * (1.0f + z * (1.0f - s));
+        out[t] += w3[u][r] * a2[u][t][r];
       }
     }
   }
@@ -154,35 +199,32 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
     dout[t] = 2.0f * d * inv_n;
     sq += d * d;
   }
-  // ---- layer 3 and b2, W3 gradients; dZ2
+  float *G = grad + (size_t)wave * kGradStride;
+  // ---- layer 3 and b2, W3 gradients (summed over the 16 sample lanes); dZ2
   bf16x4 dz2b[4][4];  // [u][t] as the B operand of dH1^T = W2^T dZ2^T
-  float gW3[4][4], gB2[4][4];  // [u][r]
 #pragma unroll
   for (int u = 0; u < 4; ++u)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int h2 = 16 * u + 4 * g + r;
-      const float w3 = P[kOffW3 + h2];
       float aw = 0.f, ab = 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const float z = z2[u][t][r];
-        aw += dout[t] * silu(z);
-        const float dz = dout[t] * w3 * dsilu(z);
+        aw += dout[t] * a2[u][t][r];
+        const float dz = dout[t] * w3[u][r] * d2[u][t][r];
         ab += dz;
         dz2b[u][t][r] = f2bf(dz);
+        dzT[(16 * u + 4 * g + r) * kLdT + 16 * t + c] = dz2b[u][t][r];
       }
-      gW3[u][r] = aw, gB2[u][r] = ab;
+      aw = sum16(aw), ab = sum16(ab);
+      if (c == 0) G[kOffW3 + 16 * u + 4 * g + r] = aw, G[kOffB2 + 16 * u + 4 * g + r] = ab;
     }
   // ---- dH1^T = W2^T dZ2^T  (tiles q over h1, t over samples), then dZ1
-  float gW1[4][4][3], gB1[4][4];  // [q][e]
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     bf16x4 a[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) a[u] = *reinterpret_cast<const bf16x4 *>(W2Tb + (16 * q + c) * kH + 16 * u + 4 * g);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) gW1[q][e][0] = gW1[q][e][1] = gW1[q][e][2] = gB1[q][e] = 0.f;
+    float gW1[4][3] = {}, gB1[4] = {};
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -190,31 +232,22 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
       for (int u = 0; u < 4; u += 2) acc = mfma32(a[u], a[u + 1], dz2b[u][t], dz2b[u + 1][t], acc);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float dz = acc[e] * dsilu(z1[q][t][e]);
-        gB1[q][e] += dz;
-        gW1[q][e][0] += dz * x[t][0];
-        gW1[q][e][1] += dz * x[t][1];
-        gW1[q][e][2] += dz * x[t][2];
+        const float dz = acc[e] * d1[q][t][e];
+        gB1[e] += dz;
+        gW1[e][0] += dz * x[t][0];
+        gW1[e][1] += dz * x[t][1];
+        gW1[e][2] += dz * x[t][2];
       }
     }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float v0 = sum16(gW1[e][0]), v1 = sum16(gW1[e][1]), v2 = sum16(gW1[e][2]), vb = sum16(gB1[e]);
+      const int h = 16 * q + 4 * g + e;
+      if (c == 0) G[kOffW1 + 3 * h] = v0, G[kOffW1 + 3 * h + 1] = v1, G[kOffW1 + 3 * h + 2] = v2, G[kOffB1 + h] = vb;
+    }
   }
-  // ---- dW2 = dZ2^T H1 via an LDS transpose of both operands
-  short *dzT = lds[w][0];
-  short *h1T = lds[w][1];
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dzT[(16 * u + 4 * g + r) * kH + 16 * t + c] = dz2b[u][t][r];
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) h1T[(16 * q + 4 * g + e) * kH + 16 * t + c] = h1[q][t][e];
+  // ---- dW2 = dZ2^T H1 from the transposed operands in LDS
   __syncthreads();
-  float *G = grad + (size_t)wave * kParams;
 #pragma unroll
   for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -222,7 +255,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int t = 0; t < 4; t += 2) {
-        const short *ar = dzT + (16 * u + c) * kH + 4 * g, *br = h1T + (16 * q + c) * kH + 4 * g;
+        const short *ar = dzT + (16 * u + c) * kLdT + 4 * g, *br = h1T + (16 * q + c) * kLdT + 4 * g;
         acc = mfma32(*reinterpret_cast<const bf16x4 *>(ar + 16 * t), *reinterpret_cast<const bf16x4 *>(ar + 16 * t + 16),
                      *reinterpret_cast<const bf16x4 *>(br + 16 * t), *reinterpret_cast<const bf16x4 *>(br + 16 * t + 16),
                      acc);
@@ -230,50 +263,30 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
 #pragma unroll
       for (int r = 0; r < 4; ++r) G[kOffW2 + (16 * u + 4 * g + r) * kH + 16 * q + c] = acc[r];
     }
-  // ---- reduce the per-lane partials over the 16 sample lanes (c) of each group g
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float a = gW3[u][r], b = gB2[u][r];
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
-      if (c == 0) G[kOffW3 + 16 * u + 4 * g + r] = a, G[kOffB2 + 16 * u + 4 * g + r] = b;
-    }
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float v[4] = {gW1[q][e][0], gW1[q][e][1], gW1[q][e][2], gB1[q][e]};
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) v[k] += __shfl_xor(v[k], o, 64);
-      const int h = 16 * q + 4 * g + e;
-      if (c == 0) G[kOffW1 + 3 * h] = v[0], G[kOffW1 + 3 * h + 1] = v[1], G[kOffW1 + 3 * h + 2] = v[2], G[kOffB1 + h] = v[3];
-    }
   // b3: sum of dout over the wave's samples (group g = 0 holds each sample once)
   float db = (g == 0) ? (dout[0] + dout[1] + dout[2] + dout[3]) : 0.f;
   float ls = (g == 0) ? sq : 0.f;
+  db = sum16(db), ls = sum16(ls);
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) db += __shfl_xor(db, o, 64), ls += __shfl_xor(ls, o, 64);
+  for (int o = 16; o < 64; o <<= 1) db += __shfl_xor(db, o, 64), ls += __shfl_xor(ls, o, 64);
   if (l == 0) G[kOffB3] = db, loss[wave] = ls;
 }
 
-// Fixed-order column sums of the wave partials: column p of the nw x kParams
+// Fixed-order column sums of the wave partials: column p of the nw x kGradStride
 // array, added in row (wave) order in FP32, whatever the grid.  One thread per
 // column walking the rows waits for memory once per few rows (289 us for the
 // 1,024 rows of a 65,536-sample batch).  Here a workgroup of 1,024 threads owns
 // kSumCols columns: all of it loads kSumRows rows into LDS, 16 loads in flight a
 // thread and the next chunk's loads issued before the current one is added, and
 // one thread per column adds from LDS in order.  32 columns are one 128-byte
-// line of a row and make 141 workgroups of the 4,481 columns; with 64 columns
-// half the chip would idle.
+// line of a row and make 141 workgroups of the 4,481 columns; the training step
+// gives the CUs they leave the next step's samples.
 constexpr int kSumCols = 32;
 constexpr int kSumRows = 512;
 constexpr int kSumThreads = 1024;
 constexpr int kSumPer = kSumRows * kSumCols / kSumThreads;          // rows a thread loads of a chunk
 constexpr int kSumBlocks = (kParams + kSumCols - 1) / kSumCols;     // workgroups of the columns
+static_assert(kGradStride == kSumBlocks * kSumCols, "a partial's row is the workgroups' columns");
 static_assert(kSumThreads % kSumCols == 0 && kSumPer * (kSumThreads / kSumCols) == kSumRows, "chunk split");
 
 // The sum of column col0 + threadIdx.x in the threads below kSumCols (0 for
@@ -288,7 +301,7 @@ __device__ __forceinline__ float ordered_column_sum(const float *__restrict__ pa
 #pragma unroll
     for (int k = 0; k < kSumPer; ++k) {
       const int r = base + r0 + k * kStep;
-      v[k] = in && r < nw ? part[(size_t)r * kParams + col0 + c] : 0.f;
+      v[k] = in && r < nw ? part[(size_t)r * kGradStride + col0 + c] : 0.f;
     }
   };
   load(0);
@@ -339,15 +352,24 @@ __device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss
 }
 
 // Sum of the wave partials in wave order, then Adam (bias-corrected) with a
-// cosine learning-rate schedule.  The last workgroup sums the losses instead
-// and advances the step: step[1] is this step's number, which k_mlp_gen copied
+// cosine learning-rate schedule.  The next workgroup sums the losses instead
+// and advances the step: step[1] is this step's number, which k_mlp_grad copied
 // from step[0]; only this workgroup writes step[0], which nobody reads here.
+// The workgroups after it write the next step's samples, which k_mlp_grad of
+// this step has finished reading (a launch of 6.7 us by itself).
 __global__ __launch_bounds__(kSumThreads) void k_mlp_adam(float *P, float *Mo, float *Vo, short *W2b, short *W2Tb,
                                                           const float *grad, int nwaves, uint32_t *step,
                                                           int total_steps, float lr0, const float *loss,
-                                                          float *loss_hist) {
+                                                          float *loss_hist, Batch next) {
   __shared__ float lds[kSumRows][kSumCols];
   const uint32_t s = step[1];
+  if (blockIdx.x > kSumBlocks) {
+    const int i = (blockIdx.x - kSumBlocks - 1) * kSumThreads + threadIdx.x;
+    if (i < next.n)
+      put_sample(next.gamma, next.seed, (uint64_t)(s + 1u) * (uint64_t)next.n + (uint64_t)i, i, next.norm, next.X,
+                 next.Y, next.OK);
+    return;
+  }
   if (blockIdx.x == kSumBlocks) {
     const float t = ordered_loss_sum(loss, nwaves, &lds[0][0]);
     if (threadIdx.x == 0) {
@@ -447,22 +469,23 @@ __global__ void k_mlp_selftest(float *out) {
   for (int r = 0; r < 4; ++r) out[4 * l + r] = acc[r];
 }
 
-hipError_t launch_gen(double gamma, uint64_t seed, uint32_t *step, int n, const float *norm, float *X, float *Y,
-                      float *OK, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_gen, dim3((n + 255) / 256), dim3(256), 0, s, gamma, seed, step, n, norm, X, Y, OK);
+hipError_t launch_gen(double gamma, uint64_t seed, int n, const float *norm, float *X, float *Y, float *OK,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(k_mlp_gen, dim3((n + 255) / 256), dim3(256), 0, s, gamma, seed, n, norm, X, Y, OK);
   return hipGetLastError();
 }
 hipError_t launch_grad(const float *P, const short *W2b, const short *W2Tb, const float *X, const float *Y,
-                       const float *OK, float inv_n, int n, float *grad, float *loss, hipStream_t s) {
+                       const float *OK, float inv_n, int n, float *grad, float *loss, uint32_t *step, hipStream_t s) {
   // n is a multiple of 256 (4 waves of 64 samples per workgroup)
-  hipLaunchKernelGGL(k_mlp_grad, dim3(n / 256), dim3(256), 0, s, P, W2b, W2Tb, X, Y, OK, inv_n, n, grad, loss);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(n / 256), dim3(256), 0, s, P, W2b, W2Tb, X, Y, OK, inv_n, n, grad, loss, step);
   return hipGetLastError();
 }
 hipError_t launch_adam(float *P, float *M, float *V, short *W2b, short *W2Tb, const float *grad, int nwaves,
                        uint32_t *step, int total_steps, float lr0, const float *loss, float *loss_hist,
-                       hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_adam, dim3(kSumBlocks + 1), dim3(kSumThreads), 0, s, P, M, V, W2b, W2Tb, grad, nwaves, step,
-                     total_steps, lr0, loss, loss_hist);
+                       const Batch &next, hipStream_t s) {
+  const unsigned int blocks = kSumBlocks + 1 + (next.n + kSumThreads - 1) / kSumThreads;
+  hipLaunchKernelGGL(k_mlp_adam, dim3(blocks), dim3(kSumThreads), 0, s, P, M, V, W2b, W2Tb, grad, nwaves, step,
+                     total_steps, lr0, loss, loss_hist, next);
   return hipGetLastError();
 }
 hipError_t launch_sum(const float *part, const float *lpart, int nw, float *grad, float *loss, hipStream_t s) {
