@@ -37,6 +37,7 @@ struct Scalars {
   unsigned long long max_residual_bits;
   unsigned long long mlp_starts;
   unsigned long long fix_mark;  // fix_fail when the moments of rhllc_add_rad_flux arrived
+  unsigned int unusual;  // FP64 path: a state that is not `ordinary` was stored (stays set)
   unsigned int mlp_count[kSpeedBufs];  // cells appended to Dev::mlp_list by the step of each slot buffer
 };
 

@@ -225,7 +225,8 @@ __device__ __forceinline__ FaceIn<MIXED> tile_face_in(const Dev &d, int t, int i
 // One face: gather of the two cells' state at the start of the step, HLLC
 // flux into F (S * flux in the global frame; on the mixed path F.p is the
 // flux of tau = E - D); returns max(lL, lR).
-template <bool MIXED, int EOS>
+// A: the FP64 path's arithmetic, IeeeOrd when the stored states are ordinary.
+template <bool MIXED, int EOS, typename A = Ieee>
 __device__ __forceinline__ double face_flux(const Dev &d, const FaceIn<MIXED> &fi, State<double> &F) {
   const int2 lr = fi.lr;
   if constexpr (!MIXED) {
@@ -241,7 +242,7 @@ __device__ __forceinline__ double face_flux(const Dev &d, const FaceIn<MIXED> &f
       wall_mirror(nS.x, nS.y, nS.z, UR.v);
       wall_mirror(nS.x, nS.y, nS.z, WR.v);
     }
-    return hllc_flux<double, Ieee, EOS>(d.gamma, d.Gg, UL, UR, WL, WR, nS.x, nS.y, nS.z, nS.w, F);
+    return hllc_flux<double, A, EOS>(d.gamma, d.Gg, UL, UR, WL, WR, nS.x, nS.y, nS.z, nS.w, F);
   } else {
     // FP32 cell records, FP64 geometry and arithmetic with the fast
     // divide/sqrt policy.
@@ -406,6 +407,24 @@ __device__ __forceinline__ void update_U(const Dev &d, int c, double tau, const 
   dtau = s.p - s.d;
 }
 
+// Every kernel that stores an FP64 state calls this: the faces of a step use
+// IeeeOrd only while all stored states are ordinary.
+__device__ __forceinline__ void note_unusual(const Dev &d, const State<double> &U, const State<double> &W) {
+  if (!(ordinary(U) & ordinary(W))) d.sc->unusual = 1;
+}
+
+// c2p of a cell: on the FP64 path IeeeOrd where the state is ordinary.
+template <bool MIXED, int EOS>
+__device__ __forceinline__ int cell_c2p(const Dev &d, const State<double> &U, State<double> &W, double guess,
+                                        int &iters) {
+  if constexpr (MIXED) {
+    return c2p<Fast, EOS>(d.Gg, U, W, guess, iters);
+  } else {
+    // (No quotient has the start p alone above or below the line; alpha = E + p must not overflow.)
+    return ordinary(U) & (guess < 0x1p100) ? c2p<IeeeOrd, EOS>(d.Gg, U, W, guess, iters) : c2p<Ieee, EOS>(d.Gg, U, W, guess, iters);
+  }
+}
+
 // The radiation source of one cell and the c2p after it, from the cell's
 // state W after the hydro update; U and W are updated in place.
 //   radRHD_main.cpp:117-132: U += (ds*tau)*G(W), ds = 1, then c2p (code ignored).
@@ -434,14 +453,14 @@ __device__ __forceinline__ void apply_rad(const Dev &d, int c, double tau, State
   U.v[1] += ds * tau * G[2];
   U.v[2] += ds * tau * G[3];
   int it = 0;
-  int code = c2p<A, EOS>(d.Gg, U, W, MIXED ? W.p : -1.0, it);
+  int code = cell_c2p<MIXED, EOS>(d, U, W, MIXED ? W.p : -1.0, it);
   iters += it;
   if (d.tab && code) {
     // HllcConvToPhys: the reference start, then PhysPressureFix of the state
     // that c2p left (the pre-source W).
     if (MIXED) {
       it = 0;
-      code = c2p<A, EOS>(d.Gg, U, W, -1.0, it);
+      code = cell_c2p<MIXED, EOS>(d, U, W, -1.0, it);
       iters += it;
     }
     if (code) {
@@ -461,24 +480,23 @@ template <int VARIANT, bool RAD, bool STATS, int EOS>
 __device__ __forceinline__ void finish_cell(const Dev &d, int c, bool live, State<double> U, double guess,
                                             bool from_mlp, double tau) {
   constexpr bool MIXED = VARIANT >= kMixedPrev;
-  using A = typename std::conditional<MIXED, Fast, Ieee>::type;
   int iters = 0, code = 0;
   bool fell_back = false, fixed = false, fix_failed = false;
   double resid = 0.0;
   State<double> W;
   if (live) {
     // c2p writes W only when it succeeds.
-    code = c2p<A, EOS>(d.Gg, U, W, guess, iters);
+    code = cell_c2p<MIXED, EOS>(d, U, W, guess, iters);
     if (code && from_mlp) {
       int it2 = 0;
       fell_back = true;
-      code = c2p<A, EOS>(d.Gg, U, W, (double)ld(d.Wva, c).w, it2);
+      code = cell_c2p<MIXED, EOS>(d, U, W, (double)ld(d.Wva, c).w, it2);
       iters += it2;
     }
     if (code && VARIANT != kFp64Ref) {
       int it2 = 0;
       fell_back = true;
-      code = c2p<A, EOS>(d.Gg, U, W, -1.0, it2);
+      code = cell_c2p<MIXED, EOS>(d, U, W, -1.0, it2);
       iters += it2;
     }
     if (code) {
@@ -497,6 +515,7 @@ __device__ __forceinline__ void finish_cell(const Dev &d, int c, bool live, Stat
     if (!MIXED) {
       st(d.W4o, c, make_double4(W.d, W.v[0], W.v[1], W.v[2]));
       st(d.Wpo, c, W.p);
+      note_unusual(d, U, W);
     } else {
       store_W32<EOS>(d, d.Wvao, d.Wsgo, c, W);
     }
@@ -607,17 +626,26 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
   double2 *A = lds_flux, *B = lds_flux + nf;
   double *C = reinterpret_cast<double *>(lds_flux + 2 * nf);
   double speed = 0.0;
-  for (int k = threadIdx.x; k < nf; k += kBlock) {
-    // One index into one set of arrays (the extra faces' copies follow the
-    // faces): a select between two sets of base pointers would hold them in
-    // VGPRs through the loop.
-    const FaceIn<MIXED> fi = tile_face_in<MIXED>(d, t, k < tm.y ? tm.x + k : d.n_faces + tm.z + (k - tm.y));
-    State<double> F;
-    speed = smax(speed, face_flux<MIXED, EOS>(d, fi, F));
-    A[k] = make_double2(F.d, F.v[0]);
-    B[k] = make_double2(F.v[1], F.v[2]);
-    C[k] = F.p;
-  }
+  auto faces = [&](auto arith) {
+    for (int k = threadIdx.x; k < nf; k += kBlock) {
+      // One index into one set of arrays (the extra faces' copies follow the
+      // faces): a select between two sets of base pointers would hold them in
+      // VGPRs through the loop.
+      const FaceIn<MIXED> fi = tile_face_in<MIXED>(d, t, k < tm.y ? tm.x + k : d.n_faces + tm.z + (k - tm.y));
+      State<double> F;
+      speed = smax(speed, face_flux<MIXED, EOS, decltype(arith)>(d, fi, F));
+      A[k] = make_double2(F.d, F.v[0]);
+      B[k] = make_double2(F.v[1], F.v[2]);
+      C[k] = F.p;
+    }
+  };
+  // The FP64 faces of ordinary states, all of a step's input or none (a flag
+  // set in this launch concerns the next step's input; either way the bits are
+  // the same).
+  if (!MIXED && d.sc->unusual == 0)
+    faces(IeeeOrd());
+  else
+    faces(Ieee());
   const double tau = fold_speed(d, speed);  // its barrier also publishes the LDS fluxes
   const int c = t * d.tile_cells + (int)threadIdx.x;
   bool live = (int)threadIdx.x < d.tile_cells && c < d.n_cells;
@@ -693,6 +721,9 @@ __global__ void k_ghost_cell(Dev d, bool mixed) {
   const double4 w = make_double4(W.d, W.v[0], W.v[1], W.v[2]);
   d.U4[c] = u, d.UE[c] = gu[4], d.W4[c] = w, d.Wp[c] = W.p;
   d.U4o[c] = u, d.UEo[c] = gu[4], d.W4o[c] = w, d.Wpo[c] = W.p;
+  State<double> U;
+  U.d = gu[0], U.v[0] = gu[1], U.v[1] = gu[2], U.v[2] = gu[3], U.p = gu[4];
+  if (W.d != 0.0 || U.d != 0.0) note_unusual(d, U, W);  // an entry that no face uses is all zeros
 }
 
 // The radiation source on its own, after a step without it: AddRadFlux then
@@ -723,6 +754,7 @@ __global__ __launch_bounds__(kBlock) void k_add_rad(Dev d, double tau) {
     if (!MIXED) {
       d.W4[c] = make_double4(W.d, W.v[0], W.v[1], W.v[2]);
       d.Wp[c] = W.p;
+      note_unusual(d, U, W);
     } else {
       store_W32<EOS>(d, d.Wva, d.Wsg, c, W);
     }
@@ -790,6 +822,7 @@ __global__ __launch_bounds__(kBlock) void k_unpack_state(Dev d, const int32_t *o
   } else {
     st(d.W4, c, make_double4(W.d, W.v[0], W.v[1], W.v[2]));
     st(d.Wp, c, W.p);
+    note_unusual(d, U, W);
   }
 }
 
