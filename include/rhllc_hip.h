@@ -216,8 +216,8 @@ int rhllc_add_rad_flux_tensor(rhllc_solver *h, double tau, const float *Ur, cons
  * (1..4096, after twenty untimed ones while the clock settles), enqueued
  * back to back with one wait at the end; the steps advance the state:
  * out[0] face kernel (tiled step: the tile kernel, faces and cells),
- * out[1] cell kernel and surrogate-list kernel (tiled step: the list kernel
- * only), out[2] dt kernel, out[3] whole step. */
+ * out[1] cell kernel (tiled step: nothing but the gap between two events),
+ * out[2] dt kernel, out[3] whole step. */
 int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]);
 
 /* The tiled step's layout of a mesh at 256 cells a tile (a handle on a mesh

@@ -82,11 +82,6 @@ __global__ void k_mlp_gen(double gamma, uint64_t seed, int n, const float *norm,
   if (i < n) put_sample(gamma, seed, (uint64_t)i, i, norm, X, Y, OK);
 }
 
-// Four consecutive floats of the model, which a caller may hold at any float's
-// address (one 16-byte load either way).
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ f32x4u ld4(const float *p) { return *reinterpret_cast<const f32x4u *>(p); }
-
 // v plus v of the lane across bit 0, 1, 2 or 3 of the lane number, the sum of
 // 16 lanes in the order of a butterfly of lane exchanges: each level adds two
 // values that all lanes of their halves hold alike, so a mirrored lane serves

@@ -241,12 +241,6 @@ struct rhllc_solver {
   // The current state, updated in place.
   Dev now() const { return dev(cur, cur); }
 
-  // Cell kernel, plus the list kernel of the surrogate-start variant.
-  hipError_t enqueue_cells(const Dev &e) {
-    hipError_t r = launch_cell(e, variant, rad, prm.collect_stats != 0, stream);
-    if (r == hipSuccess && variant == kMixedMlp) r = launch_cell_mlp(e, rad, prm.collect_stats != 0, stream);
-    return r;
-  }
   // State and slot buffers both return after six steps.
   static constexpr int kGraphSteps = 2 * kSpeedBufs;
 
@@ -262,7 +256,6 @@ struct rhllc_solver {
       x.fold = open;
       if (tau) x.use_tau = 1, x.tau = *tau;
       e = launch_tile(x, mixed, variant, rad, prm.collect_stats != 0, n_tiles, tile_slots, stream);
-      if (e == hipSuccess && variant == kMixedMlp) e = launch_cell_mlp(x, rad, prm.collect_stats != 0, stream);
       if (e == hipSuccess) {
         last_in = cur;
         cur ^= 1;
@@ -276,7 +269,7 @@ struct rhllc_solver {
     if (tau) x.use_tau = 1, x.tau = *tau;
     e = launch_face(x, mixed, stream);
     x.use_tau = 0;  // the cell kernels read it from the scalars
-    if (e == hipSuccess) e = enqueue_cells(x);
+    if (e == hipSuccess) e = launch_cell(x, variant, rad, prm.collect_stats != 0, stream);
     if (e == hipSuccess) {
       last_in = cur;
       open = true;
@@ -492,7 +485,6 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
       h->Wvab[k] = h->Wvab[0], h->Wsgb[k] = h->Wsgb[0];
     }
   }
-  if (variant == kMixedMlp) HIP_TRY(h->alloc(&d.mlp_list, N));
   HIP_TRY(h->alloc(&d.sc, 1));
   HIP_TRY(h->alloc(&d.speed_slots, (size_t)kSpeedBufs * kSpeedSlots * kSlotStride));
   std::memset(h->host_sc, 0, sizeof(Scalars));
@@ -890,12 +882,7 @@ extern "C" int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]
       e = h->tiled ? launch_tile(x, h->mixed, h->variant, h->rad, stats, h->n_tiles, h->tile_slots, h->stream)
                    : launch_face(x, h->mixed, h->stream);
     if (e == hipSuccess && e4) e = hipEventRecord(e4[1], h->stream);
-    if (e == hipSuccess) {
-      if (!h->tiled)
-        e = h->enqueue_cells(x);
-      else if (h->variant == kMixedMlp)
-        e = launch_cell_mlp(x, h->rad, stats, h->stream);
-    }
+    if (e == hipSuccess && !h->tiled) e = launch_cell(x, h->variant, h->rad, stats, h->stream);
     if (e == hipSuccess && e4) e = hipEventRecord(e4[2], h->stream);
     if (e == hipSuccess) e = launch_dt(x, nullptr, h->stream);
     if (e == hipSuccess && e4) e = hipEventRecord(e4[3], h->stream);

@@ -37,8 +37,7 @@ struct Scalars {
   unsigned long long max_residual_bits;
   unsigned long long mlp_starts;
   unsigned long long fix_mark;  // fix_fail when the moments of rhllc_add_rad_flux arrived
-  unsigned int unusual;  // FP64 path: a state that is not `ordinary` was stored (stays set)
-  unsigned int mlp_count[kSpeedBufs];  // cells appended to Dev::mlp_list by the step of each slot buffer
+  unsigned long long unusual;  // FP64 path: a state that is not `ordinary` was stored (stays set)
 };
 
 // Everything a kernel needs, passed by value.  Cells and faces are in the
@@ -114,7 +113,6 @@ struct Dev {
   // surrogate c2p guess (RHLLC_GUESS_MLP): FP32 model and bf16 W2
   const float *mlpP;
   const short *mlpW2b;
-  int32_t *mlp_list;  // kMixedMlp: cells deferred to k_cell_mlp (n_cells entries)
   Scalars *sc;
   double *speed_slots;  // kSpeedBufs buffers of kSpeedSlots * kSlotStride
   // The slot buffer this step's maximum goes to, and whether the previous
@@ -150,7 +148,6 @@ hipError_t launch_unpack_fields(const int32_t *old_to_new, int first, int n, con
                                 float2 *k, bool kappa, float *T, Scalars *mark, hipStream_t s);
 hipError_t launch_face(const Dev &d, bool mixed, hipStream_t s);
 hipError_t launch_cell(const Dev &d, int variant, bool rad, bool stats, hipStream_t s);
-hipError_t launch_cell_mlp(const Dev &d, bool rad, bool stats, hipStream_t s);
 // The tiled step: faces into LDS, then the cells of the tile from LDS.
 // lds_slots = the largest face count of any tile.
 hipError_t launch_tile(const Dev &d, bool mixed, int variant, bool rad, bool stats, int n_tiles, int lds_slots,

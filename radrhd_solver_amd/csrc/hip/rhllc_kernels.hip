@@ -8,8 +8,7 @@
 //           U -= tau/V * sum, c2p (Newton, FP64) with the PhysPressureFix
 //           fallback, optional radiation source + second c2p; tau from the
 //           previous step's maxima or from k_dt,
-// then k_cell_mlp (surrogate start only) and, on large meshes and after the
-// last step of a call,
+// and, on large meshes and after the last step of a call,
 //   k_dt    one wave: max over the slots, tau = CFL*h_min/speed, t += tau.
 // The two-kernel step is k_face (fluxes to memory), k_cell, k_dt.
 // No float atomics: face fluxes are written once and read by a fixed-order
@@ -99,20 +98,18 @@ __device__ __forceinline__ double slots_max(const Dev &d, int buf) {
 static_assert(kSpeedSlots == 64, "one slot per lane");
 
 // The bookkeeping between two steps (rhllc_utils.cpp:15-23): tau = CFL*h_min /
-// speed of the step whose slot buffer is `buf`.  Built before the maximum is
+// speed of the last step.  Built before the maximum is
 // known, so the scalars' loads overlap its load; store() by one thread.
 struct StepClose {
   double t, tau0;
-  unsigned long long steps, starts;
-  __device__ __forceinline__ StepClose(const Dev &d, int buf)
-      : t(d.sc->t), tau0(d.sc->tau), steps(d.sc->steps), starts(d.sc->mlp_starts + d.sc->mlp_count[buf]) {}
+  unsigned long long steps;
+  __device__ __forceinline__ explicit StepClose(const Dev &d) : t(d.sc->t), tau0(d.sc->tau), steps(d.sc->steps) {}
   __device__ __forceinline__ void store(const Dev &d, double speed, double tau) const {
     Scalars *sc = d.sc;
     sc->t = t + tau0;
     sc->last_speed = speed;
     sc->tau = tau;
     sc->steps = steps + 1;
-    sc->mlp_starts = starts;
   }
 };
 
@@ -152,10 +149,7 @@ __device__ __forceinline__ double fold_speed(const Dev &d, double speed) {
     if ((threadIdx.x & 63) == 0) tau_lds = tau;
     if (blockIdx.x == 0) {
       *speed_slot(d, next, threadIdx.x & 63) = 0;
-      if ((threadIdx.x & 63) == 0) {
-        StepClose(d, prev).store(d, s, tau);
-        d.sc->mlp_count[next] = 0;
-      }
+      if ((threadIdx.x & 63) == 0) StepClose(d).store(d, s, tau);
     }
   }
   __syncthreads();
@@ -310,25 +304,6 @@ __device__ __forceinline__ void count_if(unsigned long long *ctr, bool pred) {
   if (m && (threadIdx.x & 63) == __ffsll((long long)m) - 1) atomicAdd(ctr, (unsigned long long)__popcll(m));
 }
 
-// Surrogate start: every lane of the wave takes part (MFMA), dead lanes with
-// a dummy state; returns the predicted pressure of this lane's cell.
-__device__ __forceinline__ double mlp_guess(const Dev &d, bool live, const State<double> &U) {
-  using namespace rhllc_mlp;
-  const float *norm = d.mlpP + kOffNorm;
-  float xl[3] = {0.f, 0.f, 0.f};
-  double p0 = 0.0;
-  if (live) features(norm, d.Gg, U.d, sqrt(dot3(U.v, U.v)), U.p, xl, p0);
-  const int l = threadIdx.x & 63;
-  float x[4][3];
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int f = 0; f < 3; ++f) x[t][f] = __shfl(xl[f], 16 * t + (l & 15), 64);
-  float out[4];
-  forward_wave(d.mlpP, d.mlpW2b, x, out);
-  return predicted_pressure(norm, out[l >> 4], p0);
-}
-
 // Surrogate start only where the previous pressure is stale: the cell's
 // tau = E - D changed by more than this fraction in the step.  Measured on
 // the same states (a 48^3-hex blast, steps 1-60): where tau moved by 5-20%,
@@ -337,6 +312,48 @@ __device__ __forceinline__ double mlp_guess(const Dev &d, bool live, const State
 // the two are within a quarter iteration either way, and below 0.5% the
 // previous pressure converges in one iteration where the surrogate needs two.
 constexpr double kMlpGate = 0.05;
+
+// Whether a cell starts from the surrogate, and its predicted pressure then.
+// Called by all lanes of a wave (MFMA); a wave without such a cell does
+// nothing, the others evaluate theirs in groups of 16.  The cells sit at the
+// front of a flow, in few waves (0.1-0.2% of the cells of the 24M-cell blast):
+// in place they lengthen those waves' chain by about 4 us, where a list of them
+// finished by a kernel of its own cost every step 8 to 10.  The first 100 steps
+// of a blast, list -> in place: 16.3 -> 11.9 us a step at 34,992 cells, 23.9 ->
+// 18.6 at 162,000, 39.7 -> 36.8 at 663,552, 346 -> 342 at 6M (with radiation).
+__device__ __forceinline__ bool mlp_start(const Dev &d, bool live, const State<double> &U, double dtau,
+                                          double &guess) {
+  using namespace rhllc_mlp;
+  const bool stale = live && !(fabs(dtau) <= kMlpGate * fabs(U.p - U.d));
+  const unsigned long long m = __ballot(stale);
+  if (m == 0) return false;
+  const float *norm = d.mlpP + kOffNorm;
+  float xl[3] = {0.f, 0.f, 0.f};
+  double p0 = 0.0;
+  if (stale) features(norm, d.Gg, U.d, sqrt(dot3(U.v, U.v)), U.p, xl, p0);
+  // The k-th stale lane's features go to sample k: lane k learns which lane that
+  // is, and each stale lane takes its output back from its sample's group.
+  const int l = threadIdx.x & 63, rank = __popcll(m & ((1ull << l) - 1ull));
+  const int src = __builtin_amdgcn_ds_permute(stale ? 4 * rank : 4 * (63 - l + rank), l);
+  const int groups = (__popcll(m) + 15) / 16;
+  float o = 0.f;
+#pragma unroll 1
+  for (int t = 0; t < groups; ++t) {
+    const int from = __shfl(src, 16 * t + (l & 15), 64);
+    const float x[3] = {__shfl(xl[0], from, 64), __shfl(xl[1], from, 64), __shfl(xl[2], from, 64)};
+    // The model's addresses anew in each pass: its loads, hoisted, would take
+    // more registers than the whole kernel.
+    const float *P = d.mlpP;
+    const short *W2b = d.mlpW2b;
+    int lane = l;
+    asm volatile("" : "+s"(P), "+s"(W2b), "+v"(lane));
+    const float ot = __shfl(forward_16(P, W2b, x, lane), rank & 15, 64);
+    if ((rank >> 4) == t) o = ot;
+  }
+  if (stale) guess = predicted_pressure(norm, o, p0);
+  count_if(&d.sc->mlp_starts, stale);
+  return stale;
+}
 
 // Where a cell's four face fluxes come from.  GlobalFlux: the arrays the
 // face kernel of the two-kernel step wrote (face index | bit 31 when the cell
@@ -554,32 +571,9 @@ __device__ __forceinline__ void finish_cell(const Dev &d, int c, bool live, Stat
   }
 }
 
-// The surrogate-start variant defers cells whose tau changed by more than
-// kMlpGate: they are appended to d.mlp_list (one atomic per wave), their
-// updated U is stored, and k_cell_mlp finishes them on full waves.  Returns
-// whether this lane's cell stays live here.  Called by all lanes of a wave.
-__device__ __forceinline__ bool defer_stale(const Dev &d, int c, bool live, const State<double> &U, double dtau) {
-  const bool stale = live && !(fabs(dtau) <= kMlpGate * fabs(U.p - U.d));
-  const unsigned long long m = __ballot(stale);
-  if (m) {
-    const int lane = threadIdx.x & 63;
-    const int first = __ffsll((long long)m) - 1;
-    unsigned int base = 0;
-    if (lane == first) base = atomicAdd(&d.sc->mlp_count[d.slot], (unsigned int)__popcll(m));
-    base = __shfl(base, first, 64);
-    if (stale) {
-      st(d.mlp_list, base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)), c);
-      st(d.U4o, c, make_double4(U.d, U.v[0], U.v[1], U.v[2]));
-      st(d.UEo, c, U.p);
-      return false;
-    }
-  }
-  return live;
-}
-
 // One thread per cell.  Start of the Newton iteration: the reference start
-// (kFp64Ref), the FP64 previous pressure (kFp64Prev) or the FP32 one (mixed).
-// kMixedMlp: stale cells go to k_cell_mlp (defer_stale).
+// (kFp64Ref), the FP64 previous pressure (kFp64Prev) or the FP32 one (mixed);
+// kMixedMlp: the surrogate's in stale cells (mlp_start).
 template <int VARIANT, bool RAD, bool STATS, int EOS>
 __global__ __launch_bounds__(kBlock) void k_cell(Dev d) {
   constexpr bool MIXED = VARIANT >= kMixedPrev;
@@ -593,11 +587,12 @@ __global__ __launch_bounds__(kBlock) void k_cell(Dev d) {
     const GlobalFlux<MIXED> src{d, ld(d.cell_faces, c)};
     update_U<MIXED>(d, c, tau, src, U, dtau, p32);
   }
-  if (VARIANT == kMixedMlp) live = defer_stale(d, c, live, U, dtau);
   double guess = -1.0;
   if (VARIANT == kFp64Prev && live) guess = ld(d.Wp, c);
   if (MIXED && live) guess = (double)p32;
-  finish_cell<VARIANT, RAD, STATS, EOS>(d, c, live, U, guess, false, tau);
+  bool from_mlp = false;
+  if constexpr (VARIANT == kMixedMlp) from_mlp = mlp_start(d, live, U, dtau, guess);
+  finish_cell<VARIANT, RAD, STATS, EOS>(d, c, live, U, guess, from_mlp, tau);
 }
 
 // The tiled step, one workgroup per tile of d.tile_cells cells (Hilbert order).
@@ -657,46 +652,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     const TileFlux<MIXED> src{A, B, C, {sl.x & 0xFFFFu, sl.x >> 16, sl.y & 0xFFFFu, sl.y >> 16}};
     update_U<MIXED>(d, c, tau, src, U, dtau, p32);
   }
-  if (VARIANT == kMixedMlp) live = defer_stale(d, c, live, U, dtau);
   double guess = -1.0;
   if (VARIANT == kFp64Prev && live) guess = ld(d.Wp, c);
   if (MIXED && live) guess = (double)p32;
-  finish_cell<VARIANT, RAD, STATS, EOS>(d, c, live, U, guess, false, tau);
-}
-
-// Cells deferred by k_cell<kMixedMlp>: list entries [0, mlp_count), 64 per
-// wave so the surrogate's MFMA pass runs on full waves.  A fixed grid loops
-// over the list (the count is only known on the device); every block runs
-// the same number of iterations, and all of them end when the list does.
-// The surrogate is trained for the ideal gas only.
-template <bool RAD, bool STATS>
-__global__ __launch_bounds__(kBlock) void k_cell_mlp(Dev d) {
-  const unsigned int n = d.sc->mlp_count[d.slot];
-  const double tau = d.sc->tau;
-  for (unsigned int b0 = blockIdx.x * kBlock; b0 < n; b0 += gridDim.x * kBlock) {
-    const unsigned int i = b0 + threadIdx.x;
-    const bool live = i < n;
-    const int c = live ? ld(d.mlp_list, i) : 0;
-    State<double> U;
-    U.d = 1.0, U.v[0] = 0.0, U.v[1] = 0.0, U.v[2] = 0.0, U.p = 2.0;  // dummy lanes
-    if (live) load_U(d, c, U);
-    const double g = mlp_guess(d, live, U);
-    finish_cell<kMixedMlp, RAD, STATS, kIdeal>(d, c, live, U, g, true, tau);
-  }
+  bool from_mlp = false;
+  if constexpr (VARIANT == kMixedMlp) from_mlp = mlp_start(d, live, U, dtau, guess);
+  finish_cell<VARIANT, RAD, STATS, EOS>(d, c, live, U, guess, from_mlp, tau);
 }
 
 // tau of the next step from the max signal speed (rhllc_utils.cpp:15-23):
 // tau = CFL*h_min / speed.  Also clears every slot buffer, so the next step
 // starts from buffer 0.  One wave.
 __global__ __launch_bounds__(64) void k_dt(Dev d, Scalars *host) {
-  const StepClose c(d, d.slot);
+  const StepClose c(d);
   const unsigned long long fix_fail = d.sc->fix_fail;
   const double s = slots_max(d, d.slot);
   if (threadIdx.x == 0) {
     const double tau = d.cfl_hmin / s;
     if (host) host->tau = tau, host->last_speed = s, host->fix_fail = fix_fail;
     c.store(d, s, tau);
-    for (int k = 0; k < kSpeedBufs; ++k) d.sc->mlp_count[k] = 0;
   }
 #pragma unroll
   for (int k = 0; k < kSpeedBufs; ++k) *speed_slot(d, k, threadIdx.x) = 0;
@@ -917,7 +891,6 @@ __global__ void k_clear(Dev d) {
     sc->steps = 0;
     for (int k = 0; k < 6; ++k) sc->c2p_fail[k] = 0;
     sc->fix_calls = sc->fix_fail = sc->fallback = sc->newton_iters = sc->mlp_starts = 0;
-    for (int k = 0; k < kSpeedBufs; ++k) sc->mlp_count[k] = 0;
     for (int k = 0; k < kHistBins; ++k) sc->hist[k] = 0;
     sc->max_residual_bits = 0;
   }
@@ -1040,26 +1013,6 @@ hipError_t launch_cell(const Dev &d, int variant, bool rad, bool stats, hipStrea
       break;
     default:
       return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
-// Grid of the list kernel: enough blocks to fill the chip; each loops over
-// the list, whose length is read on the device.
-hipError_t launch_cell_mlp(const Dev &d, bool rad, bool stats, hipStream_t s) {
-  if (d.n_cells == 0) return hipSuccess;
-  const unsigned int nb = blocks_for(d.n_cells) < 2048u ? blocks_for(d.n_cells) : 2048u;
-  const dim3 g(nb), b(kBlock);
-  if (rad) {
-    if (stats)
-      hipLaunchKernelGGL((k_cell_mlp<true, true>), g, b, 0, s, d);
-    else
-      hipLaunchKernelGGL((k_cell_mlp<true, false>), g, b, 0, s, d);
-  } else {
-    if (stats)
-      hipLaunchKernelGGL((k_cell_mlp<false, true>), g, b, 0, s, d);
-    else
-      hipLaunchKernelGGL((k_cell_mlp<false, false>), g, b, 0, s, d);
   }
   return hipGetLastError();
 }

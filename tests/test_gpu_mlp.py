@@ -180,3 +180,37 @@ def test_surrogate_start_gains_on_the_cells_it_starts():
     prev, mlp = total["prev"] / total["cells"], total["mlp"] / total["cells"]
     print("over all probed steps: previous pressure", prev, "surrogate", mlp)
     assert mlp <= prev - 0.5
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 2), (7, 5, 3), (30, 30, 31)])  # part of a wave; 64- and 256-cell tiles
+@pytest.mark.parametrize("hot", [0.02, 0.3, 1.0])
+@pytest.mark.parametrize("schedule", [capi.SCHED_TILED, capi.SCHED_TWO_KERNEL])
+def test_surrogate_start_with_few_and_many_stale_cells(shape, hot, schedule):
+    """One step from random pressures in a share of the cells, so that a wave has from none to all
+    of its cells stale: U does not depend on the c2p start, W agrees with the previous-pressure
+    start's to the Newton tolerance, and the cells counted are those whose E - D moved by 5%."""
+    from radrhd_solver_amd import surrogate
+
+    m = M.kuhn_box(*shape, seed=SEED)
+    rng = np.random.default_rng(SEED)
+    W0 = M.init_state(m, M.INIT_UNIFORM, params=[1.0, 0.0, 0.0, 0.0, 1.0])
+    sel = rng.random(m.n_cells) < hot
+    W0[sel, 4] = 10 ** rng.uniform(0, 3, sel.sum())
+    out = {}
+    for guess in (capi.GUESS_PREVIOUS, capi.GUESS_MLP):
+        s = capi.Solver(m, cfl=0.4, precision=capi.PREC_MIXED, guess=guess, schedule=schedule)
+        if guess == capi.GUESS_MLP:
+            s.set_mlp(surrogate.load(5 / 3))
+        s.upload_W(W0)
+        U0 = s.download()[1]
+        s.run(1)
+        s.sync()
+        out[guess] = (*s.download(), s.stats())
+        s.close()
+    (W, U, st), (Wp, Up, _) = out[capi.GUESS_MLP], out[capi.GUESS_PREVIOUS]
+    assert np.array_equal(U, Up) and sum(st["c2p_fail"]) == 0 and st["fallback_cells"] == 0
+    assert np.abs(W - Wp).max() <= 1e-9 * np.abs(Wp).max()
+    tau0, tau1 = U0[:, 4] - U0[:, 0], U[:, 4] - U[:, 0]
+    moved = np.abs(tau1 - tau0) / np.abs(tau1)
+    assert (moved > 0.05 * (1 + 1e-9)).sum() <= st["mlp_starts"] <= (moved > 0.05 * (1 - 1e-9)).sum()
+    assert st["mlp_starts"] > 0
