@@ -320,7 +320,7 @@ int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, const float *X
  * floats), X (n x 3), y, ok (n each), grad (RHLLC_MLP_PARAMS floats) and loss
  * (1 float) are device pointers; the work is enqueued on `stream` (a
  * hipStream_t; NULL = the null stream) and the caller synchronizes.  The
- * packed weights, per-wave partials and losses live in a scratch array the
+ * partials and losses of 64 samples each live in a scratch array the
  * library holds on each GPU (18.5 MB, for n <= RHLLC_MLP_NOALLOC_MAX_N; larger
  * n is RHLLC_ERR_ARG); grad and loss are the same bits as rhllc_mlp_grad's.
  * Calls that overlap on one GPU share that scratch and race.  No counterpart

@@ -81,9 +81,8 @@ extern "C" int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, con
     return fail(RHLLC_ERR_ARG, "bad argument (n must be a positive multiple of 256)");
   HIP_TRY(hipSetDevice(device));
   const int nw = n / 64;
-  Buf P, W2, Xd, Yd, Od, Gd, Ld, Sd;
+  Buf P, Xd, Yd, Od, Gd, Ld, Sd;
   HIP_TRY(alloc(P, sizeof(float) * kModel));
-  HIP_TRY(alloc(W2, sizeof(short) * kH * kH * 2));
   HIP_TRY(alloc(Xd, sizeof(float) * 3 * n));
   HIP_TRY(alloc(Yd, sizeof(float) * n));
   HIP_TRY(alloc(Od, sizeof(float) * n));
@@ -94,8 +93,7 @@ extern "C" int rhllc_mlp_grad(int32_t device, const float *model, int32_t n, con
   HIP_TRY(hipMemcpy(Xd.p, X, sizeof(float) * 3 * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(Yd.p, y, sizeof(float) * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(Od.p, ok, sizeof(float) * n, hipMemcpyHostToDevice));
-  HIP_TRY(launch_pack(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, nullptr));
-  HIP_TRY(launch_grad(P.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH, Xd.as<float>(), Yd.as<float>(),
+  HIP_TRY(launch_grad(P.as<float>(), nullptr, nullptr, Xd.as<float>(), Yd.as<float>(),
                       Od.as<float>(), 1.0f / (float)n, n, Gd.as<float>(), Ld.as<float>(), nullptr, nullptr));
   HIP_TRY(launch_sum(Gd.as<float>(), Ld.as<float>(), nw, Sd.as<float>(), Sd.as<float>() + kParams, nullptr));
   HIP_TRY(hipDeviceSynchronize());
@@ -211,16 +209,14 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
 }
 
 // ---------------------------------------------------------------- no-alloc
-// Scratch of rhllc_mlp_grad_noalloc: the packed BF16 weights (2 x 64 x 64
-// shorts = 4096 floats), the per-wave gradient partials (kGradStride floats a
+// Scratch of rhllc_mlp_grad_noalloc: the gradient partials (kGradStride floats a
 // wave) and the per-wave losses, for batches of up to kNoAllocMaxN samples.
 // Each GPU holds its own copy until the process ends.  Host code uses the
 // device address hipGetSymbolAddress returns, never the array's name.
 namespace {
 constexpr int kNoAllocMaxN = 65536;
 constexpr int kNoAllocMaxWaves = kNoAllocMaxN / 64;
-constexpr size_t kScratchW2 = 0;                                              // floats
-constexpr size_t kScratchGrad = kScratchW2 + (size_t)kH * kH;                 // 2 x 4096 shorts
+constexpr size_t kScratchGrad = 0;  // floats
 constexpr size_t kScratchLoss = kScratchGrad + (size_t)kGradStride * kNoAllocMaxWaves;
 constexpr size_t kScratchFloats = kScratchLoss + kNoAllocMaxWaves;
 }  // namespace
@@ -259,12 +255,10 @@ extern "C" int rhllc_mlp_grad_noalloc(int32_t device, const float *model, int32_
   if (int e = scratch_on(device, &sc)) return e;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const int nw = n / 64;
-  short *W2b = reinterpret_cast<short *>(sc + kScratchW2);
   float *part = sc + kScratchGrad, *lpart = sc + kScratchLoss;
   // Every scratch element these kernels read is written first in the same call
-  // (pack: all of W2; grad: nw partial rows and nw losses), so nothing is cleared.
-  HIP_TRY(launch_pack(model, W2b, W2b + kH * kH, st));
-  HIP_TRY(launch_grad(model, W2b, W2b + kH * kH, X, y, ok, 1.0f / (float)n, n, part, lpart, nullptr, st));
+  // (nw partial rows and nw losses), so nothing is cleared.
+  HIP_TRY(launch_grad(model, nullptr, nullptr, X, y, ok, 1.0f / (float)n, n, part, lpart, nullptr, st));
   HIP_TRY(launch_sum(part, lpart, nw, grad, loss, st));
   return RHLLC_OK;
 }

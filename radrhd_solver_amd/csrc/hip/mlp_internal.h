@@ -21,7 +21,8 @@ struct Batch {
   const float *norm;
   float *X, *Y, *OK;
 };
-// nw = n / 64 partials of kGradStride floats in grad and one loss each.  step
+// nw = n / 64 partials of kGradStride floats in grad and one loss each.  W2b,
+// W2Tb: launch_pack's copies, or null (formed from P by every workgroup).  step
 // (null outside training): {the next step's number, this step's}, step[1] =
 // step[0] here.
 hipError_t launch_grad(const float *P, const short *W2b, const short *W2Tb, const float *X, const float *Y,

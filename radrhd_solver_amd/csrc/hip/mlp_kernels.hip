@@ -1,9 +1,9 @@
 // Training and evaluation kernels of the c2p surrogate MLP (see mlp.h).
 //
 // Training step (captured in a hipGraph and replayed):
-//   k_mlp_grad   one wave per 64 samples: forward (BF16 MFMA with K = 32,
+//   k_mlp_grad   one workgroup per 64 samples: forward (BF16 MFMA with K = 32,
 //                FP32 accumulate),
-//                backward, per-wave gradient partials written to global memory;
+//                backward, gradient partials written to global memory;
 //   k_mlp_adam   fixed-order sum of the partials (deterministic), Adam on the
 //                FP32 master weights, BF16 copies of W2 and W2^T, the step's
 //                loss and the device step counter; and on the CUs that the sum
@@ -102,87 +102,117 @@ __device__ __forceinline__ float sum16(float v) {
 // padding, so the 16 rows a load touches start in different banks.
 constexpr int kLdT = kH + 4;
 
-// One wave = 64 consecutive samples.  grad[wave][kGradStride] receives the
-// wave's gradient of sum_s ok_s (out_s - y_s)^2 * inv_n; loss[wave] the sum
-// of squared errors.  A full batch is one wave per SIMD, so the kernel takes as
-// long as one wave's chain: the activations' derivatives are formed with them
-// from one sigmoid and kept instead of the pre-activations (128 exponentials a
-// lane, not 320), the sums over 16 lanes use DPP, the vectors come in 16-byte
-// loads and the LDS rows are padded: 38.2 -> 25.2 us at 65,536 samples, no
-// scratch (248 bytes a lane spilled before).
-__global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, const short *__restrict__ W2b,
-                                                  const short *__restrict__ W2Tb, const float *__restrict__ X,
-                                                  const float *__restrict__ Y, const float *__restrict__ OK,
-                                                  float inv_n, int n, float *__restrict__ grad,
-                                                  float *__restrict__ loss, uint32_t *step) {
+// One workgroup = 64 consecutive samples ("wave" of the partials: a single wave
+// once took them).  grad[wave][kGradStride] receives their gradient of
+// sum_s ok_s (out_s - y_s)^2 * inv_n; loss[wave] the sum of squared errors.
+//
+// The four waves share the hidden units: wave w has the units of block w
+// (16 w .. 16 w + 15) of both layers, and lane (g, c) of it the units
+// 16 w + 4 g + e of the samples 16 t + c.  The operands of the products that
+// contract over all units go through LDS as they are (frag), those of dW2,
+// which contracts over the samples, transposed (rows of a unit); the output's
+// sum over the units is taken in unit order from the waves' terms, so every
+// value is rounded as one wave taking all the units would.  A batch of 65,536
+// is then four waves a SIMD where it was one, waiting for its own chain; each
+// activation's derivative is formed with it from one sigmoid, the sums over 16
+// lanes use DPP and the vectors come in 16-byte loads.  Measured at 65,536
+// samples: 38.2 us as one wave with spilled registers, 25.2 as one wave
+// without, 18.4 so.
+//
+// PACKED: W2 and its transpose come as the BF16 copies that training keeps,
+// else they are rounded here from P (a call of its own would first need a
+// launch that makes the copies: 3.3 us and a gap).
+template <bool PACKED>
+__global__ __launch_bounds__(256, 3) void k_mlp_grad(const float *__restrict__ P, const short *__restrict__ W2b,
+                                                     const short *__restrict__ W2Tb, const float *__restrict__ X,
+                                                     const float *__restrict__ Y, const float *__restrict__ OK,
+                                                     float inv_n, float *__restrict__ grad, float *__restrict__ loss,
+                                                     uint32_t *step) {
   if (step && blockIdx.x == 0 && threadIdx.x == 0) step[1] = step[0];
-  __shared__ __align__(16) short lds[4][2][kH * kLdT];  // per wave: dZ2^T [h2][s] and H1^T [h1][s], bf16
+  __shared__ __align__(16) short h1T[kH * kLdT], dzT[kH * kLdT];  // H1^T [h1][s], dZ2^T [h2][s], bf16
+  __shared__ bf16x4 frag[4][4][64];                               // [block][t][lane]: H1, then dZ2
+  __shared__ f32x4 part0[64], term[3][4][64];  // block 0's sum and the others' terms [r][lane] of the 4 samples
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = l >> 4, c = l & 15;
-  const int wave = blockIdx.x * 4 + w;
-  const int base = wave * 64;
-  short *dzT = lds[w][0];
-  short *h1T = lds[w][1];
-  // own sample (lane l) and the 4 samples s_t = 16 t + c this lane works on
-  float xl[3] = {0.f, 0.f, 0.f}, yl = 0.f, okl = 0.f;
-  if (base + l < n) {
-    xl[0] = X[3 * (base + l)], xl[1] = X[3 * (base + l) + 1], xl[2] = X[3 * (base + l) + 2];
-    yl = Y[base + l], okl = OK[base + l];
-  }
+  const int base = blockIdx.x * 64;
+  const int h0 = 16 * w + 4 * g;  // this lane's units of both layers
+  // the 4 samples s_t = 16 t + c this lane works on
   float x[4][3], y[4], ok[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
+    const int i = base + 16 * t + c;
 #pragma unroll
-    for (int f = 0; f < 3; ++f) x[t][f] = __shfl(xl[f], 16 * t + c, 64);
-    y[t] = __shfl(yl, 16 * t + c, 64);
-    ok[t] = __shfl(okl, 16 * t + c, 64);
+    for (int f = 0; f < 3; ++f) x[t][f] = X[3 * i + f];
+    y[t] = Y[i], ok[t] = OK[i];
   }
-  // ---- forward
-  float d1[4][4][4];  // [q][t][e] dsilu of layer 1
-  bf16x4 h1[4][4];    // [q][t]
+  float w1[12];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) *reinterpret_cast<f32x4u *>(w1 + 4 * k) = ld4(P + kOffW1 + 3 * h0 + 4 * k);
+  const f32x4u b1 = ld4(P + kOffB1 + h0), b2 = ld4(P + kOffB2 + h0), w3 = ld4(P + kOffW3 + h0);
+  bf16x4 a2w[4], a1w[4];  // rows of W2 and of W2^T
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int h0 = 16 * q + 4 * g;
-    float wr[12];
+    if constexpr (PACKED) {
+      a2w[q] = *reinterpret_cast<const bf16x4 *>(W2b + (16 * w + c) * kH + 16 * q + 4 * g);
+      a1w[q] = *reinterpret_cast<const bf16x4 *>(W2Tb + (16 * w + c) * kH + 16 * q + 4 * g);
+    } else {
+      const f32x4u row = ld4(P + kOffW2 + (16 * w + c) * kH + 16 * q + 4 * g);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) *reinterpret_cast<f32x4u *>(wr + 4 * k) = ld4(P + kOffW1 + 3 * h0 + 4 * k);
-    const f32x4u bb = ld4(P + kOffB1 + h0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float z = ((wr[3 * e] * x[t][0] + wr[3 * e + 1] * x[t][1]) + wr[3 * e + 2] * x[t][2]) + bb[e];
-        const float s = sigmoid(z);
-        d1[q][t][e] = s * (1.0f + z * (1.0f - s));
-        h1[q][t][e] = f2bf(z * s);
-        h1T[(h0 + e) * kLdT + 16 * t + c] = h1[q][t][e];
-      }
-  }
-  float a2[4][4][4], d2[4][4][4];  // [u][t][r] silu and dsilu of layer 2, unit 16 u + 4 g + r, sample s_t
-  f32x4u w3[4];
-  float out[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    bf16x4 a[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const bf16x4 *>(W2b + (16 * u + c) * kH + 16 * q + 4 * g);
-    const f32x4u b2 = ld4(P + kOffB2 + 16 * u + 4 * g);
-    w3[u] = ld4(P + kOffW3 + 16 * u + 4 * g);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int q = 0; q < 4; q += 2) acc = mfma32(a[q], a[q + 1], h1[q][t], h1[q + 1][t], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float z = acc[r] + b2[r];
-        const float s = sigmoid(z);
-        a2[u][t][r] = z * s;
-        d2[u][t][r] = s * (1.0f + z * (1.0f - s));
-        out[t] += w3[u][r] * a2[u][t][r];
+      for (int e = 0; e < 4; ++e) {
+        a2w[q][e] = f2bf(row[e]);
+        a1w[q][e] = f2bf(P[kOffW2 + (16 * q + 4 * g + e) * kH + 16 * w + c]);
       }
     }
   }
+  // ---- layer 1
+  float d1[4][4];  // [t][e] dsilu
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    bf16x4 h;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float z = ((w1[3 * e] * x[t][0] + w1[3 * e + 1] * x[t][1]) + w1[3 * e + 2] * x[t][2]) + b1[e];
+      const float s = sigmoid(z);
+      d1[t][e] = s * (1.0f + z * (1.0f - s));
+      h[e] = f2bf(z * s);
+      h1T[(h0 + e) * kLdT + 16 * t + c] = h[e];
+    }
+    frag[w][t][l] = h;
+  }
+  __syncthreads();
+  // ---- layer 2
+  float a2[4][4], d2[4][4];  // [t][r] silu and dsilu
+  f32x4 tr[4];               // [r] the terms of the 4 samples' outputs
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4; q += 2) acc = mfma32(a2w[q], a2w[q + 1], frag[q][t][l], frag[q + 1][t][l], acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float z = acc[r] + b2[r];
+      const float s = sigmoid(z);
+      a2[t][r] = z * s;
+      d2[t][r] = s * (1.0f + z * (1.0f - s));
+      tr[r][t] = w3[r] * a2[t][r];
+    }
+  }
+  if (w == 0) {
+    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p += tr[r];
+    part0[l] = p;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) term[w - 1][r][l] = tr[r];
+  }
+  __syncthreads();
+  // ---- output, the same in all four waves
+  f32x4 out = part0[l];
+#pragma unroll
+  for (int u = 0; u < 3; ++u)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out += term[u][r][l];
   float dout[4];
   float sq = 0.f;
 #pragma unroll
@@ -194,77 +224,73 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
     dout[t] = 2.0f * d * inv_n;
     sq += d * d;
   }
-  float *G = grad + (size_t)wave * kGradStride;
-  // ---- layer 3 and b2, W3 gradients (summed over the 16 sample lanes); dZ2
-  bf16x4 dz2b[4][4];  // [u][t] as the B operand of dH1^T = W2^T dZ2^T
+  float *G = grad + (size_t)blockIdx.x * kGradStride;
+  // ---- dZ2; b2 and W3 gradients, summed over the 16 sample lanes
+  float aw[4] = {}, ab[4] = {};
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
+  for (int t = 0; t < 4; ++t) {
+    bf16x4 dzb;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float aw = 0.f, ab = 0.f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        aw += dout[t] * a2[u][t][r];
-        const float dz = dout[t] * w3[u][r] * d2[u][t][r];
-        ab += dz;
-        dz2b[u][t][r] = f2bf(dz);
-        dzT[(16 * u + 4 * g + r) * kLdT + 16 * t + c] = dz2b[u][t][r];
-      }
-      aw = sum16(aw), ab = sum16(ab);
-      if (c == 0) G[kOffW3 + 16 * u + 4 * g + r] = aw, G[kOffB2 + 16 * u + 4 * g + r] = ab;
+      aw[r] += dout[t] * a2[t][r];
+      const float dz = dout[t] * w3[r] * d2[t][r];
+      ab[r] += dz;
+      dzb[r] = f2bf(dz);
+      dzT[(h0 + r) * kLdT + 16 * t + c] = dzb[r];
     }
-  // ---- dH1^T = W2^T dZ2^T  (tiles q over h1, t over samples), then dZ1
+    frag[w][t][l] = dzb;  // every wave has read H1's before the last barrier
+  }
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    bf16x4 a[4];
+  for (int r = 0; r < 4; ++r) {
+    const float sw = sum16(aw[r]), sb = sum16(ab[r]);
+    if (c == 0) G[kOffW3 + h0 + r] = sw, G[kOffB2 + h0 + r] = sb;
+  }
+  __syncthreads();
+  // ---- dH1^T = W2^T dZ2^T, dZ1; W1 and b1 gradients
+  float gW1[4][3] = {}, gB1[4] = {};
 #pragma unroll
-    for (int u = 0; u < 4; ++u) a[u] = *reinterpret_cast<const bf16x4 *>(W2Tb + (16 * q + c) * kH + 16 * u + 4 * g);
-    float gW1[4][3] = {}, gB1[4] = {};
+  for (int t = 0; t < 4; ++t) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int u = 0; u < 4; u += 2) acc = mfma32(a[u], a[u + 1], dz2b[u][t], dz2b[u + 1][t], acc);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float dz = acc[e] * d1[q][t][e];
-        gB1[e] += dz;
-        gW1[e][0] += dz * x[t][0];
-        gW1[e][1] += dz * x[t][1];
-        gW1[e][2] += dz * x[t][2];
-      }
-    }
+    for (int u = 0; u < 4; u += 2) acc = mfma32(a1w[u], a1w[u + 1], frag[u][t][l], frag[u + 1][t][l], acc);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float v0 = sum16(gW1[e][0]), v1 = sum16(gW1[e][1]), v2 = sum16(gW1[e][2]), vb = sum16(gB1[e]);
-      const int h = 16 * q + 4 * g + e;
-      if (c == 0) G[kOffW1 + 3 * h] = v0, G[kOffW1 + 3 * h + 1] = v1, G[kOffW1 + 3 * h + 2] = v2, G[kOffB1 + h] = vb;
+      const float dz = acc[e] * d1[t][e];
+      gB1[e] += dz;
+      gW1[e][0] += dz * x[t][0];
+      gW1[e][1] += dz * x[t][1];
+      gW1[e][2] += dz * x[t][2];
     }
   }
-  // ---- dW2 = dZ2^T H1 from the transposed operands in LDS
-  __syncthreads();
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
+  for (int e = 0; e < 4; ++e) {
+    const float v0 = sum16(gW1[e][0]), v1 = sum16(gW1[e][1]), v2 = sum16(gW1[e][2]), vb = sum16(gB1[e]);
+    const int h = h0 + e;
+    if (c == 0) G[kOffW1 + 3 * h] = v0, G[kOffW1 + 3 * h + 1] = v1, G[kOffW1 + 3 * h + 2] = v2, G[kOffB1 + h] = vb;
+  }
+  // ---- dW2 = dZ2^T H1 from the transposed operands
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int q = 0; q < 4; ++q) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int t = 0; t < 4; t += 2) {
-        const short *ar = dzT + (16 * u + c) * kLdT + 4 * g, *br = h1T + (16 * q + c) * kLdT + 4 * g;
-        acc = mfma32(*reinterpret_cast<const bf16x4 *>(ar + 16 * t), *reinterpret_cast<const bf16x4 *>(ar + 16 * t + 16),
-                     *reinterpret_cast<const bf16x4 *>(br + 16 * t), *reinterpret_cast<const bf16x4 *>(br + 16 * t + 16),
-                     acc);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) G[kOffW2 + (16 * u + 4 * g + r) * kH + 16 * q + c] = acc[r];
+    for (int t = 0; t < 4; t += 2) {
+      const short *ar = dzT + (16 * w + c) * kLdT + 4 * g, *br = h1T + (16 * q + c) * kLdT + 4 * g;
+      acc = mfma32(*reinterpret_cast<const bf16x4 *>(ar + 16 * t), *reinterpret_cast<const bf16x4 *>(ar + 16 * t + 16),
+                   *reinterpret_cast<const bf16x4 *>(br + 16 * t), *reinterpret_cast<const bf16x4 *>(br + 16 * t + 16),
+                   acc);
     }
-  // b3: sum of dout over the wave's samples (group g = 0 holds each sample once)
-  float db = (g == 0) ? (dout[0] + dout[1] + dout[2] + dout[3]) : 0.f;
-  float ls = (g == 0) ? sq : 0.f;
-  db = sum16(db), ls = sum16(ls);
 #pragma unroll
-  for (int o = 16; o < 64; o <<= 1) db += __shfl_xor(db, o, 64), ls += __shfl_xor(ls, o, 64);
-  if (l == 0) G[kOffB3] = db, loss[wave] = ls;
+    for (int r = 0; r < 4; ++r) G[kOffW2 + (h0 + r) * kH + 16 * q + c] = acc[r];
+  }
+  // b3: sum of dout over the samples (group g = 0 holds each sample once)
+  if (w == 0) {
+    float db = (g == 0) ? (dout[0] + dout[1] + dout[2] + dout[3]) : 0.f;
+    float ls = (g == 0) ? sq : 0.f;
+    db = sum16(db), ls = sum16(ls);
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) db += __shfl_xor(db, o, 64), ls += __shfl_xor(ls, o, 64);
+    if (l == 0) G[kOffB3] = db, loss[blockIdx.x] = ls;
+  }
 }
 
 // Fixed-order column sums of the wave partials: column p of the nw x kGradStride
@@ -272,22 +298,40 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ P, c
 // column walking the rows waits for memory once per few rows (289 us for the
 // 1,024 rows of a 65,536-sample batch).  Here a workgroup of 1,024 threads owns
 // kSumCols columns: all of it loads kSumRows rows into LDS, 16 loads in flight a
-// thread and the next chunk's loads issued before the current one is added, and
-// one thread per column adds from LDS in order.  32 columns are one 128-byte
-// line of a row and make 141 workgroups of the 4,481 columns; the training step
-// gives the CUs they leave the next step's samples.
+// thread, and one thread per column adds them in order, four rows a read, while
+// the next chunk is on its way into the other buffer.  32 columns are one
+// 128-byte line of a row and make 141 workgroups of the 4,481 columns; the
+// training step gives the CUs they leave the next step's samples.  10.0 us for
+// 1,024 rows.
 constexpr int kSumCols = 32;
 constexpr int kSumRows = 512;
 constexpr int kSumThreads = 1024;
 constexpr int kSumPer = kSumRows * kSumCols / kSumThreads;          // rows a thread loads of a chunk
 constexpr int kSumBlocks = (kParams + kSumCols - 1) / kSumCols;     // workgroups of the columns
+constexpr int kSumLd = kSumRows + 4;  // rows of a column in LDS, padded: 16-byte reads of 16 columns meet all banks
 static_assert(kGradStride == kSumBlocks * kSumCols, "a partial's row is the workgroups' columns");
 static_assert(kSumThreads % kSumCols == 0 && kSumPer * (kSumThreads / kSumCols) == kSumRows, "chunk split");
+struct SumLds {
+  float v[2][kSumCols][kSumLd];
+};
+
+// s plus v[0..m) in order.
+__device__ __forceinline__ float add_in_order(float s, const float *v, int m) {
+  int r = 0;
+  for (; r + 16 <= m; r += 16) {
+    f32x4 t[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t[k] = *reinterpret_cast<const f32x4 *>(v + r + 4 * k);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s += t[k / 4][k % 4];
+  }
+  for (; r < m; ++r) s += v[r];
+  return s;
+}
 
 // The sum of column col0 + threadIdx.x in the threads below kSumCols (0 for
 // columns past the last; other threads: unspecified).  Called by the whole block.
-__device__ __forceinline__ float ordered_column_sum(const float *__restrict__ part, int nw, int col0,
-                                                    float (*lds)[kSumCols]) {
+__device__ __forceinline__ float ordered_column_sum(const float *__restrict__ part, int nw, int col0, SumLds &lds) {
   const int c = threadIdx.x % kSumCols, r0 = threadIdx.x / kSumCols;
   constexpr int kStep = kSumThreads / kSumCols;
   const bool in = col0 + c < kParams;
@@ -300,48 +344,28 @@ __device__ __forceinline__ float ordered_column_sum(const float *__restrict__ pa
     }
   };
   load(0);
-  for (int base = 0; base < nw; base += kSumRows) {
-    __syncthreads();  // the previous chunk has been added
+  for (int base = 0, b = 0; base < nw; base += kSumRows, b ^= 1) {
+    // The buffer was last read two chunks ago, before the last barrier.
 #pragma unroll
-    for (int k = 0; k < kSumPer; ++k) lds[r0 + k * kStep][c] = v[k];
-    __syncthreads();
+    for (int k = 0; k < kSumPer; ++k) lds.v[b][c][r0 + k * kStep] = v[k];
     if (base + kSumRows < nw) load(base + kSumRows);
-    if (threadIdx.x < kSumCols) {
-      const int m = nw - base < kSumRows ? nw - base : kSumRows;
-      int r = 0;
-      for (; r + 16 <= m; r += 16) {
-        float t[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) t[k] = lds[r + k][c];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) s += t[k];
-      }
-      for (; r < m; ++r) s += lds[r][c];
-    }
+    __syncthreads();
+    if (threadIdx.x < kSumCols) s = add_in_order(s, lds.v[b][c], nw - base < kSumRows ? nw - base : kSumRows);
   }
   return s;
 }
 
 // The sum of the nw wave losses in wave order, in thread 0 of the block.
-__device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss, int nw, float *lds) {
-  constexpr int kChunk = kSumRows * kSumCols;
+__device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss, int nw, SumLds &lds) {
+  constexpr int kChunk = kSumCols * kSumLd;
+  float *v = &lds.v[0][0][0];
   float s = 0.f;
   for (int base = 0; base < nw; base += kChunk) {
     const int m = nw - base < kChunk ? nw - base : kChunk;
     __syncthreads();
-    for (int k = threadIdx.x; k < m; k += kSumThreads) lds[k] = loss[base + k];
+    for (int k = threadIdx.x; k < m; k += kSumThreads) v[k] = loss[base + k];
     __syncthreads();
-    if (threadIdx.x == 0) {
-      int r = 0;
-      for (; r + 16 <= m; r += 16) {
-        float t[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) t[k] = lds[r + k];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) s += t[k];
-      }
-      for (; r < m; ++r) s += lds[r];
-    }
+    if (threadIdx.x == 0) s = add_in_order(s, v, m);
   }
   return s;
 }
@@ -350,23 +374,26 @@ __device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss
 // cosine learning-rate schedule.  The next workgroup sums the losses instead
 // and advances the step: step[1] is this step's number, which k_mlp_grad copied
 // from step[0]; only this workgroup writes step[0], which nobody reads here.
-// The workgroups after it write the next step's samples, which k_mlp_grad of
-// this step has finished reading (a launch of 6.7 us by itself).
+// The workgroups after it write the next step's samples over this step's, which
+// k_mlp_grad has finished reading: kGenPer each, so that 65,536 take the 114 CUs
+// the sum leaves and end with it (12.0 us together; 14.4 with a sample for each
+// of a workgroup's threads, 10 + 6.7 and a gap as two launches).
+constexpr int kGenPer = 640;
 __global__ __launch_bounds__(kSumThreads) void k_mlp_adam(float *P, float *Mo, float *Vo, short *W2b, short *W2Tb,
                                                           const float *grad, int nwaves, uint32_t *step,
                                                           int total_steps, float lr0, const float *loss,
                                                           float *loss_hist, Batch next) {
-  __shared__ float lds[kSumRows][kSumCols];
+  __shared__ __align__(16) SumLds lds;
   const uint32_t s = step[1];
   if (blockIdx.x > kSumBlocks) {
-    const int i = (blockIdx.x - kSumBlocks - 1) * kSumThreads + threadIdx.x;
-    if (i < next.n)
+    const int i = (blockIdx.x - kSumBlocks - 1) * kGenPer + threadIdx.x;
+    if (threadIdx.x < kGenPer && i < next.n)
       put_sample(next.gamma, next.seed, (uint64_t)(s + 1u) * (uint64_t)next.n + (uint64_t)i, i, next.norm, next.X,
                  next.Y, next.OK);
     return;
   }
   if (blockIdx.x == kSumBlocks) {
-    const float t = ordered_loss_sum(loss, nwaves, &lds[0][0]);
+    const float t = ordered_loss_sum(loss, nwaves, lds);
     if (threadIdx.x == 0) {
       loss_hist[s] = t;
       step[0] = s + 1u;
@@ -399,9 +426,9 @@ __global__ __launch_bounds__(kSumThreads) void k_mlp_adam(float *P, float *Mo, f
 // wave order in FP32.
 __global__ __launch_bounds__(kSumThreads) void k_mlp_sum(const float *part, const float *lpart, int nw, float *grad,
                                                          float *loss) {
-  __shared__ float lds[kSumRows][kSumCols];
+  __shared__ __align__(16) SumLds lds;
   if (blockIdx.x == kSumBlocks) {
-    const float t = ordered_loss_sum(lpart, nw, &lds[0][0]);
+    const float t = ordered_loss_sum(lpart, nw, lds);
     if (threadIdx.x == 0) *loss = t;
     return;
   }
@@ -471,14 +498,19 @@ hipError_t launch_gen(double gamma, uint64_t seed, int n, const float *norm, flo
 }
 hipError_t launch_grad(const float *P, const short *W2b, const short *W2Tb, const float *X, const float *Y,
                        const float *OK, float inv_n, int n, float *grad, float *loss, uint32_t *step, hipStream_t s) {
-  // n is a multiple of 256 (4 waves of 64 samples per workgroup)
-  hipLaunchKernelGGL(k_mlp_grad, dim3(n / 256), dim3(256), 0, s, P, W2b, W2Tb, X, Y, OK, inv_n, n, grad, loss, step);
+  // n is a multiple of 256, so of the 64 samples of a workgroup
+  if (W2b)
+    hipLaunchKernelGGL(k_mlp_grad<true>, dim3(n / 64), dim3(256), 0, s, P, W2b, W2Tb, X, Y, OK, inv_n, grad, loss,
+                       step);
+  else
+    hipLaunchKernelGGL(k_mlp_grad<false>, dim3(n / 64), dim3(256), 0, s, P, W2b, W2Tb, X, Y, OK, inv_n, grad, loss,
+                       step);
   return hipGetLastError();
 }
 hipError_t launch_adam(float *P, float *M, float *V, short *W2b, short *W2Tb, const float *grad, int nwaves,
                        uint32_t *step, int total_steps, float lr0, const float *loss, float *loss_hist,
                        const Batch &next, hipStream_t s) {
-  const unsigned int blocks = kSumBlocks + 1 + (next.n + kSumThreads - 1) / kSumThreads;
+  const unsigned int blocks = kSumBlocks + 1 + (next.n + kGenPer - 1) / kGenPer;
   hipLaunchKernelGGL(k_mlp_adam, dim3(blocks), dim3(kSumThreads), 0, s, P, M, V, W2b, W2Tb, grad, nwaves, step,
                      total_steps, lr0, loss, loss_hist, next);
   return hipGetLastError();
