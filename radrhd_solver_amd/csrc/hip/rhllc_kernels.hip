@@ -131,18 +131,21 @@ struct StepClose {
 // clears the buffer of the step after this one, which the step before the
 // previous one used.  This replaces a kernel between every two steps (4.2 us
 // and a launch gap) by one load of the last wave; kFoldMaxTiles has the sizes.
+//
+// ANY = false: neither d.use_tau nor d.fold.
+template <bool ANY = true>
 __device__ __forceinline__ double fold_speed(const Dev &d, double speed) {
   __shared__ unsigned long long part[kBlock];
   __shared__ double tau_lds;
   part[threadIdx.x] = (unsigned long long)__double_as_longlong(speed);
   double tau = 0.0;
-  if (d.use_tau) {
+  if (ANY && d.use_tau) {
     tau = d.tau;
     if (blockIdx.x == 0 && threadIdx.x == 0) d.sc->tau = tau;
-  } else if (!d.fold) {
+  } else if (ANY && !d.fold) {
     tau = d.sc->tau;  // before the barrier: a cold load
   }
-  if (d.fold && threadIdx.x >= kBlock - 64) {
+  if (ANY && d.fold && threadIdx.x >= kBlock - 64) {
     const int prev = d.slot == 0 ? kSpeedBufs - 1 : d.slot - 1, next = d.slot == kSpeedBufs - 1 ? 0 : d.slot + 1;
     const double s = slots_max(d, prev);
     tau = d.cfl_hmin / s;
@@ -163,6 +166,7 @@ __device__ __forceinline__ double fold_speed(const Dev &d, double speed) {
     m = __ockl_wfred_max_u64(m);
     if (threadIdx.x == 0) atomicMax(speed_slot(d, d.slot, blockIdx.x % kSpeedSlots), m);
   }
+  if (!ANY) return d.sc->tau;
   return d.fold ? tau_lds : tau;
 }
 
@@ -201,7 +205,7 @@ __device__ __forceinline__ FaceIn<MIXED> face_in(const Dev &d, int i) {
 // path the cell in the tile is bits 21-28 of the vector's fourth word (bit 29
 // set when it is the right cell) and face_far holds the other side.
 template <bool MIXED>
-__device__ __forceinline__ FaceIn<MIXED> tile_face_in(const Dev &d, int t, int i) {
+__device__ __forceinline__ FaceIn<MIXED> tile_face_in(const Dev &d, int tile_cells, int t, int i) {
   if constexpr (!MIXED) {
     return face_in<MIXED>(d, i);
   } else {
@@ -209,7 +213,7 @@ __device__ __forceinline__ FaceIn<MIXED> tile_face_in(const Dev &d, int t, int i
     o.g = ld(d.face_Sn, i);
     const int far = ld(d.face_far, i);
     const unsigned int w = (unsigned int)__float_as_int(o.g.w);
-    const int nc = t * d.tile_cells + (int)((w >> 21) & 0xFFu);
+    const int nc = t * tile_cells + (int)((w >> 21) & 0xFFu);
     const bool right = (w >> 29) & 1u;
     o.lr = right ? make_int2(far, nc) : make_int2(nc, far);
     return o;
@@ -606,11 +610,17 @@ __global__ __launch_bounds__(kBlock) void k_cell(Dev d) {
 // tiles is evaluated by both from the same inputs, to the same bits.
 // At most 96 VGPRs (five waves a SIMD): without the floor the compiler takes
 // 116 for the mixed variants and the kernel runs at four waves.
-template <int VARIANT, bool RAD, bool STATS, int EOS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_tile(Dev d) {
+//
+// ANY = false is the step as a long run on a large mesh has it, without the
+// forms that only other steps take (fold_speed's, tiles of other than 256
+// cells): branches on them cost its radiation variants 0.8% (1297 against 1286
+// us a step at 24M cells), by the registers they take in the cell phase.
+template <int VARIANT, bool RAD, bool STATS, int EOS, bool ANY>
+__device__ __forceinline__ void tile_step(const Dev &d) {
   static_assert(kTileCells <= kBlock && kSmallTileCells <= kBlock, "at most one cell per thread in the cell phase");
   constexpr bool MIXED = VARIANT >= kMixedPrev;
   extern __shared__ double2 lds_flux[];
+  const int tile_cells = ANY ? d.tile_cells : kTileCells;
   // Every other step walks the tiles backwards, so a step starts on the tiles
   // (and the arrays' ends) the previous one touched last, which the
   // memory-side cache still holds.
@@ -626,7 +636,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
       // One index into one set of arrays (the extra faces' copies follow the
       // faces): a select between two sets of base pointers would hold them in
       // VGPRs through the loop.
-      const FaceIn<MIXED> fi = tile_face_in<MIXED>(d, t, k < tm.y ? tm.x + k : d.n_faces + tm.z + (k - tm.y));
+      const FaceIn<MIXED> fi = tile_face_in<MIXED>(d, tile_cells, t, k < tm.y ? tm.x + k : d.n_faces + tm.z + (k - tm.y));
       State<double> F;
       speed = smax(speed, face_flux<MIXED, EOS, decltype(arith)>(d, fi, F));
       A[k] = make_double2(F.d, F.v[0]);
@@ -641,9 +651,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     faces(IeeeOrd());
   else
     faces(Ieee());
-  const double tau = fold_speed(d, speed);  // its barrier also publishes the LDS fluxes
-  const int c = t * d.tile_cells + (int)threadIdx.x;
-  bool live = (int)threadIdx.x < d.tile_cells && c < d.n_cells;
+  const double tau = fold_speed<ANY>(d, speed);  // its barrier also publishes the LDS fluxes
+  const int c = t * tile_cells + (int)threadIdx.x;
+  bool live = (!ANY || (int)threadIdx.x < tile_cells) && c < d.n_cells;
   State<double> U;
   double dtau = 0.0;
   float p32 = -1.f;
@@ -658,6 +668,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
   bool from_mlp = false;
   if constexpr (VARIANT == kMixedMlp) from_mlp = mlp_start(d, live, U, dtau, guess);
   finish_cell<VARIANT, RAD, STATS, EOS>(d, c, live, U, guess, from_mlp, tau);
+}
+
+template <int VARIANT, bool RAD, bool STATS, int EOS>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_tile(Dev d) {
+  tile_step<VARIANT, RAD, STATS, EOS, false>(d);
+}
+template <int VARIANT, bool RAD, bool STATS, int EOS>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_tile_any(Dev d) {
+  tile_step<VARIANT, RAD, STATS, EOS, true>(d);
 }
 
 // tau of the next step from the max signal speed (rhllc_utils.cpp:15-23):
@@ -1020,14 +1039,19 @@ hipError_t launch_cell(const Dev &d, int variant, bool rad, bool stats, hipStrea
 template <int V, int EOS>
 static void launch_tile_v(const Dev &d, bool rad, bool stats, dim3 g, size_t lds, hipStream_t s) {
   const dim3 b(kBlock);
+  const bool any = d.fold || d.use_tau || d.tile_cells != kTileCells;
   if (rad) {
     if (stats)
-      hipLaunchKernelGGL((k_tile<V, true, true, EOS>), g, b, lds, s, d);
+      hipLaunchKernelGGL((k_tile_any<V, true, true, EOS>), g, b, lds, s, d);
+    else if (any)
+      hipLaunchKernelGGL((k_tile_any<V, true, false, EOS>), g, b, lds, s, d);
     else
       hipLaunchKernelGGL((k_tile<V, true, false, EOS>), g, b, lds, s, d);
   } else {
     if (stats)
-      hipLaunchKernelGGL((k_tile<V, false, true, EOS>), g, b, lds, s, d);
+      hipLaunchKernelGGL((k_tile_any<V, false, true, EOS>), g, b, lds, s, d);
+    else if (any)
+      hipLaunchKernelGGL((k_tile_any<V, false, false, EOS>), g, b, lds, s, d);
     else
       hipLaunchKernelGGL((k_tile<V, false, false, EOS>), g, b, lds, s, d);
   }
