@@ -63,12 +63,14 @@ __device__ __forceinline__ f32x4 mfma32(bf16x4 a_lo, bf16x4 a_hi, bf16x4 b_lo, b
                                                  0, 0, 0);
 }
 
-__device__ __forceinline__ short f2bf(float x) {  // round to nearest even
-  uint32_t u = __float_as_uint(x);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (short)(u >> 16);
+// Round to nearest even: v_cvt_pk_bf16_f32, one instruction for two values
+// (in integer arithmetic it is seven; the two agree on every finite and
+// infinite value).
+__device__ __forceinline__ short f2bf(float x) { return __builtin_bit_cast(short, (__bf16)x); }
+__device__ __forceinline__ bf16x4 f2bf4(f32x4 x) {
+  typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bf16x4, __builtin_convertvector(x, b4));
 }
-__device__ __forceinline__ float bf2f(short b) { return __uint_as_float(((uint32_t)(uint16_t)b) << 16); }
 
 // silu = z s, d silu / dz = s (1 + z (1 - s)), s = sigmoid(z)
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
@@ -118,6 +120,7 @@ __device__ __forceinline__ void forward_wave(const float *__restrict__ P, const 
   bf16x4 h1[4][4];  // [q][t]
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
+    f32x4 a1[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int h = 16 * q + 4 * g + e;
@@ -125,9 +128,11 @@ __device__ __forceinline__ void forward_wave(const float *__restrict__ P, const 
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const float z = ((w0 * x[t][0] + w1 * x[t][1]) + w2 * x[t][2]) + bb;
-        h1[q][t][e] = f2bf(silu(z));
+        a1[t][e] = silu(z);
       }
     }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) h1[q][t] = f2bf4(a1[t]);
   }
   // Z2^T[h2][s] = sum_h1 W2[h2][h1] H1^T[h1][s]: tiles (u over h2, t over samples).
   float part[4] = {0.f, 0.f, 0.f, 0.f};
@@ -180,9 +185,11 @@ __device__ __forceinline__ float forward_16(const float *__restrict__ P, const s
 #pragma unroll
     for (int k = 0; k < 3; ++k) *reinterpret_cast<f32x4u *>(w + 4 * k) = ld4(P + kOffW1 + 3 * h0 + 4 * k);
     const f32x4u b = ld4(P + kOffB1 + h0);
+    f32x4 a1;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      h1[q][e] = f2bf(silu(((w[3 * e] * x[0] + w[3 * e + 1] * x[1]) + w[3 * e + 2] * x[2]) + b[e]));
+      a1[e] = silu(((w[3 * e] * x[0] + w[3 * e + 1] * x[1]) + w[3 * e + 2] * x[2]) + b[e]);
+    h1[q] = f2bf4(a1);
     __builtin_amdgcn_sched_barrier(0);  // a block of units at a time: registers
   }
   float part = 0.f;

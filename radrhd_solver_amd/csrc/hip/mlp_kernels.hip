@@ -98,9 +98,16 @@ __device__ __forceinline__ float sum16(float v) {
   return dpp_add<0x140>(v);  // row_mirror
 }
 
-// Row length of the transposed operands in LDS: 64 samples and 4 shorts of
-// padding, so the 16 rows a load touches start in different banks.
-constexpr int kLdT = kH + 4;
+// The operand of a product that contracts over the samples, from the block of
+// 16 samples x 16 units that f holds as the lanes made it (lane (g, c): units
+// 4 g + e of sample c): lane (g, c) gets unit c of the samples 4 g + e.  The
+// transposing read hands lane i of each 16 the element i % 4 of the lanes
+// i / 4, i / 4 + 4, .. of the 16, so lane (g, c) names the entry (c % 4, 4 g + c / 4);
+// the 64 lanes read all 512 bytes once.
+__device__ __forceinline__ bf16x4 read_transposed(bf16x4 *f, int g, int c) {
+  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4 *)(f + 16 * (c & 3) + 4 * g + (c >> 2)));
+}
 
 // One workgroup = 64 consecutive samples ("wave" of the partials: a single wave
 // once took them).  grad[wave][kGradStride] receives their gradient of
@@ -109,77 +116,77 @@ constexpr int kLdT = kH + 4;
 // The four waves share the hidden units: wave w has the units of block w
 // (16 w .. 16 w + 15) of both layers, and lane (g, c) of it the units
 // 16 w + 4 g + e of the samples 16 t + c.  The operands of the products that
-// contract over all units go through LDS as they are (frag), those of dW2,
-// which contracts over the samples, transposed (rows of a unit); the output's
+// contract over all units go through LDS as they are, and dW2's, which
+// contracts over the samples, are read from there transposed; the output's
 // sum over the units is taken in unit order from the waves' terms, so every
 // value is rounded as one wave taking all the units would.  A batch of 65,536
 // is then four waves a SIMD where it was one, waiting for its own chain; each
 // activation's derivative is formed with it from one sigmoid, the sums over 16
-// lanes use DPP and the vectors come in 16-byte loads.  Measured at 65,536
-// samples: 38.2 us as one wave with spilled registers, 25.2 as one wave
-// without, 18.4 so.
+// lanes use DPP and the vectors come in 16-byte loads.  Values used late are
+// loaded late, which leaves registers for four workgroups a CU: all 1,024 of
+// such a batch run at once.  dW2's partials, 16.8 MB of it, are stored past L2:
+// the sum reads them on other XCDs, and the kernel's end would wait for them to
+// be written back.  Measured at 65,536 samples: 38.2 us as one wave with spilled
+// registers, 25.2 as one wave without, 18.4 as four waves with three workgroups
+// a CU and operands transposed by 2-byte LDS writes, 17.6 without those, 14.0
+// with the streaming stores (11.4 with no stores of dW2 at all).
 //
 // PACKED: W2 and its transpose come as the BF16 copies that training keeps,
 // else they are rounded here from P (a call of its own would first need a
 // launch that makes the copies: 3.3 us and a gap).
 template <bool PACKED>
-__global__ __launch_bounds__(256, 3) void k_mlp_grad(const float *__restrict__ P, const short *__restrict__ W2b,
+__global__ __launch_bounds__(256, 4) void k_mlp_grad(const float *__restrict__ P, const short *__restrict__ W2b,
                                                      const short *__restrict__ W2Tb, const float *__restrict__ X,
                                                      const float *__restrict__ Y, const float *__restrict__ OK,
                                                      float inv_n, float *__restrict__ grad, float *__restrict__ loss,
                                                      uint32_t *step) {
   if (step && blockIdx.x == 0 && threadIdx.x == 0) step[1] = step[0];
-  __shared__ __align__(16) short h1T[kH * kLdT], dzT[kH * kLdT];  // H1^T [h1][s], dZ2^T [h2][s], bf16
-  __shared__ bf16x4 frag[4][4][64];                               // [block][t][lane]: H1, then dZ2
+  __shared__ bf16x4 h1s[4][4][64], dzs[4][4][64];  // [block][t][lane]: H1 and dZ2
   __shared__ f32x4 part0[64], term[3][4][64];  // block 0's sum and the others' terms [r][lane] of the 4 samples
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = l >> 4, c = l & 15;
   const int base = blockIdx.x * 64;
   const int h0 = 16 * w + 4 * g;  // this lane's units of both layers
   // the 4 samples s_t = 16 t + c this lane works on
-  float x[4][3], y[4], ok[4];
+  float x[4][3];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int i = base + 16 * t + c;
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int f = 0; f < 3; ++f) x[t][f] = X[3 * i + f];
-    y[t] = Y[i], ok[t] = OK[i];
-  }
+    for (int f = 0; f < 3; ++f) x[t][f] = X[3 * (base + 16 * t + c) + f];
   float w1[12];
 #pragma unroll
   for (int k = 0; k < 3; ++k) *reinterpret_cast<f32x4u *>(w1 + 4 * k) = ld4(P + kOffW1 + 3 * h0 + 4 * k);
   const f32x4u b1 = ld4(P + kOffB1 + h0), b2 = ld4(P + kOffB2 + h0), w3 = ld4(P + kOffW3 + h0);
-  bf16x4 a2w[4], a1w[4];  // rows of W2 and of W2^T
+  bf16x4 a2w[4];  // rows of W2
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     if constexpr (PACKED) {
       a2w[q] = *reinterpret_cast<const bf16x4 *>(W2b + (16 * w + c) * kH + 16 * q + 4 * g);
-      a1w[q] = *reinterpret_cast<const bf16x4 *>(W2Tb + (16 * w + c) * kH + 16 * q + 4 * g);
     } else {
       const f32x4u row = ld4(P + kOffW2 + (16 * w + c) * kH + 16 * q + 4 * g);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        a2w[q][e] = f2bf(row[e]);
-        a1w[q][e] = f2bf(P[kOffW2 + (16 * q + 4 * g + e) * kH + 16 * w + c]);
-      }
+      for (int e = 0; e < 4; ++e) a2w[q][e] = f2bf(row[e]);
     }
   }
   // ---- layer 1
   float d1[4][4];  // [t][e] dsilu
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    bf16x4 h;
+    f32x4 h;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float z = ((w1[3 * e] * x[t][0] + w1[3 * e + 1] * x[t][1]) + w1[3 * e + 2] * x[t][2]) + b1[e];
       const float s = sigmoid(z);
       d1[t][e] = s * (1.0f + z * (1.0f - s));
-      h[e] = f2bf(z * s);
-      h1T[(h0 + e) * kLdT + 16 * t + c] = h[e];
+      h[e] = z * s;
     }
-    frag[w][t][l] = h;
+    h1s[w][t][l] = f2bf4(h);
   }
   __syncthreads();
+  // The sample, its target and W2^T's rows are loaded (again) where they are
+  // used: through pointers the compiler cannot tell to be the ones above, else
+  // it would hold the values in registers.
+  asm volatile("" : "+s"(X), "+s"(Y), "+s"(OK), "+s"(W2Tb));
   // ---- layer 2
   float a2[4][4], d2[4][4];  // [t][r] silu and dsilu
   f32x4 tr[4];               // [r] the terms of the 4 samples' outputs
@@ -187,7 +194,7 @@ __global__ __launch_bounds__(256, 3) void k_mlp_grad(const float *__restrict__ P
   for (int t = 0; t < 4; ++t) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int q = 0; q < 4; q += 2) acc = mfma32(a2w[q], a2w[q + 1], frag[q][t][l], frag[q + 1][t][l], acc);
+    for (int q = 0; q < 4; q += 2) acc = mfma32(a2w[q], a2w[q + 1], h1s[q][t][l], h1s[q + 1][t][l], acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float z = acc[r] + b2[r];
@@ -220,7 +227,7 @@ __global__ __launch_bounds__(256, 3) void k_mlp_grad(const float *__restrict__ P
     float v = out[t];
     v += __shfl_xor(v, 16, 64);
     v += __shfl_xor(v, 32, 64);
-    const float d = (v + P[kOffB3] - y[t]) * ok[t];
+    const float d = (v + P[kOffB3] - Y[base + 16 * t + c]) * OK[base + 16 * t + c];
     dout[t] = 2.0f * d * inv_n;
     sq += d * d;
   }
@@ -229,16 +236,15 @@ __global__ __launch_bounds__(256, 3) void k_mlp_grad(const float *__restrict__ P
   float aw[4] = {}, ab[4] = {};
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    bf16x4 dzb;
+    f32x4 dzv;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       aw[r] += dout[t] * a2[t][r];
       const float dz = dout[t] * w3[r] * d2[t][r];
       ab[r] += dz;
-      dzb[r] = f2bf(dz);
-      dzT[(h0 + r) * kLdT + 16 * t + c] = dzb[r];
+      dzv[r] = dz;
     }
-    frag[w][t][l] = dzb;  // every wave has read H1's before the last barrier
+    dzs[w][t][l] = f2bf4(dzv);
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -247,19 +253,30 @@ __global__ __launch_bounds__(256, 3) void k_mlp_grad(const float *__restrict__ P
   }
   __syncthreads();
   // ---- dH1^T = W2^T dZ2^T, dZ1; W1 and b1 gradients
+  bf16x4 a1w[4];  // rows of W2^T
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (PACKED) {
+      a1w[q] = *reinterpret_cast<const bf16x4 *>(W2Tb + (16 * w + c) * kH + 16 * q + 4 * g);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a1w[q][e] = f2bf(P[kOffW2 + (16 * q + 4 * g + e) * kH + 16 * w + c]);
+    }
+  }
   float gW1[4][3] = {}, gB1[4] = {};
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < 4; u += 2) acc = mfma32(a1w[u], a1w[u + 1], frag[u][t][l], frag[u + 1][t][l], acc);
+    for (int u = 0; u < 4; u += 2) acc = mfma32(a1w[u], a1w[u + 1], dzs[u][t][l], dzs[u + 1][t][l], acc);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float dz = acc[e] * d1[t][e];
+      const float *xs = X + 3 * (base + 16 * t + c);
       gB1[e] += dz;
-      gW1[e][0] += dz * x[t][0];
-      gW1[e][1] += dz * x[t][1];
-      gW1[e][2] += dz * x[t][2];
+      gW1[e][0] += dz * xs[0];
+      gW1[e][1] += dz * xs[1];
+      gW1[e][2] += dz * xs[2];
     }
   }
 #pragma unroll
@@ -268,19 +285,18 @@ __global__ __launch_bounds__(256, 3) void k_mlp_grad(const float *__restrict__ P
     const int h = h0 + e;
     if (c == 0) G[kOffW1 + 3 * h] = v0, G[kOffW1 + 3 * h + 1] = v1, G[kOffW1 + 3 * h + 2] = v2, G[kOffB1 + h] = vb;
   }
-  // ---- dW2 = dZ2^T H1 from the transposed operands
+  // ---- dW2^T = H1^T dZ2: a lane's 4 values are 4 of a row of dW2
+  bf16x4 dzt[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) dzt[t] = read_transposed(dzs[w][t], g, c);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < 4; t += 2) {
-      const short *ar = dzT + (16 * w + c) * kLdT + 4 * g, *br = h1T + (16 * q + c) * kLdT + 4 * g;
-      acc = mfma32(*reinterpret_cast<const bf16x4 *>(ar + 16 * t), *reinterpret_cast<const bf16x4 *>(ar + 16 * t + 16),
-                   *reinterpret_cast<const bf16x4 *>(br + 16 * t), *reinterpret_cast<const bf16x4 *>(br + 16 * t + 16),
-                   acc);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) G[kOffW2 + (h0 + r) * kH + 16 * q + c] = acc[r];
+    for (int t = 0; t < 4; t += 2)
+      acc = mfma32(read_transposed(h1s[q][t], g, c), read_transposed(h1s[q][t + 1], g, c), dzt[t], dzt[t + 1], acc);
+    __builtin_nontemporal_store((f32x4u)acc,
+                                reinterpret_cast<f32x4u *>(G + kOffW2 + (16 * w + c) * kH + 16 * q + 4 * g));
   }
   // b3: sum of dout over the samples (group g = 0 holds each sample once)
   if (w == 0) {
