@@ -72,6 +72,20 @@ def test_gradient_is_the_sum_of_the_waves_in_order(n):
     assert np.float32(loss) == sl
 
 
+@pytest.mark.parametrize("batch", [256, 7168, 7424, 16384, 65536, 116736, 116992])
+def test_training_takes_the_next_samples_of_the_stream(batch):
+    """Step k of a training with batch B takes the samples k B .. k B + B - 1, however they are
+    spread over workgroups (64 each up to 7,296 samples, 1,024 each at 116,736, 640 above).  At a
+    learning rate too small to change a weight, its loss is the sum of those of the batches of 256
+    of the same stream.  Each is an FP32 sum in order of the waves' terms, none negative: m terms
+    are off by at most m 2^-24 of their sum."""
+    kw = dict(lr=1e-30, gamma=1.4, seed=SEED, norm_samples=4096)
+    _, parts = capi.mlp_train(steps=3 * batch // 256, batch=256, **kw)
+    _, hist = capi.mlp_train(steps=3, batch=batch, **kw)
+    want = parts.astype(np.float64).reshape(3, -1).mean(axis=1)
+    assert np.all(np.abs(hist - want) <= (batch // 64 + 4 + 2) * 2.0 ** -24 * want)
+
+
 def test_forward_matches_cpu_restatement():
     rng = np.random.default_rng(SEED + 1)
     model = _model(rng)
