@@ -1,6 +1,6 @@
 // Training and evaluation kernels of the c2p surrogate MLP (see mlp.h).
 //
-// Training step (captured in a hipGraph and replayed):
+// Training step (captured several to a hipGraph and replayed):
 //   k_mlp_grad   one workgroup per 64 samples: forward (BF16 MFMA with K = 32,
 //                FP32 accumulate),
 //                backward, gradient partials written to global memory;
@@ -393,7 +393,8 @@ __device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss
 // The workgroups after it write the next step's samples over this step's, which
 // k_mlp_grad has finished reading, spread over the 114 CUs that the sum leaves
 // (a workgroup's LDS fills its CU): the fewer waves a SIMD has, the sooner its
-// samples are done.  A training step takes 18.5 us at 1,024 samples (24.8 with
+// samples are done.  With one step a graph, which adds about 5 us to each, a
+// training step takes 18.5 us at 1,024 samples (24.8 with
 // 640 samples a workgroup at every size), 19.9 at 16,384 (26.5), 28 at 49,152
 // (31), 34 at 65,536 (34; with a launch of its own for the samples 7 more), 41 at
 // 98,304 (51).  A batch that does not fit the idle CUs at once takes 640 each:

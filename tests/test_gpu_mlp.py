@@ -86,6 +86,16 @@ def test_training_takes_the_next_samples_of_the_stream(batch):
     assert np.all(np.abs(hist - want) <= (batch // 64 + 4 + 2) * 2.0 ** -24 * want)
 
 
+def test_training_of_any_number_of_steps():
+    """Steps are replayed eight at a time, the rest launched one by one: at a learning rate too
+    small to change a weight, the losses of a shorter training are the first of a longer one."""
+    run = lambda steps: capi.mlp_train(steps=steps, batch=256, lr=1e-30, gamma=1.4, seed=SEED, norm_samples=4096)[1]
+    longest = run(25)
+    assert len(np.unique(longest)) == 25
+    for steps in (1, 7, 8, 9, 16, 24):
+        assert np.array_equal(run(steps), longest[:steps]), steps
+
+
 def test_forward_matches_cpu_restatement():
     rng = np.random.default_rng(SEED + 1)
     model = _model(rng)
