@@ -186,11 +186,12 @@ struct rhllc_solver {
   // meshes of more than kFoldMaxTiles tiles every step is closed at once.
   int slot = 0;
   bool open = false;
-  // Captured step graphs: the two-kernel step keeps one step in [0]; the
-  // tiled step keeps kGraphSteps steps starting from state buffer k in [k]
-  // (folding: from slot 1 and an open step), so a replay leaves them as they were.
+  // Captured graphs of kGraphSteps steps: the tiled step's starting from state
+  // buffer k in [k] (folding: from slot 1 and an open step), the two-kernel
+  // step's in [0]; a replay leaves buffer and slot as they were.
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   hipGraph_t graph_src[2] = {nullptr, nullptr};
+  int singles = 0;  // steps that rhllc_run launched singly for want of a graph
   float *mlp_P = nullptr;
   short *mlp_W2b = nullptr;
 
@@ -204,6 +205,7 @@ struct rhllc_solver {
   }
 
   void drop_graph() {
+    singles = 0;
     for (int k = 0; k < 2; ++k) {
       if (graph[k]) (void)hipGraphExecDestroy(graph[k]);
       if (graph_src[k]) (void)hipGraphDestroy(graph_src[k]);
@@ -241,8 +243,16 @@ struct rhllc_solver {
   // The current state, updated in place.
   Dev now() const { return dev(cur, cur); }
 
-  // State and slot buffers both return after six steps.
-  static constexpr int kGraphSteps = 2 * kSpeedBufs;
+  // State and slot buffers both return after kCycle steps.  Between two graphs
+  // the GPU idles longer than between two kernels of one, so a graph holds
+  // several cycles; more would leave more steps of a run to single launches and
+  // take longer to capture.  us a step with 6 / 12 / 24 steps a graph: 5.8 / 5.4 /
+  // 5.2 at 162 cells, 6.8 / 6.4 / 6.2 at 6,000, 17.8 / 17.4 / 17.1 at 118,098 (FP64),
+  // 32.2 / 31.8 / 31.8 at 663,552 (mixed).  A first run of 20 steps of 162 cells,
+  // which then captures nothing, takes 122 us with 24 and 188 with 6.
+  static constexpr int kCycle = 2 * kSpeedBufs;
+  static constexpr int kGraphSteps = 4 * kCycle;
+  static constexpr int kGraphWorth = 3 * kGraphSteps;
 
   bool folds() const { return tiled && n_tiles <= kFoldMaxTiles; }
 
@@ -292,13 +302,13 @@ struct rhllc_solver {
     const hipError_t e = launch_report(d, host_sc_dev, stream);
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
   }
-  // Captures graph[cur]: kGraphSteps steps (tiled) or one (two-kernel).
+  // Captures graph[cur].
   hipError_t capture() {
     const int k = cur, saved_in = last_in, saved_slot = slot;
     const bool saved_open = open;
     hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
-    for (int s = 0; s < (tiled ? kGraphSteps : 1) && e == hipSuccess; ++s) e = enqueue_step();
+    for (int s = 0; s < kGraphSteps && e == hipSuccess; ++s) e = enqueue_step();
     hipGraph_t g = nullptr;
     const hipError_t e2 = hipStreamEndCapture(stream, &g);
     cur = k;  // capture enqueues nothing; replays leave these as they find them
@@ -582,10 +592,21 @@ extern "C" int rhllc_run(rhllc_solver *h, int32_t nsteps, int32_t use_graph) {
   int32_t k = 0;
   hipError_t e = hipSuccess;
   if (use_graph) {
-    // A folding step's graph continues from an open step: the first step goes out by itself.
-    const int per = h->tiled ? rhllc_solver::kGraphSteps : 1, before = h->folds() ? 1 : 0;
-    if (nsteps >= before + per) {
-      for (; k < before && e == hipSuccess; ++k) e = h->enqueue_step();
+    // A folding step's graph continues from an open step, so the first step goes
+    // out by itself.  So do the steps that fill no graph, first (folding, in
+    // whole cycles: the slot has to be the graph's), so that the GPU has work
+    // while one is captured.  A graph is captured once its replays would have
+    // served kGraphWorth steps of this and earlier runs: a capture takes as long
+    // as about two replays save (first runs of 30 steps were 10% slower with a
+    // capture each).
+    constexpr int per = rhllc_solver::kGraphSteps, cycle = rhllc_solver::kCycle;
+    const int open = h->folds() ? 1 : 0, whole = nsteps < open ? 0 : (nsteps - open) / per * per;
+    const int rest = nsteps - whole, lead = open ? open + (rest - open) / cycle * cycle : rest;
+    const int first = h->tiled ? h->cur ^ (lead & 1) : 0;
+    if (whole > 0 && !h->graph[first] && h->singles + whole < rhllc_solver::kGraphWorth) {
+      h->singles += whole;
+    } else if (whole > 0) {
+      for (; k < lead && e == hipSuccess; ++k) e = h->enqueue_step();
       if (e == hipSuccess && !h->graph[h->cur]) e = h->capture();
       for (; k + per <= nsteps && e == hipSuccess; k += per) e = hipGraphLaunch(h->graph[h->cur], h->stream);
       h->last_in = h->tiled ? h->cur ^ 1 : h->cur;

@@ -22,6 +22,30 @@ def _l1(a, b, V):
     return [float((np.abs(a[:, k] - b[:, k]) * V).sum() / (np.abs(b[:, k]) * V).sum()) for k in range(5)]
 
 
+@pytest.mark.parametrize("schedule", [capi.SCHED_TILED, capi.SCHED_TWO_KERNEL])
+@pytest.mark.parametrize("shape", [(5, 4, 3), (77, 77, 118)])  # folding; 4,197,732 cells, 16,398 tiles: not folding
+def test_graph_replays_equal_single_launches(shape, schedule):
+    """Runs below, at and above whole graphs of 24 steps, with and without whole cycles of six
+    left over and from either state buffer, are the single launches bit for bit."""
+    m = M.kuhn_box(*shape, seed=SEED)
+    print("mesh", m.n_cells, m.n_faces, flush=True)
+    W0 = M.init_state(m, M.INIT_BLAST)
+    out = []
+    for graph in (True, False):
+        s = capi.Solver(m, cfl=0.4, schedule=schedule)
+        s.upload_W(W0)
+        got = []
+        for n in (24, 25, 23, 31, 38, 49, 55):
+            s.run(n, graph=graph)
+            s.sync()
+            st = s.stats()
+            got.append((*s.download(), st["steps"], st["t"], st["max_speed"]))
+        s.close()
+        out.append(got)
+    for a, b in zip(*out):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]) and a[2:] == b[2:]
+
+
 def test_tiled_buffer_parity_across_graph_and_eager_steps():
     """7 graph steps (three pair replays and one eager step), 3 eager, 5 graph, one
     host-tau step: 16 steps bitwise the oracle, stats and face fluxes included."""
