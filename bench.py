@@ -8,10 +8,10 @@ r < 0.1 else 1, gamma = 5/3, CFL 0.4, with a seeded FP32 radiation field
 (Ur log-uniform [1e-3, 1], |Fr| <= Ur, kappa_a, kappa_s in [0.1, 10]) applied
 as an explicit 4-momentum source after every hydro update.
 
-A "step" is one hipGraph replay of the step over the whole mesh with the
+A "step" is one step over the whole mesh, replayed from a hipGraph with the
 state resident in HBM: the tiled kernel (each workgroup computes the faces of
-256 cells into LDS and updates those cells), the surrogate-list kernel and the
-dt kernel.  `value` is the cell-updates per second of the mixed step (FP32
+256 cells into LDS and updates those cells, with the surrogate's start where it
+applies) and the dt kernel.  `value` is the cell-updates per second of the mixed step (FP32
 cell records, face vectors in FP32 plus residual bits; FP64 U, 1/V, fluxes and
 arithmetic) with the c2p surrogate start (the stored model for gamma 5/3, trained on the
 device first when there is none).  Beside it, on the same mesh and state: the
