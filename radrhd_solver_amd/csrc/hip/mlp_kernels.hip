@@ -313,14 +313,17 @@ __global__ __launch_bounds__(256, 4) void k_mlp_grad(const float *__restrict__ P
 // array, added in row (wave) order in FP32, whatever the grid.  One thread per
 // column walking the rows waits for memory once per few rows (289 us for the
 // 1,024 rows of a 65,536-sample batch).  Here a workgroup of 1,024 threads owns
-// kSumCols columns: all of it loads kSumRows rows into LDS, 16 loads in flight a
-// thread, and one thread per column adds them in order, four rows a read, while
-// the next chunk is on its way into the other buffer.  32 columns are one
+// kSumCols columns: all of it loads kSumRows rows into LDS and one thread per
+// column adds them in order, four rows a read and the next reads in flight,
+// while the next chunk is on its way into the other buffer.  32 columns are one
 // 128-byte line of a row and make 141 workgroups of the 4,481 columns; the
-// training step gives the CUs they leave the next step's samples.  10.0 us for
-// 1,024 rows.
+// training step gives the CUs they leave the next step's samples.  What bounds
+// it is the chain of adds and, before it, the first chunk's arrival: a call for
+// 65,536 gradients takes 24.0 us with 512 rows and each read waited for, 22.6
+// with the next reads in flight, 21.4 so with 256 rows, 21.3 with 128 (22.4 with
+// the loads of four chunks in flight).
 constexpr int kSumCols = 32;
-constexpr int kSumRows = 512;
+constexpr int kSumRows = 128;
 constexpr int kSumThreads = 1024;
 constexpr int kSumPer = kSumRows * kSumCols / kSumThreads;          // rows a thread loads of a chunk
 constexpr int kSumBlocks = (kParams + kSumCols - 1) / kSumCols;     // workgroups of the columns
@@ -331,15 +334,33 @@ struct SumLds {
   float v[2][kSumCols][kSumLd];
 };
 
-// s plus v[0..m) in order.
+// s plus v[0..m) in order.  The barriers keep the reads where they are, half a
+// turn before their adds.
 __device__ __forceinline__ float add_in_order(float s, const float *v, int m) {
   int r = 0;
-  for (; r + 16 <= m; r += 16) {
-    f32x4 t[4];
+  const auto load = [&](f32x4(&t)[4], int at) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) t[k] = *reinterpret_cast<const f32x4 *>(v + r + 4 * k);
+    for (int k = 0; k < 4; ++k) t[k] = *reinterpret_cast<const f32x4 *>(v + at + 4 * k);
+  };
+  const auto add = [&](const f32x4(&t)[4]) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) s += t[k / 4][k % 4];
+  };
+  if (m >= 32) {
+    f32x4 a[4], b[4];
+    load(a, 0);
+    for (; r + 64 <= m; r += 32) {
+      load(b, r + 16);
+      __builtin_amdgcn_sched_barrier(0);
+      add(a);
+      load(a, r + 32);
+      __builtin_amdgcn_sched_barrier(0);
+      add(b);
+    }
+    load(b, r + 16);
+    add(a);
+    add(b);
+    r += 32;
   }
   for (; r < m; ++r) s += v[r];
   return s;
@@ -392,7 +413,7 @@ __device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss
 // from step[0]; only this workgroup writes step[0], which nobody reads here.
 // The workgroups after it write the next step's samples over this step's, which
 // k_mlp_grad has finished reading, spread over the 114 CUs that the sum leaves
-// (a workgroup's LDS fills its CU): the fewer waves a SIMD has, the sooner its
+// (a workgroup's 16 waves fill its CU): the fewer waves a SIMD has, the sooner its
 // samples are done.  With one step a graph, which adds about 5 us to each, a
 // training step takes 18.5 us at 1,024 samples (24.8 with
 // 640 samples a workgroup at every size), 19.9 at 16,384 (26.5), 28 at 49,152

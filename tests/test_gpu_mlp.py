@@ -72,6 +72,12 @@ def test_gradient_is_the_sum_of_the_waves_in_order(n):
     assert np.float32(loss) == sl
 
 
+@pytest.mark.parametrize("waves", [32, 36, 60, 64, 100, 128, 132, 192, 288])
+def test_gradient_sum_at_the_edges_of_chunks_and_reads(waves):
+    """The same at whole and partial chunks of 128 waves and turns of 32 of their reads."""
+    test_gradient_is_the_sum_of_the_waves_in_order(64 * waves)
+
+
 @pytest.mark.parametrize("batch", [256, 7168, 7424, 16384, 65536, 116736, 116992])
 def test_training_takes_the_next_samples_of_the_stream(batch):
     """Step k of a training with batch B takes the samples k B .. k B + B - 1, however they are
