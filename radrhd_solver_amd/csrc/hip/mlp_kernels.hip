@@ -53,7 +53,10 @@ __device__ void make_sample(double gamma, uint64_t seed, uint64_t k, float x[3],
   const double Gg = gamma / (gamma - 1.0);
   rhllc_dev::p2c<double, Ieee>(Gg, W, U);
   int it = 0;
-  const int code = rhllc_dev::c2p(Gg, U, Wc, -1.0, it);
+  // The states of the box are ordinary unless gamma is extreme; the same bits
+  // either way (k_mlp_adam, which waits for these, 12.0 -> 11.8 us).
+  const int code = rhllc_dev::ordinary(U) ? rhllc_dev::c2p<rhllc_dev::IeeeOrd>(Gg, U, Wc, -1.0, it)
+                                          : rhllc_dev::c2p<Ieee>(Gg, U, Wc, -1.0, it);
   const double m = sqrt(rhllc_dev::dot3(U.v, U.v));
   double p0;
   raw_features(Gg, U.d, m, U.p, x, p0);
