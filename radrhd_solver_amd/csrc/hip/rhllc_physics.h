@@ -604,10 +604,12 @@ struct MixedIn {
   double sigma;  // s - D
 };
 
-// The record of an FP64 primitive state (|v| < 1).
+// The record of an FP64 primitive state (|v| < 1).  Its sums are fused as
+// written: `fp contract(fast)` leaves the choice between two products of a sum
+// to the kernel around it, and a state uploaded with TAUB then had a sigma
+// other than the one the step stores for the same state.
 template <int EOS = kIdeal>
 __device__ __forceinline__ void mixed_record(double Gg, const State<double> &W, float4 &va, double2 &sg) {
-#pragma clang fp contract(fast)
   using A = FaceFast;  // 4.2e-15: sigma and D match the FP32 v and p far below their rounding
   va = make_float4((float)W.v[0], (float)W.v[1], (float)W.v[2], (float)W.p);
   const double rho = (float)W.d, p = va.w;
@@ -615,16 +617,17 @@ __device__ __forceinline__ void mixed_record(double Gg, const State<double> &W, 
   const double vv = dot3c(v, v);
   const double lor = A::rsqrt(1.0 - vv);  // one reciprocal root: 4.2e-15
   const double lor2 = lor * lor;
-  double rhm1;  // rho (h - 1)
-  if (EOS == kIdeal) {
-    rhm1 = Gg * p;
+  const double wm1 = A::div(lor2 * vv, lor + 1.0);  // W - 1 = W^2 v^2 / (W + 1)
+  // sigma = s - D = rho W (h W - 1) = W (rho (h - 1) W + rho (W - 1))
+  if constexpr (EOS == kIdeal) {
+    sg.x = lor * fma(Gg * p, lor, rho * wm1);
   } else {
-    const double th = A::div(p, rho);
-    const double r = A::sqrt_(2.25 * th * th + 1.0);
-    rhm1 = 2.5 * p + rho * A::div(2.25 * th * th, r + 1.0);  // rho (h - 1) without the cancellation
+    const double th = A::div(p, rho), th2 = 2.25 * th;
+    const double r = A::sqrt_(fma(th2, th, 1.0));
+    // rho (h - 1) without the cancellation
+    const double rhm1 = fma(2.5, p, rho * A::div(th2 * th, r + 1.0));
+    sg.x = lor * fma(rho, wm1, rhm1 * lor);
   }
-  // sigma = s - D = rho W (h W - 1) = W (rho (h - 1) W + rho (W - 1)), W - 1 = W^2 v^2 / (W + 1)
-  sg.x = lor * (rhm1 * lor + rho * A::div(lor2 * vv, lor + 1.0));
   sg.y = rho * lor;
 }
 
