@@ -441,8 +441,11 @@ __device__ __forceinline__ int cell_c2p(const Dev &d, const State<double> &U, St
   if constexpr (MIXED) {
     return c2p<Fast, EOS>(d.Gg, U, W, guess, iters);
   } else {
-    // (No quotient has the start p alone above or below the line; alpha = E + p must not overflow.)
-    return ordinary(U) & (guess < 0x1p100) ? c2p<IeeeOrd, EOS>(d.Gg, U, W, guess, iters) : c2p<Ieee, EOS>(d.Gg, U, W, guess, iters);
+    // The start counts as well: where D h Gamma is E to the last bit, the first
+    // quotient's numerator is the start alone, and the residual of a quotient
+    // of 1e-304 is subnormal.  alpha = E + p must not overflow either.
+    const bool plain = ordinary(U) & ((guess <= 0.0) | ordinary_pos(guess));
+    return plain ? c2p<IeeeOrd, EOS>(d.Gg, U, W, guess, iters) : c2p<Ieee, EOS>(d.Gg, U, W, guess, iters);
   }
 }
 

@@ -59,3 +59,45 @@ def test_single_cells_beyond_the_line(cell, eos):
     W0[7, 0], W0[7, 4] = cell
     W0[7, 1:4] = 0.0
     _check(W0, m, eos, steps=6)
+
+
+def _check_starts(W0, m, eos, steps):
+    """Each step's W from its U, cell by cell, with the scaled quotients and the stored pressure as
+    the start.  Cells that PhysPressureFix rewrote are left out: they hold its pressure, 1e-12, and a U
+    of its own.  Returns the share of the others."""
+    s = capi.Solver(m, cfl=0.4, h_min=m.h_min(), eos=eos, guess=capi.GUESS_PREVIOUS)
+    s.upload_W(W0)
+    W, fixed = s.download()[0], 0
+    for _ in range(steps):
+        s.run(1)
+        start = W[:, 4].copy()
+        W, U = s.download()
+        ref, code, _ = capi.eval_c2p(U, guess=start, eos=eos)
+        ok = W[:, 4] != 1e-12
+        fixed += (~ok).sum()
+        assert (code[ok] == 0).all()
+        assert np.array_equal(W[ok].view(np.uint64), ref[ok].view(np.uint64))
+    assert fixed == s.stats()["fix_calls"]
+    s.close()
+    return 1 - fixed / (steps * m.n_cells)
+
+
+@pytest.mark.parametrize("eos", [capi.EOS_IDEAL, capi.EOS_TAUB])
+@pytest.mark.parametrize("log2", [-140, -100, 0, 92, 99, 140])
+def test_previous_pressure_starts(log2, eos):
+    m = M.kuhn_box(7, 6, 5, seed=SEED)
+    W0 = M.init_state(m, M.INIT_BLAST, params=[0.5, 0.5, 0.5, 0.3, 1.0, 1000.0, 1.0])
+    W0[:, [0, 4]] *= 2.0 ** log2
+    assert _check_starts(W0, m, eos, steps=8) > 0.9
+
+
+@pytest.mark.parametrize("eos", [capi.EOS_IDEAL, capi.EOS_TAUB])
+@pytest.mark.parametrize("log10", [-323, -312, -308, -305, -303, -200, -31, -28, 31])
+def test_previous_pressure_starts_beyond_the_line(log10, eos):
+    """Moving gas whose U is ordinary and whose pressures are far from the line (up to a decade
+    above the given power of ten; cold enough, the first quotient is the start over a number near 1)."""
+    m = M.kuhn_box(12, 11, 10, seed=SEED)
+    rng = np.random.default_rng(SEED)
+    W0 = M.init_state(m, M.INIT_UNIFORM, params=[1.0, 0.1, 0.2, -0.15, 1.0])
+    W0[:, 4] = 10.0 ** log10 * 10 ** rng.uniform(0, 1, m.n_cells)
+    assert _check_starts(W0, m, eos, steps=2) > 0.1
