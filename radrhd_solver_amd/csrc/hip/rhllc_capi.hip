@@ -218,6 +218,7 @@ struct rhllc_solver {
     drop_graph();
     if (stream) (void)hipStreamSynchronize(stream);
     for (void *p : allocs) (void)hipFree(p);
+    if (face_old_to_new) (void)hipFree(face_old_to_new);
     if (rad_FU) (void)hipFree(rad_FU);
     if (rad_FU_add) (void)hipFree(rad_FU_add);
     if (rad_T) (void)hipFree(rad_T);
@@ -685,12 +686,13 @@ extern "C" int rhllc_download_face_flux(rhllc_solver *h, double *F) {
     std::memset(F, 0, sizeof(double) * 5 * (size_t)nf);
     return RHLLC_OK;
   }
-  if (!h->face_old_to_new) {
-    HIP_TRY(h->alloc(&h->face_old_to_new, nf));
-    HIP_TRY(hipMemcpy(h->face_old_to_new, h->face_old_to_new_host.data(), sizeof(int32_t) * nf,
-                      hipMemcpyHostToDevice));
-    rhllc_mesh::RawVec<int32_t>().swap(h->face_old_to_new_host);
-  }
+  HIP_TRY(rhllc_records::fill_once(
+      h->face_old_to_new, [&](int32_t **p) { return hipMalloc((void **)p, sizeof(int32_t) * nf); },
+      [&](int32_t *p) {
+        return hipMemcpy(p, h->face_old_to_new_host.data(), sizeof(int32_t) * nf, hipMemcpyHostToDevice);
+      },
+      [](int32_t *p) { (void)hipFree(p); }));
+  rhllc_mesh::RawVec<int32_t>().swap(h->face_old_to_new_host);
   // The tiled step keeps its fluxes in LDS; they are recomputed, to the same
   // bits, from the state the last step read (its input buffer is intact).
   const Dev d = h->tiled ? h->dev(h->last_in, h->last_in) : h->now();

@@ -15,4 +15,22 @@ void scatter(void *recs, int64_t stride, int64_t off_a, int64_t off_b, int64_t n
 // memcpy over several threads.
 void copy(void *dst, const void *src, size_t bytes);
 
+// Fills an array on its first use.  alloc(&p), then fill(p); slot is set once
+// both have returned 0, so a failure leaves it null for the next use to try
+// again, with release(p) called if only fill failed.
+template <typename T, typename Alloc, typename Fill, typename Release>
+auto fill_once(T *&slot, Alloc alloc, Fill fill, Release release) -> decltype(alloc(&slot)) {
+  if (slot) return decltype(alloc(&slot))(0);
+  T *p = nullptr;
+  auto e = alloc(&p);
+  if (e != 0) return e;
+  e = fill(p);
+  if (e != 0) {
+    release(p);
+    return e;
+  }
+  slot = p;
+  return e;
+}
+
 }  // namespace rhllc_records
