@@ -141,8 +141,11 @@ int rhllc_step(rhllc_solver *h, double tau, double *max_speed);
 
 /* nsteps steps with tau computed on the device between steps
  * (tau_{k+1} = CFL*h_min/max_speed_k, rhllc_utils.cpp:15-23), starting from
- * the device's current tau.  use_graph = 1 replays a captured hipGraph of
- * the step.  Asynchronous on the handle's stream; rhllc_sync waits. */
+ * the device's current tau.  use_graph = 1 replays hipGraphs of 24 steps, one
+ * captured for each state buffer that runs start from, once its replays would
+ * have served 72 steps of this and earlier runs; steps that fill no graph (and
+ * the first of a run where the steps fold the maximum) are launched singly.
+ * Asynchronous on the handle's stream; rhllc_sync waits. */
 int rhllc_run(rhllc_solver *h, int32_t nsteps, int32_t use_graph);
 int rhllc_sync(rhllc_solver *h);
 
@@ -219,6 +222,14 @@ int rhllc_add_rad_flux_tensor(rhllc_solver *h, double tau, const float *Ur, cons
  * out[1] cell kernel (tiled step: nothing but the gap between two events),
  * out[2] dt kernel, out[3] whole step. */
 int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]);
+
+/* How a handle takes its steps, for tests and tools; no counterpart in the
+ * reference.  out[0] cells a tile (0: the two-kernel step), out[1] 1 when the
+ * steps of a run take the previous step's speed maximum themselves (0: a
+ * kernel between the steps does), out[2] graphs replayed by rhllc_run so far
+ * (of 24 steps each), out[3] FP64 path: 1 while the faces take the unscaled
+ * quotients of ordinary states.  Waits for the queued steps. */
+int rhllc_step_form(rhllc_solver *h, int64_t out[4]);
 
 /* The tiled step's layout of a mesh at 256 cells a tile (a handle on a mesh
  * too small to fill the chip uses 64), computed on the host (no device is

@@ -111,6 +111,7 @@ SIGNATURES = {
     "rhllc_set_opacity_table": (C.c_int, [_vp, _i32, _i32, _vp, _vp]),
     "rhllc_time_kernels": (C.c_int, [_vp, _i32, _vp]),
     "rhllc_info": (C.c_int, [_vp, _vp, _vp, _vp]),
+    "rhllc_step_form": (C.c_int, [_vp, _vp]),
     "rhllc_tile_layout": (C.c_int, [_i64, _vp, _i64, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "rhllc_pack_face_vectors": (C.c_int, [_i64, _vp, _vp]),
     "rhllc_eval_flux": (C.c_int, [_i32, _i32, _dbl, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
@@ -305,6 +306,11 @@ class Solver:
         out = np.zeros(4)
         check(_lib().rhllc_time_kernels(self.h, nsteps, out.ctypes.data))
         return {"face_ms": out[0], "cell_ms": out[1], "dt_ms": out[2], "step_ms": out[3]}
+
+    def step_form(self) -> dict:
+        out = np.zeros(4, np.int64)
+        check(_lib().rhllc_step_form(self.h, out.ctypes.data))
+        return {"tile_cells": int(out[0]), "folds": bool(out[1]), "replays": int(out[2]), "unscaled": bool(out[3])}
 
     def algorithmic_bytes(self) -> int:
         b = C.c_int64()

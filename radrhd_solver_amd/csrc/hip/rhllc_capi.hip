@@ -192,6 +192,7 @@ struct rhllc_solver {
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   hipGraph_t graph_src[2] = {nullptr, nullptr};
   int singles = 0;  // steps that rhllc_run launched singly for want of a graph
+  int64_t replays = 0;
   float *mlp_P = nullptr;
   short *mlp_W2b = nullptr;
 
@@ -609,7 +610,8 @@ extern "C" int rhllc_run(rhllc_solver *h, int32_t nsteps, int32_t use_graph) {
     } else if (whole > 0) {
       for (; k < lead && e == hipSuccess; ++k) e = h->enqueue_step();
       if (e == hipSuccess && !h->graph[h->cur]) e = h->capture();
-      for (; k + per <= nsteps && e == hipSuccess; k += per) e = hipGraphLaunch(h->graph[h->cur], h->stream);
+      for (; k + per <= nsteps && e == hipSuccess; k += per)
+        if ((e = hipGraphLaunch(h->graph[h->cur], h->stream)) == hipSuccess) ++h->replays;
       h->last_in = h->tiled ? h->cur ^ 1 : h->cur;
     }
   }
@@ -949,6 +951,17 @@ extern "C" int rhllc_info(rhllc_solver *h, int64_t *n_cells, int64_t *n_faces, i
     *device_bytes = h->mixed ? 161 * N + 64 * F : 233 * N + 120 * F;
     if (h->rad) *device_bytes += 24 * N;
   }
+  return RHLLC_OK;
+}
+
+extern "C" int rhllc_step_form(rhllc_solver *h, int64_t out[4]) {
+  if (!h || !out) return fail(RHLLC_ERR_ARG, "null argument");
+  HIP_TRY(hipSetDevice(h->prm.device));
+  HIP_TRY(h->fetch_scalars());
+  out[0] = h->tiled ? h->d.tile_cells : 0;
+  out[1] = h->folds();
+  out[2] = h->replays;
+  out[3] = h->tiled && !h->mixed && h->host_sc->unusual == 0;
   return RHLLC_OK;
 }
 
