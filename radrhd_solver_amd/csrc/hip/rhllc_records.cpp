@@ -3,18 +3,26 @@
 #include <algorithm>
 #include <cstring>
 
+#include <omp.h>
+
 namespace rhllc_records {
 namespace {
 
 constexpr int64_t kField = 40;
 // Below this many bytes one thread is faster than waking the others.
 constexpr int64_t kParallelBytes = 1 << 18;
+// More threads than this bring nothing (3.07M records of 136 bytes up / down,
+// ms: 10.2 / 14.5 with 1 thread, 3.0 / 5.0 with 4, 2.8 / 4.9 with 8, 2.6 / 4.9 with
+// 16), and the copies of several processes of a node would take each other's
+// cores.
+constexpr int kMaxThreads = 16;
 
 template <typename Fn>
 void over_blocks(int64_t n, int64_t bytes_each, Fn fn) {
   constexpr int64_t kBlock = 1024;
   const int64_t nb = (n + kBlock - 1) / kBlock;
-#pragma omp parallel for schedule(static) if (n * bytes_each > kParallelBytes)
+  const int threads = n * bytes_each > kParallelBytes ? std::min(omp_get_max_threads(), kMaxThreads) : 1;
+#pragma omp parallel for schedule(static) num_threads(threads)
   for (int64_t b = 0; b < nb; ++b) fn(b * kBlock, std::min(n, (b + 1) * kBlock));
 }
 
