@@ -193,6 +193,7 @@ struct rhllc_solver {
   hipGraph_t graph_src[2] = {nullptr, nullptr};
   int singles = 0;  // steps that rhllc_run launched singly for want of a graph
   int64_t replays = 0;
+  unsigned int upload = 1;  // number of the last state upload (Scalars::upload; 1: none yet)
   float *mlp_P = nullptr;
   short *mlp_W2b = nullptr;
 
@@ -502,6 +503,7 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   std::memset(h->host_sc, 0, sizeof(Scalars));
   h->host_sc->tau = d.cfl_hmin / 1.0;
   h->host_sc->last_speed = 1.0;
+  h->host_sc->upload = h->upload;
   HIP_TRY(hipMemcpy(d.sc, h->host_sc, sizeof(Scalars), hipMemcpyHostToDevice));
   HIP_TRY(launch_clear_scalars(h->now(), h->stream));
   HIP_TRY(launch_ghost_cell(h->dev(0, 1), mixed, h->stream));
@@ -524,14 +526,16 @@ extern "C" int rhllc_upload_state(rhllc_solver *h, const void *recs, int64_t str
   // On the handle's stream, so after what rhllc_run left in flight.
   const Dev d = h->now();
   const bool conv = off_conv >= 0;
+  h->has_state = false;  // until all of it is on its way
+  ++h->upload;
   HIP_TRY(h->staging.send(
       h->n_cells, conv ? 80 : 40, h->stream,
       [&](int64_t i, int64_t n, void *chunk) {
         rhllc_records::gather(static_cast<const uint8_t *>(recs) + i * stride, stride, off_phys, off_conv, n, chunk);
       },
       [&](int i, int n, void *chunk) {
-        return launch_unpack_state(d, h->mixed, h->cell_old_to_new, i, n, conv, !conv, static_cast<double *>(chunk),
-                                   h->stream);
+        return launch_unpack_state(d, h->mixed, h->cell_old_to_new, i, n, conv, !conv, h->upload,
+                                   static_cast<double *>(chunk), h->stream);
       }));
   h->has_state = true;
   h->last_in = -1;
@@ -961,7 +965,7 @@ extern "C" int rhllc_step_form(rhllc_solver *h, int64_t out[4]) {
   out[0] = h->tiled ? h->d.tile_cells : 0;
   out[1] = h->folds();
   out[2] = h->replays;
-  out[3] = h->tiled && !h->mixed && h->host_sc->unusual == 0;
+  out[3] = h->tiled && !h->mixed && h->host_sc->unusual != h->host_sc->upload;
   return RHLLC_OK;
 }
 

@@ -37,7 +37,12 @@ struct Scalars {
   unsigned long long max_residual_bits;
   unsigned long long mlp_starts;
   unsigned long long fix_mark;  // fix_fail when the moments of rhllc_add_rad_flux arrived
-  unsigned long long unusual;  // FP64 path: a state that is not `ordinary` was stored (stays set)
+  // FP64 path: the number of the last upload, and the one since which a state
+  // that is not `ordinary` was stored: equal, so one word holds both, and an
+  // upload clears the mark by its number alone, whatever its other blocks find.
+  unsigned int upload, unusual;
+  unsigned int ghost_unusual;  // a ghost state is not ordinary: every upload's mark is set
+  unsigned int pad;
 };
 
 // Everything a kernel needs, passed by value.  Cells and faces are in the
@@ -135,9 +140,10 @@ enum Variant : int {
 // State transfer of cells [first, first + n) of the caller's numbering, n
 // entries of 5 or 10 doubles at `staged` (pinned host memory, 16-byte aligned).
 // unpack: W, or W and U (conv); without U the state is W's (HllcPhysToConv).
-// reset: the time loop starts over (rhllc::Init).
+// reset: the time loop starts over (rhllc::Init).  upload: its number, the same
+// for all its chunks and another than the last one's.
 hipError_t launch_unpack_state(const Dev &d, bool mixed, const int32_t *old_to_new, int first, int n, bool conv,
-                               bool reset, const double *staged, hipStream_t s);
+                               bool reset, unsigned int upload, const double *staged, hipStream_t s);
 hipError_t launch_pack_state(const Dev &d, bool mixed, const int32_t *old_to_new, int first, int n, bool phys,
                              bool conv, double *staged, hipStream_t s);
 // Per-cell FP32 fields of cells [first, first + n): the regions Ur[n], Fr[3 n]

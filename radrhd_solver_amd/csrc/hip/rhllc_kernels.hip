@@ -429,10 +429,16 @@ __device__ __forceinline__ void update_U(const Dev &d, int c, double tau, const 
 }
 
 // Every kernel that stores an FP64 state calls this: the faces of a step use
-// IeeeOrd only while all stored states are ordinary.
+// IeeeOrd only while all states stored since the last upload are ordinary.
 __device__ __forceinline__ void note_unusual(const Dev &d, const State<double> &U, const State<double> &W) {
-  if (!(ordinary(U) & ordinary(W))) d.sc->unusual = 1;
+  if (!(ordinary(U) & ordinary(W))) d.sc->unusual = d.sc->upload;
 }
+__device__ __forceinline__ bool all_ordinary(const Dev &d) {
+  const uint2 u = *reinterpret_cast<const uint2 *>(&d.sc->upload);
+  return u.x != u.y;
+}
+static_assert(offsetof(Scalars, upload) % 8 == 0 && offsetof(Scalars, unusual) == offsetof(Scalars, upload) + 4,
+              "one word");
 
 // c2p of a cell: on the FP64 path IeeeOrd where the state is ordinary.
 template <bool MIXED, int EOS>
@@ -650,7 +656,7 @@ __device__ __forceinline__ void tile_step(const Dev &d) {
   // The FP64 faces of ordinary states, all of a step's input or none (a flag
   // set in this launch concerns the next step's input; either way the bits are
   // the same).
-  if (!MIXED && d.sc->unusual == 0)
+  if (!MIXED && all_ordinary(d))
     faces(IeeeOrd());
   else
     faces(Ieee());
@@ -719,7 +725,10 @@ __global__ void k_ghost_cell(Dev d, bool mixed) {
   d.U4o[c] = u, d.UEo[c] = gu[4], d.W4o[c] = w, d.Wpo[c] = W.p;
   State<double> U;
   U.d = gu[0], U.v[0] = gu[1], U.v[1] = gu[2], U.v[2] = gu[3], U.p = gu[4];
-  if (W.d != 0.0 || U.d != 0.0) note_unusual(d, U, W);  // an entry that no face uses is all zeros
+  if ((W.d != 0.0 || U.d != 0.0) && !(ordinary(U) & ordinary(W))) {  // an entry that no face uses is all zeros
+    d.sc->ghost_unusual = 1;
+    d.sc->unusual = d.sc->upload;
+  }
 }
 
 // The radiation source on its own, after a step without it: AddRadFlux then
@@ -795,13 +804,18 @@ __device__ __forceinline__ void staged_store(double *__restrict__ dst, const dou
 // the cell records.  reset: rhllc::Init's time (rhllc_init.cpp:190-192).
 template <bool MIXED, int EOS>
 __global__ __launch_bounds__(kBlock) void k_unpack_state(Dev d, const int32_t *old_to_new, int first, int n,
-                                                         bool conv, bool reset, const double *staged) {
+                                                         bool conv, bool reset, unsigned int upload,
+                                                         const double *staged) {
   __shared__ __align__(16) double buf[10 * kBlock];
   const int b0 = blockIdx.x * kBlock, w = conv ? 10 : 5;
   const int m = n - b0 < kBlock ? n - b0 : kBlock;
   staged_load(staged + (size_t)b0 * w, buf, m * w);
   __syncthreads();
   if (reset && b0 == 0 && threadIdx.x == 0) d.sc->tau = d.cfl_hmin / 1.0, d.sc->t = 0.0, d.sc->last_speed = 1.0;
+  if (!MIXED && first + b0 == 0 && threadIdx.x == 0) {
+    d.sc->upload = upload;
+    if (d.sc->ghost_unusual) d.sc->unusual = upload;
+  }
   if ((int)threadIdx.x >= m) return;
   const int c = old_to_new[first + b0 + threadIdx.x];
   const double *p = buf + threadIdx.x * w;
@@ -818,7 +832,7 @@ __global__ __launch_bounds__(kBlock) void k_unpack_state(Dev d, const int32_t *o
   } else {
     st(d.W4, c, make_double4(W.d, W.v[0], W.v[1], W.v[2]));
     st(d.Wp, c, W.p);
-    note_unusual(d, U, W);
+    if (!(ordinary(U) & ordinary(W))) d.sc->unusual = upload;  // (the word `upload` may not be written yet)
   }
 }
 
@@ -931,9 +945,9 @@ static void pack_state_v(const Dev &d, const int32_t *o2n, int first, int n, boo
 }
 template <bool MIXED, int EOS>
 static void unpack_state_v(const Dev &d, const int32_t *o2n, int first, int n, bool conv, bool reset,
-                           const double *staged, hipStream_t s) {
+                           unsigned int upload, const double *staged, hipStream_t s) {
   hipLaunchKernelGGL((k_unpack_state<MIXED, EOS>), dim3(blocks_for(n)), dim3(kBlock), 0, s, d, o2n, first, n, conv,
-                     reset, staged);
+                     reset, upload, staged);
 }
 template <bool MIXED, int EOS>
 static void face_out_v(const Dev &d, bool stored, const int32_t *o2n, int first, int n, double *staged,
@@ -947,12 +961,11 @@ static void face_out_v(const Dev &d, bool stored, const int32_t *o2n, int first,
 }
 
 hipError_t launch_unpack_state(const Dev &d, bool mixed, const int32_t *o2n, int first, int n, bool conv, bool reset,
-                               const double *staged, hipStream_t s) {
+                               unsigned int upload, const double *staged, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  if (d.eos == kTaub)
-    (mixed ? unpack_state_v<true, kTaub> : unpack_state_v<false, kTaub>)(d, o2n, first, n, conv, reset, staged, s);
-  else
-    (mixed ? unpack_state_v<true, kIdeal> : unpack_state_v<false, kIdeal>)(d, o2n, first, n, conv, reset, staged, s);
+  const auto launch = d.eos == kTaub ? (mixed ? unpack_state_v<true, kTaub> : unpack_state_v<false, kTaub>)
+                                     : (mixed ? unpack_state_v<true, kIdeal> : unpack_state_v<false, kIdeal>);
+  launch(d, o2n, first, n, conv, reset, upload, staged, s);
   return hipGetLastError();
 }
 hipError_t launch_pack_state(const Dev &d, bool mixed, const int32_t *o2n, int first, int n, bool phys, bool conv,

@@ -101,3 +101,66 @@ def test_previous_pressure_starts_beyond_the_line(log10, eos):
     W0 = M.init_state(m, M.INIT_UNIFORM, params=[1.0, 0.1, 0.2, -0.15, 1.0])
     W0[:, 4] = 10.0 ** log10 * 10 ** rng.uniform(0, 1, m.n_cells)
     assert _check_starts(W0, m, eos, steps=2) > 0.1
+
+
+def test_an_upload_of_ordinary_states_returns_to_the_unscaled_form():
+    """The mark of a state beyond the line lasts until the next upload, whichever chunk of an upload
+    the state comes in, with W alone or W and U, and through graph replays."""
+    m = M.kuhn_box(39, 39, 39, seed=SEED)  # 355,914 cells: two chunks of W, four of W and U
+    n = m.n_cells
+    W0 = M.init_state(m, M.INIT_BLAST, params=[0.5, 0.5, 0.5, 0.3, 1.0, 10.0, 1.0])
+    _, U0 = O.p2c(W0)
+    s = capi.Solver(m, cfl=0.4, h_min=m.h_min())
+    s.upload_W(W0)
+    assert s.step_form()["unscaled"]
+    for cell in (0, n // 2, n - 1):
+        for whole in (False, True):
+            W1 = W0.copy()
+            W1[cell, 4] = 1e-33
+            _, U1 = O.p2c(W1)
+            s.upload(W1, U1) if whole else s.upload_W(W1)
+            assert not s.step_form()["unscaled"]
+            s.run(1)
+            assert not s.step_form()["unscaled"]
+            s.upload(W0, U0) if whole else s.upload_W(W0)
+            assert s.step_form()["unscaled"]
+            s.run(1)
+            assert s.step_form()["unscaled"]
+    s.close()
+
+
+def test_the_mark_under_replays():
+    m = M.kuhn_box(6, 5, 4, seed=SEED)
+    h = m.h_min()
+    W0 = M.init_state(m, M.INIT_BLAST, params=[0.5, 0.5, 0.5, 0.3, 1.0, 10.0, 1.0])
+    W1 = W0.copy()
+    W1[7, 4] = 1e-33
+    s = capi.Solver(m, cfl=0.4, h_min=h)
+    for W in (W1, W0, W1, W0):
+        st = O.State(m, W)
+        st.run(0.4, h, 73)
+        s.upload_W(W)
+        before = s.step_form()
+        assert before["unscaled"] == (W is W0)
+        s.run(73)
+        s.sync()
+        after = s.step_form()
+        assert after["replays"] == before["replays"] + 3 and after["unscaled"] == (W is W0)
+        for a, b in zip(s.download(), (st.W, st.U)):
+            assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
+    s.close()
+
+
+def test_a_ghost_state_beyond_the_line_marks_every_upload():
+    m = M.kuhn_box(5, 4, 3, seed=SEED)
+    W0 = M.init_state(m, M.INIT_BLAST, params=[0.5, 0.5, 0.5, 0.3, 1.0, 10.0, 1.0])
+    for p, unscaled in ((0.1, True), (1e-40, False)):
+        w = np.array([[0.1, 0.9, 0.0, 0.0, p]])
+        _, u = O.p2c(w)
+        s = capi.Solver(m, cfl=0.4, out_source=(w[0], u[0]))
+        for _ in range(2):
+            s.upload_W(W0)
+            assert s.step_form()["unscaled"] == unscaled
+            s.run(1)
+            assert s.step_form()["unscaled"] == unscaled
+        s.close()
