@@ -45,22 +45,43 @@ int hip_fail(hipError_t e, const char *what) {
 // in one pass where a 256-cell tile needs three, so a step that waits for one
 // workgroup's chain of loads and divides is shorter; but only one of its four
 // waves has cells, and 37% of the faces are shared with another tile (23% at
-// 256), so it loses once every CU has several workgroups.  Measured, us a step
-// with 64 / 256 cells: FP64 7.7 / 10.8 at 6,000 cells, 11.2 / 12.7 at 34,992,
-// 15.9 / 15.5 at 55,566 (TAUB), 20.5 / 19.5 at 118,098; mixed 5.5 / 7.4, 7.4 / 8.4,
-// 9.1 / 9.7, 13.9 / 13.8, 14.5 / 15.1 at 162,000, 16.2 / 16.2 at 215,622.  Just
-// past one 256-cell tile per CU (65,536 cells) the second workgroup of a few
-// CUs costs the FP64 step 19.0 against 17.7 (82,944 cells).
-int32_t tile_cells_for(int64_t n, bool mixed) {
-  constexpr int64_t kPerRound = 256 * kTileCells;  // one tile on each of 256 CUs
-  if (mixed) return n <= 5 * kPerRound / 2 ? kSmallTileCells : kTileCells;
-  return n <= 3 * kPerRound / 4 || (n > kPerRound && n <= 3 * kPerRound / 2) ? kSmallTileCells : kTileCells;
+// 256), so it loses once every CU has several workgroups.  With 256-cell tiles
+// the time jumps wherever some CUs get a tile more than the others, at every
+// whole round (one tile on each CU: 65,536 cells on 256 CUs); with 64 it grows
+// more evenly, so just past a whole round 64 is ahead again, less each time.
+// Time of a step with 64 cells over that with 256 on both sides of each line,
+// least and most of an early and a developed blast and a shear layer on two
+// numberings of a mesh:
+//   FP64, rounds        .73      .77       .97   |   1.02     1.49 |    1.55      1.80   |   2.01     2.23 |    2.31      2.73
+//     ideal           .88-.96  .94-1.05  .96-1.07| .92-.96  .94-.96|  .99-1.02 1.02-1.10 | .97-.99  .94-.96| .99-1.00  1.02-1.06
+//     ideal, source   .91-.98  .95-1.02  .98-1.07| .94-.96  .97-1.0| 1.03-1.06 1.13-1.17 | .99-1.03 .98-1.0|1.01-1.03  1.13-1.15
+//     TAUB            .95-.97 1.05-1.08 1.07-1.09| .92-.94  .94-.95| 1.01-1.03 1.07-1.10 | .97-.99  .92-.93| .97-.98  1.02-1.03
+//   mixed, rounds      1.49      1.80      2.01      2.23     2.47   |   2.55      2.73      3.00
+//     ideal           .90-.90  .99-1.01 1.02-1.05  .90-.92  .94-.95 |  .96-.99   .95-.99 1.04-1.07
+//     ideal, source   .91-.94 1.03-1.06 1.03-1.06  .98-.99 1.02-1.04| 1.05-1.07 1.08-1.10 1.14-1.15
+//     TAUB            .90-.91 1.01-1.04  .99-1.01  .90-.94  .94-.96 |  .97-.99   .97-.99 1.06-1.09
+//     surrogate start .86-.91  .89-1.00  .90-1.02  .88-.93  .92-.94 |  .93-.97   .95-.98  .97-1.04
+// (The source is not known yet when the tiles are made.)
+int32_t tile_cells_for(int64_t n, bool mixed, int cus) {
+  const double rounds = (double)n / ((double)cus * kTileCells);
+  const bool small = mixed ? rounds <= 2.5
+                           : rounds <= 0.75 || (rounds > 1.0 && rounds <= 1.5) || (rounds > 2.0 && rounds <= 2.25);
+  return small ? kSmallTileCells : kTileCells;
 }
 
 }  // namespace
 
 namespace rhllc_capi_detail {
 int set_error(int code, const std::string &msg) { return fail(code, msg); }
+
+// Compute units of a device (256, or fewer where the GPU is partitioned).
+// Without a device 256: the calls after this one report that.
+int compute_units(int32_t device) {
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0) return cus;
+  (void)hipGetLastError();
+  return 256;
+}
 }  // namespace rhllc_capi_detail
 
 // Two pinned chunks that the transfers of a handle go through in turn: the
@@ -380,7 +401,7 @@ extern "C" int rhllc_create(const rhllc_params *params, int64_t n_cells, const v
   opt.lock_wall = p.lock_wall != 0;
   opt.reject_outer_surface = p.reject_outer_surface != 0;
   opt.out_source_copy = p.out_source_copy != 0;
-  opt.tile_cells = tile_cells_for(n_cells, mixed);
+  opt.tile_cells = tile_cells_for(n_cells, mixed, rhllc_capi_detail::compute_units(p.device));
   rhllc_layout::Layout L;
   {
     std::string err;
