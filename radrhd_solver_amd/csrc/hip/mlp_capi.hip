@@ -19,6 +19,7 @@ extern "C" const char *rhllc_last_error(void);
 
 namespace rhllc_capi_detail {
 int set_error(int code, const std::string &msg);
+int compute_units(int32_t device);
 }
 
 namespace {
@@ -185,6 +186,7 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
   // The first step's samples; each step makes the next one's.
   const Batch batch{cfg->gamma, cfg->seed, B, norm, X.as<float>(), Y.as<float>(), O.as<float>()};
   HIP_TRY(launch_gen(cfg->gamma, cfg->seed, B, norm, batch.X, batch.Y, batch.OK, st));
+  const int cus = rhllc_capi_detail::compute_units(cfg->device);
   // The launches of a training step are the same each time (its number is on
   // the device), so several are captured once and replayed.
   const auto launch_step = [&] {
@@ -193,7 +195,7 @@ extern "C" int rhllc_mlp_train(const rhllc_mlp_config *cfg, float *model_out, fl
     if (r == hipSuccess)
       r = launch_adam(P.as<float>(), M.as<float>(), V.as<float>(), W2.as<short>(), W2.as<short>() + kH * kH,
                       G.as<float>(), nw, S.as<uint32_t>(), cfg->steps, (float)cfg->lr, L.as<float>(), H.as<float>(),
-                      batch, st);
+                      batch, cus, st);
     return r;
   };
   hipError_t e = hipSuccess;

@@ -29,7 +29,9 @@ hipError_t launch_grad(const float *P, const short *W2b, const short *W2Tb, cons
                        const float *OK, float inv_n, int n, float *grad, float *loss, uint32_t *step, hipStream_t s);
 hipError_t launch_adam(float *P, float *M, float *V, short *W2b, short *W2Tb, const float *grad, int nwaves,
                        uint32_t *step, int total_steps, float lr0, const float *loss, float *loss_hist,
-                       const Batch &next, hipStream_t s);
+                       const Batch &next, int cus, hipStream_t s);
+// Samples of the next step that a workgroup of that launch makes, on a device of `cus` CUs.
+int gen_per(int n, int cus);
 // grad[p] = sum_w part[w * kGradStride + p] and *loss = sum_w lpart[w], in w order (FP32).
 hipError_t launch_sum(const float *part, const float *lpart, int nw, float *grad, float *loss, hipStream_t s);
 hipError_t launch_pack(const float *P, short *W2b, short *W2Tb, hipStream_t s);

@@ -415,18 +415,19 @@ __device__ __forceinline__ float ordered_loss_sum(const float *__restrict__ loss
 // and advances the step: step[1] is this step's number, which k_mlp_grad copied
 // from step[0]; only this workgroup writes step[0], which nobody reads here.
 // The workgroups after it write the next step's samples over this step's, which
-// k_mlp_grad has finished reading, spread over the 114 CUs that the sum leaves
-// (a workgroup's 16 waves fill its CU): the fewer waves a SIMD has, the sooner its
-// samples are done.  With one step a graph, which adds about 5 us to each, a
+// k_mlp_grad has finished reading, spread over the CUs that the sum leaves (114
+// of 256; a workgroup's 16 waves fill its CU): the fewer waves a SIMD has, the
+// sooner its samples are done.  With one step a graph, which adds about 5 us to each, a
 // training step takes 18.5 us at 1,024 samples (24.8 with
 // 640 samples a workgroup at every size), 19.9 at 16,384 (26.5), 28 at 49,152
 // (31), 34 at 65,536 (34; with a launch of its own for the samples 7 more), 41 at
 // 98,304 (51).  A batch that does not fit the idle CUs at once takes 640 each:
-// 55 us at 131,072, 60 with all 1,024 threads.
-constexpr int kIdleCus = 256 - (kSumBlocks + 1);
-constexpr int gen_per(int n) {
-  const int per = ((n + kIdleCus - 1) / kIdleCus + 63) / 64 * 64;
-  return per <= kSumThreads ? per : 640;
+// 55 us at 131,072, 60 with all 1,024 threads.  (So does any batch where the sum
+// takes every CU, as on a partitioned GPU.)
+int gen_per(int n, int cus) {
+  const int idle = cus - (kSumBlocks + 1);
+  if (idle < 1 || (n + idle - 1) / idle > kSumThreads) return 640;
+  return ((n + idle - 1) / idle + 63) / 64 * 64;
 }
 __global__ __launch_bounds__(kSumThreads) void k_mlp_adam(float *P, float *Mo, float *Vo, short *W2b, short *W2Tb,
                                                           const float *grad, int nwaves, uint32_t *step,
@@ -558,8 +559,8 @@ hipError_t launch_grad(const float *P, const short *W2b, const short *W2Tb, cons
 }
 hipError_t launch_adam(float *P, float *M, float *V, short *W2b, short *W2Tb, const float *grad, int nwaves,
                        uint32_t *step, int total_steps, float lr0, const float *loss, float *loss_hist,
-                       const Batch &next, hipStream_t s) {
-  const int per = gen_per(next.n);
+                       const Batch &next, int cus, hipStream_t s) {
+  const int per = gen_per(next.n, cus);
   const unsigned int blocks = kSumBlocks + 1 + (next.n + per - 1) / per;
   hipLaunchKernelGGL(k_mlp_adam, dim3(blocks), dim3(kSumThreads), 0, s, P, M, V, W2b, W2Tb, grad, nwaves, step,
                      total_steps, lr0, loss, loss_hist, next, per);
