@@ -220,7 +220,9 @@ int rhllc_add_rad_flux_tensor(rhllc_solver *h, double tau, const float *Ur, cons
  * back to back with one wait at the end; the steps advance the state:
  * out[0] face kernel (tiled step: the tile kernel, faces and cells),
  * out[1] cell kernel (tiled step: nothing but the gap between two events),
- * out[2] dt kernel, out[3] whole step. */
+ * out[2] dt kernel, out[3] whole step.  Where the steps of a run take the
+ * speed maximum themselves (rhllc_step_form) the step is the tile kernel alone:
+ * out[1] = out[2] = 0 and out[3] is the span of the timed steps over nsteps. */
 int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]);
 
 /* How a handle takes its steps, for tests and tools; no counterpart in the

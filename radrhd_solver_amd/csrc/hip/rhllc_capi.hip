@@ -280,23 +280,28 @@ struct rhllc_solver {
 
   bool folds() const { return tiled && n_tiles <= kFoldMaxTiles; }
 
-  // One step from buffer cur, at *tau or the device's own; the tiled step flips
-  // cur and, if it folds, stays open.  With a tau nothing is open before.
+  // The tiled step's kernel from buffer cur, at *tau or the device's own; it flips
+  // cur and leaves the step open.  With a tau nothing is open before.
+  hipError_t enqueue_tile(const double *tau = nullptr) {
+    Dev x = dev(cur, cur ^ 1);
+    x.slot = slot;
+    x.fold = open;
+    if (tau) x.use_tau = 1, x.tau = *tau;
+    const hipError_t e = launch_tile(x, mixed, variant, rad, prm.collect_stats != 0, n_tiles, tile_slots, stream);
+    if (e == hipSuccess) {
+      last_in = cur;
+      cur ^= 1;
+      slot = (slot + 1) % kSpeedBufs;
+      open = true;
+    }
+    return e;
+  }
+  // One step, closed unless it folds or is at the caller's tau.
   hipError_t enqueue_step(const double *tau = nullptr) {
     hipError_t e;
     if (tiled) {
-      Dev x = dev(cur, cur ^ 1);
-      x.slot = slot;
-      x.fold = open;
-      if (tau) x.use_tau = 1, x.tau = *tau;
-      e = launch_tile(x, mixed, variant, rad, prm.collect_stats != 0, n_tiles, tile_slots, stream);
-      if (e == hipSuccess) {
-        last_in = cur;
-        cur ^= 1;
-        slot = (slot + 1) % kSpeedBufs;
-        open = true;
-        if (!tau && !folds()) e = close_steps();
-      }
+      e = enqueue_tile(tau);
+      if (e == hipSuccess && !tau && !folds()) e = close_steps();
       return e;
     }
     Dev x = now();
@@ -923,40 +928,45 @@ extern "C" int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]
       rc = hip_fail(err, "kernel timing");
       break;
     }
-  const bool stats = h->prm.collect_stats != 0;
+  const bool stats = h->prm.collect_stats != 0, folds = h->folds();
   for (int32_t k = 0; k < kLead + nsteps && rc == RHLLC_OK; ++k) {
     hipEvent_t *e4 = k >= kLead ? &ev[4 * (size_t)(k - kLead)] : nullptr;
-    const Dev x = h->tiled ? h->dev(h->cur, h->cur ^ 1) : h->now();
     hipError_t e = e4 ? hipEventRecord(e4[0], h->stream) : hipSuccess;
-    if (e == hipSuccess)
-      e = h->tiled ? launch_tile(x, h->mixed, h->variant, h->rad, stats, h->n_tiles, h->tile_slots, h->stream)
-                   : launch_face(x, h->mixed, h->stream);
-    if (e == hipSuccess && e4) e = hipEventRecord(e4[1], h->stream);
-    if (e == hipSuccess && !h->tiled) e = launch_cell(x, h->variant, h->rad, stats, h->stream);
-    if (e == hipSuccess && e4) e = hipEventRecord(e4[2], h->stream);
-    if (e == hipSuccess) e = launch_dt(x, nullptr, h->stream);
-    if (e == hipSuccess && e4) e = hipEventRecord(e4[3], h->stream);
-    if (e != hipSuccess) {
-      rc = hip_fail(e, "kernel timing");
-      break;
+    if (h->tiled) {
+      if (e == hipSuccess) e = h->enqueue_tile();
+    } else {
+      if (e == hipSuccess) e = launch_face(h->now(), h->mixed, h->stream);
+      if (e == hipSuccess) h->last_in = h->cur, h->open = true;
     }
-    h->last_in = h->cur;
-    if (h->tiled) h->cur ^= 1;
+    if (e == hipSuccess && e4) e = hipEventRecord(e4[1], h->stream);
+    if (!folds) {  // a folding step is the tile kernel alone
+      if (e == hipSuccess && !h->tiled) e = launch_cell(h->now(), h->variant, h->rad, stats, h->stream);
+      if (e == hipSuccess && e4) e = hipEventRecord(e4[2], h->stream);
+      if (e == hipSuccess) e = h->close_steps();
+      if (e == hipSuccess && e4) e = hipEventRecord(e4[3], h->stream);
+    }
+    if (e != hipSuccess) rc = hip_fail(e, "kernel timing");
   }
+  if (hipError_t e = h->close_steps(); e != hipSuccess && rc == RHLLC_OK) rc = hip_fail(e, "kernel timing");
   double acc[4] = {0, 0, 0, 0};
   if (rc == RHLLC_OK) {
     if (hipError_t e = hipStreamSynchronize(h->stream); e != hipSuccess) rc = hip_fail(e, "kernel timing");
   }
+  const auto add = [&](int i, hipEvent_t from, hipEvent_t to) {
+    float ms = 0;
+    if (hipError_t e = hipEventElapsedTime(&ms, from, to); e != hipSuccess && rc == RHLLC_OK)
+      rc = hip_fail(e, "kernel timing");
+    acc[i] += ms;
+  };
   for (int32_t k = 0; k < nsteps && rc == RHLLC_OK; ++k) {
     const hipEvent_t *e4 = &ev[4 * (size_t)k];
-    float ms[4] = {0, 0, 0, 0};
-    hipError_t e = hipEventElapsedTime(&ms[0], e4[0], e4[1]);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms[1], e4[1], e4[2]);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms[2], e4[2], e4[3]);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms[3], e4[0], e4[3]);
-    if (e != hipSuccess) rc = hip_fail(e, "kernel timing");
-    for (int i = 0; i < 4; ++i) acc[i] += ms[i];
+    add(0, e4[0], e4[1]);
+    if (folds) continue;
+    add(1, e4[1], e4[2]);
+    add(2, e4[2], e4[3]);
+    add(3, e4[0], e4[3]);
   }
+  if (folds && rc == RHLLC_OK) add(3, ev[0], ev[4 * (size_t)(nsteps - 1) + 1]);
   for (auto &e : ev)
     if (e) (void)hipEventDestroy(e);
   if (rc != RHLLC_OK) return rc;
