@@ -233,9 +233,9 @@ int rhllc_time_kernels(rhllc_solver *h, int32_t nsteps, double out[4]);
  * quotients of ordinary states.  Waits for the queued steps. */
 int rhllc_step_form(rhllc_solver *h, int64_t out[4]);
 
-/* The tiled step's layout of a mesh at 256 cells a tile (a handle on a mesh
- * too small to fill the chip uses 64), computed on the host (no device is
- * touched), for tests and tools; no counterpart in the reference.  Returns
+/* The tiled step's layout of a mesh at 256 cells a tile, computed on the host
+ * (no device is touched), for tests and tools; no counterpart in the
+ * reference.  Returns
  * the tile count, the total of extra faces and the largest face count of a
  * tile; each non-NULL array receives: cell_new_to_old[n_cells] and
  * face_new_to_old[n_faces] (device numbering -> caller's), tile_meta
@@ -246,6 +246,13 @@ int rhllc_step_form(rhllc_solver *h, int64_t out[4]);
 int rhllc_tile_layout(int64_t n_cells, const void *geo_cells, int64_t n_faces, const void *geo_faces, int32_t reorder,
                       int32_t *n_tiles, int64_t *n_extra, int32_t *max_slots, int32_t *cell_new_to_old,
                       int32_t *face_new_to_old, int32_t *tile_meta, int32_t *tile_extra, uint32_t *cell_slots);
+
+/* rhllc_tile_layout at tile_cells cells a tile: 256, or the 64 of handles on
+ * meshes too small to fill the chip. */
+int rhllc_tile_layout_of(int64_t n_cells, const void *geo_cells, int64_t n_faces, const void *geo_faces,
+                         int32_t reorder, int32_t tile_cells, int32_t *n_tiles, int64_t *n_extra, int32_t *max_slots,
+                         int32_t *cell_new_to_old, int32_t *face_new_to_old, int32_t *tile_meta, int32_t *tile_extra,
+                         uint32_t *cell_slots);
 
 /* The mixed path's 16-byte form of n face vectors S n (3 doubles each) into
  * out (4 floats each), as rhllc_create stores them: the FP32 vector, and in

@@ -113,6 +113,7 @@ SIGNATURES = {
     "rhllc_info": (C.c_int, [_vp, _vp, _vp, _vp]),
     "rhllc_step_form": (C.c_int, [_vp, _vp]),
     "rhllc_tile_layout": (C.c_int, [_i64, _vp, _i64, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "rhllc_tile_layout_of": (C.c_int, [_i64, _vp, _i64, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "rhllc_pack_face_vectors": (C.c_int, [_i64, _vp, _vp]),
     "rhllc_eval_flux": (C.c_int, [_i32, _i32, _dbl, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "rhllc_eval_c2p": (C.c_int, [_i32, _i32, _dbl, _i64, _vp, _vp, _vp, _vp, _vp]),
@@ -318,12 +319,12 @@ class Solver:
         return b.value
 
 
-def tile_layout(mesh, reorder=True):
+def tile_layout(mesh, reorder=True, tile_cells=256):
     """The tiled step's host layout of a mesh (no device): a dict of arrays."""
     L = _lib()
     nt, ne, ms = C.c_int32(), C.c_int64(), C.c_int32()
-    args = (mesh.n_cells, mesh.cells.ctypes.data, mesh.n_faces, mesh.faces.ctypes.data, int(reorder))
-    check(L.rhllc_tile_layout(*args, C.byref(nt), C.byref(ne), C.byref(ms), None, None, None, None, None))
+    args = (mesh.n_cells, mesh.cells.ctypes.data, mesh.n_faces, mesh.faces.ctypes.data, int(reorder), tile_cells)
+    check(L.rhllc_tile_layout_of(*args, C.byref(nt), C.byref(ne), C.byref(ms), None, None, None, None, None))
     out = {
         "cell_new_to_old": np.zeros(mesh.n_cells, np.int32),
         "face_new_to_old": np.zeros(mesh.n_faces, np.int32),
@@ -331,8 +332,8 @@ def tile_layout(mesh, reorder=True):
         "tile_extra": np.zeros(max(ne.value, 1), np.int32),
         "cell_slots": np.zeros((mesh.n_cells, 2), np.uint32),
     }
-    check(L.rhllc_tile_layout(*args, C.byref(nt), C.byref(ne), C.byref(ms),
-                              *[out[k].ctypes.data for k in ("cell_new_to_old", "face_new_to_old", "tile_meta",
+    check(L.rhllc_tile_layout_of(*args, C.byref(nt), C.byref(ne), C.byref(ms),
+                                 *[out[k].ctypes.data for k in ("cell_new_to_old", "face_new_to_old", "tile_meta",
                                                               "tile_extra", "cell_slots")]))
     out["tile_extra"] = out["tile_extra"][:ne.value]
     out["max_slots"] = ms.value

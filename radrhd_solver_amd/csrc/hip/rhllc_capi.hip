@@ -1004,14 +1004,24 @@ extern "C" int rhllc_tile_layout(int64_t n_cells, const void *geo_cells, int64_t
                                  int32_t reorder, int32_t *n_tiles, int64_t *n_extra, int32_t *max_slots,
                                  int32_t *cell_new_to_old, int32_t *face_new_to_old, int32_t *tile_meta,
                                  int32_t *tile_extra, uint32_t *cell_slots) {
+  return rhllc_tile_layout_of(n_cells, geo_cells, n_faces, geo_faces, reorder, kTileCells, n_tiles, n_extra, max_slots,
+                              cell_new_to_old, face_new_to_old, tile_meta, tile_extra, cell_slots);
+}
+
+extern "C" int rhllc_tile_layout_of(int64_t n_cells, const void *geo_cells, int64_t n_faces, const void *geo_faces,
+                                    int32_t reorder, int32_t tile_cells, int32_t *n_tiles, int64_t *n_extra,
+                                    int32_t *max_slots, int32_t *cell_new_to_old, int32_t *face_new_to_old,
+                                    int32_t *tile_meta, int32_t *tile_extra, uint32_t *cell_slots) {
   if (!geo_cells || !geo_faces || !n_tiles || !n_extra || !max_slots) return fail(RHLLC_ERR_ARG, "null argument");
   if (n_cells < 1 || n_cells >= ((int64_t)1 << 25) || n_faces < 1 || n_faces > 0x7FFFFFFF)
     return fail(RHLLC_ERR_ARG, "mesh size out of range");
+  if (tile_cells != kTileCells && tile_cells != kSmallTileCells)
+    return fail(RHLLC_ERR_ARG, "tile_cells must be 64 or 256");
   rhllc_layout::Options opt;
   opt.reorder = reorder != 0;
   opt.tiled = true;
   opt.has_out_source = true;
-  opt.tile_cells = kTileCells;
+  opt.tile_cells = tile_cells;
   rhllc_layout::Layout L;
   std::string err;
   if (!rhllc_layout::build(opt, n_cells, geo_cells, n_faces, geo_faces, L, err)) return fail(RHLLC_ERR_ARG, err);
