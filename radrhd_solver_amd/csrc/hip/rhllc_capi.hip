@@ -577,7 +577,10 @@ extern "C" int rhllc_download_state(rhllc_solver *h, void *recs, int64_t stride,
   HIP_TRY(hipSetDevice(h->prm.device));
   const Dev d = h->now();
   const bool phys = off_phys >= 0, conv = off_conv >= 0;
-  if (!phys && !conv) return RHLLC_OK;
+  if (!phys && !conv) {  // the wait alone
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    return RHLLC_OK;
+  }
   HIP_TRY(h->staging.receive(
       h->n_cells, phys && conv ? 80 : 40, h->stream,
       [&](int i, int n, void *chunk) {

@@ -5,6 +5,8 @@ each kind (40 and 80 bytes a cell, 40 a face, 24 a cell for the radiation fields
 last one, 6 and 630 cells a part of one.  Everything is a copy, or the FP64 step and source of
 the oracle, so every comparison is for equal bits.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -65,4 +67,26 @@ def test_fields_and_fluxes_reach_their_cells_and_faces(shape):
     W, U = s.download()
     assert np.array_equal(W, st.W) and np.array_equal(U, st.U)
     assert np.array_equal(s.face_flux(), st.face_flux)
+    s.close()
+
+
+def test_a_download_of_neither_part_waits():
+    """It copies nothing, but the steps before it are done when it returns, as with either part."""
+    m = M.kuhn_box(48, 48, 48, seed=SEED)
+    s = capi.Solver(m, cfl=0.4)
+    s.upload_W(M.init_state(m, M.INIT_BLAST))
+    L, out = capi._lib(), np.full((m.n_cells, 5), -7.0)
+
+    def rest():  # seconds left for sync after the call, of a run of 2,000 steps
+        s.run(2000)
+        t0 = time.perf_counter()
+        capi.check(L.rhllc_download_state(s.h, out.ctypes.data, 40, -1, -1))
+        t1 = time.perf_counter()
+        s.sync()
+        return t1 - t0, time.perf_counter() - t1
+
+    rest()
+    waited, left = rest()
+    print("waited", waited, "left", left)
+    assert (out == -7.0).all() and left < 0.25 * (waited + left)
     s.close()
