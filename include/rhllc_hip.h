@@ -131,7 +131,11 @@ int rhllc_destroy(rhllc_solver *h);
  * at off_conv.  Upload with off_conv < 0 computes U = p2c(W) on the device
  * (HllcPhysToConv, which clamps |v| >= 1 and so may rewrite W) and resets the
  * time loop as rhllc::Init does: max_speed = 1, tau = CFL*h_min, t = 0.
- * Download with off_phys or off_conv < 0 skips that part. */
+ * Download with off_phys or off_conv < 0 skips that part.
+ * Both come after the steps queued before.  An upload returns once the records
+ * are copied out of recs, which the caller may then change or free; its kernels
+ * may still be queued, and a device error in them is reported by a later call.
+ * An upload that fails leaves no state.  A download returns when it is done. */
 int rhllc_upload_state(rhllc_solver *h, const void *recs, int64_t stride, int64_t off_phys, int64_t off_conv);
 int rhllc_download_state(rhllc_solver *h, void *recs, int64_t stride, int64_t off_phys, int64_t off_conv);
 
@@ -167,7 +171,9 @@ int rhllc_download_face_flux(rhllc_solver *h, double *F);
 /* Radiation fields for the explicit 4-momentum source, applied after the
  * hydro update as radRHD_main.cpp:117-132 does (M1 Eddington tensor).  Per
  * cell in the caller's numbering, FP32.  NULL Ur removes the source.  With an
- * opacity table set (below) kappa_a and kappa_s are not used and may be NULL. */
+ * opacity table set (below) kappa_a and kappa_s are not used and may be NULL.
+ * The fields reach the steps queued after the call; it returns once they are
+ * copied out of the caller's arrays (likewise rhllc_set_radiation_tensor). */
 int rhllc_set_radiation(rhllc_solver *h, const float *Ur, const float *Fr3, const float *kappa_a,
                         const float *kappa_s);
 

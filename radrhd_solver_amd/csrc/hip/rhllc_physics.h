@@ -88,9 +88,10 @@ struct Ieee {
 // Ieee for ordinary operands (`ordinary` below): the same correctly rounded
 // quotients and roots without the scaling that protects operands and results
 // near the ends of the exponent range.  The quotient is Newton's reciprocal and
-// one residual correction (Markstein 1990), the root the coupled iteration for
-// sqrt(x) and 1/(2 sqrt(x)) with two residual corrections; v_div_fixup and the
-// class test keep zeros, infinities and NaNs as Ieee has them.  A quotient takes
+// one residual correction (Markstein 1990), the root Goldschmidt's coupled
+// iteration for sqrt(x) and 1/(2 sqrt(x)) (Goldschmidt 1964; with fused
+// residuals as in Markstein 2004) and two residual corrections; v_div_fixup and
+// the class test keep zeros, infinities and NaNs as Ieee has them.  A quotient takes
 // 9 instructions for 11 and a hazard wait, and quotients by one denominator
 // share its reciprocal (4 more each); a root takes 13 for 18.  The tiled step
 // at 6M cells: 527 -> 490 us (TAUB), 635 -> 590 (ideal gas with the radiation
