@@ -7,6 +7,7 @@ value: a setter between two runs has to reach the second.
 import numpy as np
 import pytest
 
+import oracle as O
 from radrhd_solver_amd import capi, surrogate
 from radrhd_solver_amd import mesh as M
 from rad_cases import physical_blast, table_path
@@ -117,6 +118,26 @@ def test_tables_between_replays(path, tmp_path):
     a, b = (_stages(_solver(m, path), setters, W0, graph) for graph in (True, False))
     _compare(a, b)
     assert not np.array_equal(a[0][2], a[2][2]) and not np.array_equal(a[1][2], a[3][2])
+
+
+@pytest.mark.parametrize("schedule", [capi.SCHED_TILED, capi.SCHED_TWO_KERNEL])
+@pytest.mark.parametrize("eos", [capi.EOS_IDEAL, capi.EOS_TAUB])
+def test_replays_of_the_periodic_shear_are_the_oracles_bits(eos, schedule):
+    """FP64, 73 steps in three graphs and one single step."""
+    m = M.kuhn_box(8, 7, 6, origin=(-0.5, -0.5, -0.5), periodic=7, seed=SEED)
+    h = m.h_min()
+    W0 = M.init_state(m, M.INIT_SHEAR, seed=SEED)
+    st = O.State(m, W0, eos=eos)
+    st.run(0.4, h, 73)
+    s = capi.Solver(m, cfl=0.4, h_min=h, eos=eos, schedule=schedule)
+    s.upload_W(W0)
+    s.run(73)
+    s.sync()
+    assert s.step_form()["replays"] == 3
+    W, U = s.download()
+    for a, b in ((W, st.W), (U, st.U), (s.face_flux(), st.face_flux)):
+        assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
+    s.close()
 
 
 def test_graphs_are_captured_at_72_steps_worth():
